@@ -647,9 +647,13 @@ int pysa_amd_ais(int64_t handle, const void* temps, int32_t nt, int32_t chains, 
     HIP_TRY(sg.up(states, (size_t)chains * n, &dS, st));
     HIP_TRY(sg.alloc((size_t)chains * sizeof(double), &dE));
     HIP_TRY(sg.alloc((size_t)chains * sizeof(double), &dW));
+    void* dX = nullptr;
+    const size_t xb = pysa::energy_scratch_bytes((int)n, chains);
+    if (xb) HIP_TRY(sg.alloc(xb, &dX));
     // the initial energies in f64 (simulation.py:301)
     hipError_t le = pysa::launch_energy_f64<float>((const float*)P->dJt, (const float*)P->dh,
-                                                   (const int8_t*)dS, (double*)dE, (int)n, chains, st);
+                                                   (const int8_t*)dS, (double*)dE, (int)n, chains,
+                                                   (double*)dX, st);
     if (le != hipSuccess) {
       (void)hipStreamSynchronize(st);
       return fail(PYSA_AMD_EHIP, std::string("energy launch: ") + hipGetErrorString(le));
@@ -807,14 +811,18 @@ int pysa_amd_energy(int64_t handle, const int8_t* states, int64_t count, double*
   HIP_TRY(hipSetDevice(P->device));
   hipStream_t st = P->stream;
   Staged sg;
-  void *dS, *dO;
+  void *dS, *dO, *dX = nullptr;
   HIP_TRY(sg.up(states, (size_t)count * P->n, &dS, st));
   HIP_TRY(sg.alloc((size_t)count * sizeof(double), &dO));
+  const size_t xb = pysa::energy_scratch_bytes(P->n, count);
+  if (xb) HIP_TRY(sg.alloc(xb, &dX));
   hipError_t le = (P->dtype == 0)
                       ? pysa::launch_energy_f64<float>((const float*)P->dJt, (const float*)P->dh,
-                                                       (const int8_t*)dS, (double*)dO, P->n, count, st)
+                                                       (const int8_t*)dS, (double*)dO, P->n, count,
+                                                       (double*)dX, st)
                       : pysa::launch_energy_f64<double>((const double*)P->dJt, (const double*)P->dh,
-                                                        (const int8_t*)dS, (double*)dO, P->n, count, st);
+                                                        (const int8_t*)dS, (double*)dO, P->n, count,
+                                                        (double*)dX, st);
   if (le != hipSuccess) return fail(PYSA_AMD_EHIP, std::string("energy launch: ") + hipGetErrorString(le));
   HIP_TRY(hipMemcpyAsync(out, dO, (size_t)count * sizeof(double), hipMemcpyDeviceToHost, st));
   HIP_TRY(hipStreamSynchronize(st));

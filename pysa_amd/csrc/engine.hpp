@@ -69,9 +69,11 @@ struct AISParams {
   double* logw;           // chains
 };
 
+// f64 energies of `count` states; scratch: energy_scratch_bytes(n, count) bytes.
+size_t energy_scratch_bytes(int n, long long count);
 template <typename T>
 hipError_t launch_energy_f64(const T* Jt, const T* h, const int8_t* spins, double* out, int n,
-                             long long count, hipStream_t st);
+                             long long count, double* scratch, hipStream_t st);
 template <typename T>
 hipError_t launch_plain_pt(const PTParams<T>& p, hipStream_t st);
 template <typename T>

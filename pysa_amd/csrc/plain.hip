@@ -19,6 +19,8 @@
 // The sweep loop, best tracking, parallel tempering and log-omega run inside
 // one persistent launch; the replicas of a read meet at a workgroup barrier
 // once per sweep.
+#include <type_traits>
+
 #include "engine.hpp"
 #include "rng.hpp"
 
@@ -641,28 +643,154 @@ __global__ __launch_bounds__((64 * kernel_waves<T, G>())) void plain_ais_kernel(
   }
 }
 
-// E = s.(J s / 2 + h) in f64, one workgroup per state (ising.py:32-37).
-// Thread i accumulates F_i = sum_j J[i][j] s_j from rows of J^T (coalesced
-// across threads); the state is read through the scalar cache.
-template <typename T>
-__global__ __launch_bounds__(256) void energy_f64_kernel(const T* __restrict__ Jt,
-                                                         const T* __restrict__ h,
-                                                         const int8_t* __restrict__ spins,
+// J s in f64 for SB states per workgroup: thread t owns the elements
+// i = i0 + t, i0 + 256 + t, ... (I of them), and every coupling it loads (from
+// rows of J^T, coalesced across threads) serves all SB states.  A state's
+// spins of 64 columns j are one bit per lane, read back one column at a time,
+// so the factor of a product (1 for a set bit, else the double with the high
+// word `low`: -1 or 0) is a scalar operand.  GEN: spins of any int8 value, read
+// one by one.  Every sum runs over j in ascending order in f64, whatever SB
+// and I are, and each product J s is exact, so the results do not depend on
+// the tiling.
+template <typename T, int SB, int I, bool GEN>
+__device__ __forceinline__ void field_sums(const T* __restrict__ Jt,
+                                           const int8_t* __restrict__ spins, int n, int count,
+                                           int s0, int i0, uint32_t low, double (&f)[SB][I]) {
+  const int lane = threadIdx.x & 63;
+  // byte offsets within a row (the row's base is uniform), clamped: a thread
+  // past n repeats the last element (unused)
+  uint32_t ic[I];
+#pragma unroll
+  for (int k = 0; k < I; ++k)
+    ic[k] = (uint32_t)min(i0 + 256 * k + (int)threadIdx.x, n - 1) * (uint32_t)sizeof(T);
+#pragma unroll
+  for (int b = 0; b < SB; ++b)
+#pragma unroll
+    for (int k = 0; k < I; ++k) f[b][k] = 0.0;
+  constexpr int U = GEN ? 1 : SB * I >= 32 ? 2 : 16;  // columns whose loads are in flight together
+  for (int j0 = 0; j0 < n; j0 += 64) {
+    uint32_t up = 0;
+    if constexpr (!GEN) {
+      const int jl = min(j0 + lane, n - 1);
+#pragma unroll
+      for (int b = 0; b < SB; ++b)
+        up |= (uint32_t)(spins[(size_t)min(s0 + b, count - 1) * n + jl] == 1) << b;
+    }
+    for (int jj = 0; jj < 64 && j0 + jj < n; jj += U) {
+      T x[U][I];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        // past the last column: its values again, as zeros
+        const bool in = j0 + jj + u < n;
+        const char* row =
+            reinterpret_cast<const char*>(Jt + (size_t)(in ? j0 + jj + u : n - 1) * n);
+#pragma unroll
+        for (int k = 0; k < I; ++k) {
+          const T v = *reinterpret_cast<const T*>(row + ic[k]);
+          x[u][k] = U == 1 || in ? v : T(0);
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const uint32_t w = GEN ? 0u : rl(up, jj + u);
+#pragma unroll
+        for (int b = 0; b < SB; ++b) {
+          const double sv =
+              GEN ? (double)spins[(size_t)min(s0 + b, count - 1) * n + j0 + jj]
+                  : as_double((uint64_t)(((w >> b) & 1u) ? 0x3FF00000u : low) << 32);
+#pragma unroll
+          for (int k = 0; k < I; ++k) f[b][k] = dfma((double)x[u][k], sv, f[b][k]);
+        }
+      }
+    }
+  }
+}
+
+// E = s.(J s / 2 + h) in f64 (ising.py:32-37), SB states per workgroup.  Thread
+// t adds its elements t, t + 256, ... in this order, then the wave and the
+// workgroup add theirs.  With one workgroup per group of states (gridDim.y =
+// 1) the energies go to out; otherwise workgroup y writes the terms of its
+// 256 I elements and energy_sum_kernel adds them in the same order.
+template <typename T, int SB, int I, bool GEN>
+__device__ __forceinline__ void energy_body(const T* __restrict__ Jt, const T* __restrict__ h,
+                                            const int8_t* __restrict__ spins, double* out,
+                                            double* terms, int n, int count, uint32_t low,
+                                            double (&red)[SB][4]) {
+  const int s0 = blockIdx.x * SB;
+  double e[SB];
+#pragma unroll
+  for (int b = 0; b < SB; ++b) e[b] = 0.0;
+  for (int c = blockIdx.y; c * 256 * I < n; c += gridDim.y) {
+    double f[SB][I];
+    field_sums<T, SB, I, GEN>(Jt, spins, n, count, s0, c * 256 * I, low, f);
+#pragma unroll
+    for (int k = 0; k < I; ++k) {
+      const int i = (c * I + k) * 256 + threadIdx.x;
+      const int il = min(i, n - 1);
+      const double hi = (double)h[il];
+#pragma unroll
+      for (int b = 0; b < SB; ++b) {
+        const double t =
+            (double)spins[(size_t)min(s0 + b, count - 1) * n + il] * (0.5 * f[b][k] + hi);
+        if (terms) {
+          if (i < n && s0 + b < count) terms[(size_t)(s0 + b) * n + i] = t;
+        } else {
+          e[b] = i < n ? e[b] + t : e[b];
+        }
+      }
+    }
+  }
+  if (terms) return;
+#pragma unroll
+  for (int b = 0; b < SB; ++b) {
+    const double t = wave_sum(e[b]);
+    if ((threadIdx.x & 63) == 0) red[b][threadIdx.x >> 6] = t;
+  }
+  __syncthreads();
+  if (threadIdx.x < SB && s0 + (int)threadIdx.x < count) {
+    double t = 0.0;
+    for (int w = 0; w < 4; ++w) t += red[threadIdx.x][w];
+    out[s0 + threadIdx.x] = t;
+  }
+}
+
+// Bound: f64 fma issue (SB I per coupling loaded and converted).  16384 states
+// of 1024 spins: 8.49 ms with one state per workgroup, where every product
+// loaded its own coupling from L2, 1.17 ms with SB = 16, I = 4 (0.44 ms
+// is 2^34 f64 fma at the vector peak).
+template <typename T, int SB, int I>
+__global__ __launch_bounds__(256, SB* I >= 32 ? 2 : 4) void energy_f64_kernel(
+    const T* __restrict__ Jt, const T* __restrict__ h, const int8_t* __restrict__ spins,
+    double* out, double* terms, int n, int count) {
+  __shared__ double red[SB][4];
+  // the values these states hold: +-1, 0 / 1, or others (the entry point takes any int8)
+  const int s0 = blockIdx.x * SB;
+  bool pm = true, zo = true;
+  const size_t lo = (size_t)s0 * n, hi = (size_t)min(s0 + SB, count) * n;
+  for (size_t i = lo + threadIdx.x; i < hi; i += 256) {
+    const int v = spins[i];
+    pm = pm && (v == 1 || v == -1);
+    zo = zo && (v == 1 || v == 0);
+  }
+  pm = __syncthreads_and(pm);
+  zo = __syncthreads_and(zo);
+  if (pm || zo)
+    energy_body<T, SB, I, false>(Jt, h, spins, out, terms, n, count, pm ? 0xBFF00000u : 0u, red);
+  else
+    energy_body<T, SB, I, true>(Jt, h, spins, out, terms, n, count, 0u, red);
+}
+
+__global__ __launch_bounds__(256) void energy_sum_kernel(const double* __restrict__ terms,
                                                          double* out, int n) {
   __shared__ double red[4];
-  const int8_t* st = spins + (size_t)blockIdx.x * n;
   double e = 0.0;
-  for (int i = threadIdx.x; i < n; i += blockDim.x) {
-    double f = 0.0;
-    for (int j = 0; j < n; ++j) f += (double)Jt[(size_t)j * n + i] * (double)st[j];
-    e += (double)st[i] * (0.5 * f + (double)h[i]);
-  }
+  for (int i = threadIdx.x; i < n; i += 256) e += terms[(size_t)blockIdx.x * n + i];
   e = wave_sum(e);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = e;
   __syncthreads();
   if (threadIdx.x == 0) {
     double t = 0.0;
-    for (int w = 0; w < (int)(blockDim.x >> 6); ++w) t += red[w];
+    for (int w = 0; w < 4; ++w) t += red[w];
     out[blockIdx.x] = t;
   }
 }
@@ -723,13 +851,32 @@ hipError_t launch_plain_ais(const AISParams<T>& p, hipStream_t st) {
   }
 }
 
+// Tiling of the energy kernel: 16 states per workgroup once that fills the
+// device, else 4 states and 256 elements each, the sums in a second launch
+// (100 states of 3072 spins: 10.36 -> 0.37 ms).
+constexpr int kEnergyWide = 16 * 256;
+
+size_t energy_scratch_bytes(int n, long long count) {
+  return count >= kEnergyWide || n <= 256 ? 0 : (size_t)count * n * sizeof(double);
+}
+
 template <typename T>
 hipError_t launch_energy_f64(const T* Jt, const T* h, const int8_t* spins, double* out, int n,
-                             long long count, hipStream_t st) {
+                             long long count, double* scratch, hipStream_t st) {
   if (count <= 0) return hipSuccess;
   if (count > 0x7fffffffLL) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((energy_f64_kernel<T>), dim3((unsigned)count), dim3(256), 0, st, Jt, h,
-                     spins, out, n);
+  if (count >= kEnergyWide) {
+    hipLaunchKernelGGL((energy_f64_kernel<T, 16, 4>), dim3((unsigned)((count + 15) / 16)),
+                       dim3(256), 0, st, Jt, h, spins, out, (double*)nullptr, n, (int)count);
+    return hipGetLastError();
+  }
+  const unsigned chunks = (unsigned)((n + 255) / 256);
+  if (chunks > 1 && !scratch) return hipErrorInvalidValue;
+  hipLaunchKernelGGL((energy_f64_kernel<T, 4, 1>), dim3((unsigned)((count + 3) / 4), chunks),
+                     dim3(256), 0, st, Jt, h, spins, out, chunks > 1 ? scratch : nullptr, n,
+                     (int)count);
+  if (chunks > 1)
+    hipLaunchKernelGGL(energy_sum_kernel, dim3((unsigned)count), dim3(256), 0, st, scratch, out, n);
   return hipGetLastError();
 }
 
@@ -738,8 +885,8 @@ template hipError_t launch_plain_pt<double>(const PTParams<double>&, hipStream_t
 template hipError_t launch_plain_ais<float>(const AISParams<float>&, hipStream_t);
 template hipError_t launch_plain_ais<double>(const AISParams<double>&, hipStream_t);
 template hipError_t launch_energy_f64<float>(const float*, const float*, const int8_t*, double*, int,
-                                             long long, hipStream_t);
+                                             long long, double*, hipStream_t);
 template hipError_t launch_energy_f64<double>(const double*, const double*, const int8_t*, double*,
-                                              int, long long, hipStream_t);
+                                              int, long long, double*, hipStream_t);
 
 }  // namespace pysa
