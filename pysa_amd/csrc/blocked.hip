@@ -633,6 +633,8 @@ struct BlockedPlan {
   bool pipe, i8, inexact;
 };
 
+}  // namespace
+
 // Compute units of the current device (cached per device).
 int device_cus() {
   static std::mutex mu;
@@ -647,6 +649,8 @@ int device_cus() {
   }
   return cus[dev];
 }
+
+namespace {
 
 // Coupling encoding and kernel shape; b.exact_kind must be known.
 BlockedPlan plan_blocked(const BlockedProblem& b, int n, int reads, int R, int order, int pieces) {

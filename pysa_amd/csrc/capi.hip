@@ -200,6 +200,16 @@ int run_plain(Problem* P, const RunArgs& a, hipStream_t st, double* ms) {
   p.best_sweeps = a.best_sweeps;
   p.log_omegas = a.logw ? a.log_omegas : nullptr;
   p.accepted = (unsigned long long*)a.accepted;
+  p.plan = sparse ? pysa::kPlanReads : pysa::plan_plain(P->n, a.reads, a.R, (int)sizeof(T));
+  p.sums = nullptr;
+  p.eoff = nullptr;
+  p.chain_beta = nullptr;
+  if (p.plan == pysa::kPlanChains) {  // sums, offsets and betas of every chain
+    HIP_TRY(P->work.ensure(cnt * (n * sizeof(double) + sizeof(double) + sizeof(T))));
+    p.sums = (double*)P->work.p;
+    p.eoff = p.sums + cnt * n;
+    p.chain_beta = (T*)(p.eoff + cnt);
+  }
   // Per-read starting values: beta_idx = arange(R) (sa.py:325), the initial
   // state is the first best candidate (simulation.py:143-145).
   const unsigned nb = (unsigned)((cnt + 255) / 256);

@@ -47,7 +47,19 @@ struct PTParams {
   int* best_sweeps;       // reads
   double* log_omegas;     // reads*S or null
   unsigned long long* accepted;  // reads or null
+  int plan;               // plan_plain
+  // kPlanChains only
+  double* sums;           // reads*R*n: J s in f64
+  double* eoff;           // reads*R: the caller's initial energy minus its f64 recomputation
+  T* chain_beta;          // reads*R: the beta of every chain in the coming sweep
 };
+
+// Where the chains of a plain run go: one workgroup per read or per chain.
+enum PlainPlan : int { kPlanReads = 0, kPlanChains = 1 };
+int plan_plain(int n, int reads, int R, int elem);
+
+// Compute units of the current device (cached per device).
+int device_cus();
 
 // Annealed importance sampling over `chains` independent chains (plain form).
 template <typename T>

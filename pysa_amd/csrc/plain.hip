@@ -8,17 +8,24 @@
 //   pysa/ais.py:79-112          get_log_omega
 //   pysa/simulation.py:266-317  ais_simulation_parallel / ais_sample
 //
-// Layout.  One workgroup per read (PT) or per group of chains (AIS); each
-// wave carries one chain at a time.  A chain's local fields F = J s live in VGPRs:
-// element i sits in lane (i>>2)&63, register slot ((i>>8)<<2)|(i&3), so four
-// consecutive slots of a lane hold four consecutive elements and a coupling
-// row moves as 16-byte vectors.  Spins are one bit per slot.  A proposal reads
-// F[pos] with a readlane, so dE is O(1); an accepted flip adds one coupling row
-// (times dS in {+-1, +-2}) to every field.
+// Layout.  A wave carries one chain at a time.  A chain's local fields F = J s
+// live in VGPRs: element i sits in lane (i>>2)&63, register slot
+// ((i>>8)<<2)|(i&3), so four consecutive slots of a lane hold four consecutive
+// elements and a coupling row moves as 16-byte vectors.  Spins are one bit per
+// slot.
 //
-// The sweep loop, best tracking, parallel tempering and log-omega run inside
-// one persistent launch; the replicas of a read meet at a workgroup barrier
-// once per sweep.
+// A sweep takes its visits 64 at a time, one per lane (sweep_dense): every
+// lane holds the field of its visit and decides at once; the first accepted
+// visit flips, its coupling row updates the fields of the visits behind it,
+// and they decide again.  So rejected proposals cost nothing by themselves,
+// and a window takes as many steps as it has accepted flips.  The additions
+// to every field happen in the order of the flips, as one visit after another
+// would make them, so the results equal that to the bit.
+//
+// Where the chains run (plan_pt): one workgroup per read that carries all
+// replicas through the whole run and meets at a barrier once per sweep, or,
+// when that leaves most of the device idle, one workgroup per chain with the
+// exchanges in a launch of their own after every sweep.
 #include <type_traits>
 
 #include "engine.hpp"
@@ -54,6 +61,13 @@ __device__ __forceinline__ int wave_sum(int v) {
   return v;
 }
 
+// Orders LDS accesses of one wave across its lanes (the hardware executes them
+// in order; this keeps the compiler from moving them).
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // Element <-> (lane, slot) map of the field layout.
 __device__ __forceinline__ int elem_of(int lane, int g) {
   return ((g >> 2) << 8) + (lane << 2) + (g & 3);
@@ -69,6 +83,10 @@ __device__ __forceinline__ uint64_t shfl_bits(uint64_t w, int src) {
   const uint32_t hi = (uint32_t)__shfl((int)(uint32_t)(w >> 32), src, 64);
   return ((uint64_t)hi << 32) | lo;
 }
+
+// x dS + f for dS a power of two: rounds like the product and the sum.
+__device__ __forceinline__ float fma_t(float x, float dS, float f) { return __builtin_fmaf(x, dS, f); }
+__device__ __forceinline__ double fma_t(double x, double dS, double f) { return __builtin_fma(x, dS, f); }
 
 template <typename T>
 struct alignas(4 * sizeof(T)) T4 {
@@ -103,14 +121,23 @@ struct Chain {
   T f[G];
   B bits;  // bit g: the spin of element elem_of(lane, g) is up (+1 / 1)
 
-  __device__ void load(const T* F, const int8_t* s, int n) {
+  __device__ void load_spins(const int8_t* s, int n) {
     const int lane = threadIdx.x & 63;
     bits = 0;
 #pragma unroll
     for (int g = 0; g < G; ++g) {
       const int i = elem_of(lane, g);
-      f[g] = (i < n) ? F[i] : T(0);
+      f[g] = T(0);
       if (i < n && s[i] == 1) bits |= (B(1) << g);
+    }
+  }
+  __device__ void load(const T* F, const int8_t* s, int n) {
+    const int lane = threadIdx.x & 63;
+    load_spins(s, n);
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      const int i = elem_of(lane, g);
+      if (i < n) f[g] = F[i];
     }
   }
   __device__ void store(T* F, int8_t* s, int n, int ptype) const {
@@ -151,33 +178,50 @@ struct Chain {
 
   // F = J s accumulated in f64 and rounded once to T; returns
   // E = s.(F/2 + h) in f64 (the periodic recomputation that bounds drift).
-  __device__ double refresh(const T* __restrict__ Jt, const T* h, int n, int ptype) {
+  // Rows of J^T padded with zeros to ldp, eight in flight.
+  __device__ double refresh(const T* __restrict__ Jp, int ldp, const T* h, int n, int ptype) {
     const int lane = threadIdx.x & 63;
     double e = 0.0;
 #pragma unroll
     for (int g4 = 0; g4 < G / 4; ++g4) {
       double a[4] = {0.0, 0.0, 0.0, 0.0};
       const int i0 = (g4 << 8) + (lane << 2);
-      for (int j = 0; j < n; ++j) {
-        const bool upj = up_at(j);
-        if (ptype == 1 && !upj) continue;
-        const double sj = upj ? 1.0 : -1.0;
-        const T* row = Jt + (size_t)j * n;
+      if ((g4 << 8) < ldp) {
+        for (int j0 = 0; j0 < n; j0 += 8) {
+          T4<T> x[8];
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-          if (i0 + q < n) a[q] += (double)row[i0 + q] * sj;
-      }
+          for (int u = 0; u < 8; ++u)
+            x[u] = *reinterpret_cast<const T4<T>*>(Jp + (size_t)min(j0 + u, n - 1) * ldp + i0);
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int g = 4 * g4 + q;
-        f[g] = (T)a[q];
-        if (i0 + q < n) {
-          const double si = ((bits >> g) & 1) ? 1.0 : (ptype == 0 ? -1.0 : 0.0);
-          e += si * (0.5 * a[q] + (double)h[i0 + q]);
+          for (int u = 0; u < 8; ++u) {
+            if (j0 + u >= n) break;
+            const bool upj = up_at(j0 + u);
+            if (ptype == 1 && !upj) continue;
+            const double sj = upj ? 1.0 : -1.0;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) a[q] += (double)x[u].v[q] * sj;
+          }
         }
       }
+      e = put_fields(g4, a, h, n, ptype, e);
     }
     return wave_sum(e);
+  }
+  // Slots 4 g4 .. 4 g4 + 3 from their f64 sums; returns e plus their terms of
+  // the energy, in slot order.
+  __device__ __forceinline__ double put_fields(int g4, const double (&a)[4], const T* h, int n,
+                                               int ptype, double e) {
+    const int i0 = (g4 << 8) + ((threadIdx.x & 63) << 2);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int g = 4 * g4 + q;
+      f[g] = (T)a[q];
+      if (i0 + q < n) {
+        const double si = ((bits >> g) & 1) ? 1.0 : (ptype == 0 ? -1.0 : 0.0);
+        e += si * (0.5 * a[q] + (double)h[i0 + q]);
+      }
+    }
+    return e;
   }
 
   // The same from the nonzeros of a symmetric J (sparse form): row i's
@@ -249,36 +293,35 @@ struct Chain {
     return wave_sum(c);
   }
 
-  // Add dS times a staged row (LDS, 16-byte aligned, zero-padded to 64*G).
-  __device__ __forceinline__ void add_row(const T* row, T dS) {
-    const int lane = threadIdx.x & 63;
-    const T4<T>* r4 = reinterpret_cast<const T4<T>*>(row);
+  // Row pos of the couplings padded with zeros to ldp elements (a multiple of
+  // 256, at most 64 G, 16-byte aligned): a 256-element chunk is loaded whole
+  // or, beyond ldp, not at all (a wave-uniform test; the chunks up to G = 8 and
+  // the first half above always exist, because G is the least power of two).
+  __device__ __forceinline__ static void load_row(T4<T> (&x)[G / 4], const T* __restrict__ Jp,
+                                                  int pos, int ldp) {
+    const uint32_t row = (uint32_t)pos * (uint32_t)ldp;  // at most 4096 x 4096
+    const T4<T>* r4 = reinterpret_cast<const T4<T>*>(Jp + row);
+    const uint32_t lane = threadIdx.x & 63;
+    constexpr int HALF = G <= 8 ? G / 4 : G / 8;
 #pragma unroll
-    for (int g4 = 0; g4 < G / 4; ++g4) {
-      const T4<T> x = r4[(g4 << 6) + lane];
+    for (int g4 = 0; g4 < HALF; ++g4) x[g4] = r4[(g4 << 6) + lane];
+    if (HALF == G / 4 || ldp == 64 * G) {
 #pragma unroll
-      for (int q = 0; q < 4; ++q) f[4 * g4 + q] += x.v[q] * dS;
-    }
-  }
-  // Add dS times a coupling row padded with zeros to ldp elements (a
-  // multiple of 256, 16-byte aligned): a 256-element chunk is loaded whole
-  // or, beyond ldp, not at all (a wave-uniform test, no per-lane masks).
-  __device__ __forceinline__ void add_row_padded(const T* __restrict__ row, int ldp, T dS) {
-    const int lane = threadIdx.x & 63;
-    const T4<T>* r4 = reinterpret_cast<const T4<T>*>(row);
-    T4<T> x[G / 4];
-    if (ldp >= 64 * G) {
-#pragma unroll
-      for (int g4 = 0; g4 < G / 4; ++g4) x[g4] = r4[(g4 << 6) + lane];
+      for (int g4 = HALF; g4 < G / 4; ++g4) x[g4] = r4[(g4 << 6) + lane];
     } else {
 #pragma unroll
-      for (int g4 = 0; g4 < G / 4; ++g4)
+      for (int g4 = HALF; g4 < G / 4; ++g4)
         x[g4] = ((g4 << 8) < ldp) ? r4[(g4 << 6) + lane] : T4<T>{{T(0), T(0), T(0), T(0)}};
     }
+  }
+  __device__ __forceinline__ void add_row(const T4<T> (&x)[G / 4], T dS) {
 #pragma unroll
     for (int g4 = 0; g4 < G / 4; ++g4)
 #pragma unroll
-      for (int q = 0; q < 4; ++q) f[4 * g4 + q] += x[g4].v[q] * dS;
+      for (int q = 0; q < 4; ++q) f[4 * g4 + q] = fma_t(x[g4].v[q], dS, f[4 * g4 + q]);
+  }
+  __device__ __forceinline__ void flip(int pos) {
+    bits ^= (int)(threadIdx.x & 63) == lane_of(pos) ? B(1) << slot_of(pos) : B(0);
   }
 };
 
@@ -306,13 +349,33 @@ __device__ __forceinline__ double log_uniform(const double* rep, uint64_t chain,
 
 constexpr int kMaxR = 1024;
 
-// Waves per workgroup for G field registers of type T, keeping fields and
+// How a chain's sweep runs (the sweep variant of a kernel).
+//   kWide   many chains: the rows of accepted flips pass through a wave's LDS
+//           buffer of n elements to the lanes whose visits need them
+//   kBlock  few chains: the 64 x 64 couplings between the visits of a window
+//           are staged in LDS first, so a decision waits for LDS only, and the
+//           rows are added afterwards, several in flight
+//   kSparse one visit after another, an accepted flip updating the nonzeros of
+//           its ELL row
+constexpr int kWide = 0, kBlock = 1, kSparse = 2;
+
+// Waves per workgroup for `regs` VGPRs of fields per lane, keeping fields and
 // working registers inside the VGPR budget.
+constexpr int waves_of(int regs) { return regs <= 16 ? 16 : regs <= 32 ? 8 : 4; }
 template <typename T, int G>
 constexpr int kernel_waves() {
-  return G * (int)(sizeof(T) / 4) <= 16 ? 16 : G * (int)(sizeof(T) / 4) <= 32 ? 8 : 4;
+  return waves_of(G * (int)(sizeof(T) / 4));
 }
-
+// The sparse update and refresh need more registers per lane (half the waves).
+template <typename T, int G, int V>
+constexpr int pt_waves() {
+  return V == kSparse && kernel_waves<T, G>() > 4 ? kernel_waves<T, G>() / 2 : kernel_waves<T, G>();
+}
+// A wave's LDS buffer, in elements.
+template <int G, int V>
+constexpr int wave_buf() {
+  return V == kSparse ? 0 : V == kBlock ? 64 * 64 : 64 * G;
+}
 
 struct SweepCtx {
   int n, ptype, order, ref;
@@ -325,47 +388,56 @@ struct SweepCtx {
   int ell_d = 0;
 };
 
-// One sweep of one chain (simulation.py:41-76): visit order from the
+// The visits of one sweep (simulation.py:41-76): visit vi of a chain in the
 // sequential order, a Feistel permutation (per chain, or shared by all chains
-// of the sweep) or a replayed order; an accepted flip loads its coupling row
-// from global memory (L2 / Infinity Cache resident) as 16-byte vectors.
-// SP: the sparse form (an accepted flip updates the nonzeros of its ELL row),
-// a separate instantiation so that the dense kernels keep their registers.
-template <typename T, int G, bool AIS, bool SP = false>
-__device__ double sweep_direct(Chain<T, G>& ch, bool active, const T* hs, const SweepCtx& c,
-                               const T* __restrict__ Jp, int ldp, T beta, uint64_t cid,
-                               const double* rep_lr, const int* rep_perm,
-                               unsigned long long& acc, int& od) {
-  const int n = c.n, lane = threadIdx.x & 63;
-  od = 0;
-  if (!active) return 0.0;
-  // Visit slots: n, or 32 per block in the block-random order (padding
-  // slots of the last block visit nothing).
-  const bool brand = c.order == kBlockRandom && rep_perm == nullptr;
-  const int nv = brand ? kOrderBlock * ((n + kOrderBlock - 1) / kOrderBlock) : n;
+// of the sweep), the block-random order or a replayed order.
+struct Visits {
+  int nv;  // visit slots: n, or 32 per block in the block-random order
+  bool brand;
   FeistelKey fk;
-  if (brand)
-    fk = block_order_key((uint32_t)((n + kOrderBlock - 1) / kOrderBlock), c.sw, c.k0, c.k1);
-  else if (c.order != kSequential && rep_perm == nullptr)
-    fk = feistel_make((uint32_t)n,
-                      perm_keys(c.order == kRandomShared ? 0ull : cid, c.sw,
-                                c.order == kRandomShared ? kStreamShared : kStreamPerm, c.k0, c.k1));
-  double sum = 0.0;
-  for (int w = 0; w < nv; w += 64) {
-    const int vi = w + lane;
-    int pos_l = -1;
-    double lr_l = 0.0;
+  __device__ Visits(const SweepCtx& c, uint64_t cid, bool replay) {
+    brand = c.order == kBlockRandom && !replay;
+    const int nb = (c.n + kOrderBlock - 1) / kOrderBlock;
+    nv = brand ? kOrderBlock * nb : c.n;
+    if (brand)
+      fk = block_order_key((uint32_t)nb, c.sw, c.k0, c.k1);
+    else if (c.order != kSequential && !replay)
+      fk = feistel_make((uint32_t)c.n,
+                        perm_keys(c.order == kRandomShared ? 0ull : cid, c.sw,
+                                  c.order == kRandomShared ? kStreamShared : kStreamPerm, c.k0,
+                                  c.k1));
+  }
+  // The position (-1: a padding slot of the last block) and its log-uniform.
+  __device__ void at(int vi, const SweepCtx& c, uint64_t cid, const double* rep_lr,
+                     const int* rep_perm, int& pos, double& lr) const {
+    pos = -1;
+    lr = 0.0;
     if (vi < nv) {
       if (rep_perm)
-        pos_l = rep_perm[vi];
+        pos = rep_perm[vi];
       else if (brand)
-        pos_l = block_random_pos(fk, c.sw, (uint32_t)vi, n, c.k0, c.k1);
+        pos = block_random_pos(fk, c.sw, (uint32_t)vi, c.n, c.k0, c.k1);
       else
-        pos_l = (c.order == kSequential) ? vi : (int)feistel_perm(fk, (uint32_t)vi);
-      if (pos_l >= 0) lr_l = log_uniform(rep_lr, cid, c.sw, pos_l, c.k0, c.k1);
+        pos = (c.order == kSequential) ? vi : (int)feistel_perm(fk, (uint32_t)vi);
+      if (pos >= 0) lr = log_uniform(rep_lr, cid, c.sw, pos, c.k0, c.k1);
     }
+  }
+};
+
+// One sweep of one chain, one visit after another (sparse form).
+template <typename T, int G>
+__device__ double sweep_sparse(Chain<T, G>& ch, const T* hs, const SweepCtx& c, T beta,
+                               uint64_t cid, const double* rep_lr, const int* rep_perm,
+                               unsigned long long& acc) {
+  const int lane = threadIdx.x & 63;
+  const Visits vs(c, cid, rep_perm != nullptr);
+  double sum = 0.0;
+  for (int w = 0; w < vs.nv; w += 64) {
+    int pos_l;
+    double lr_l;
+    vs.at(w + lane, c, cid, rep_lr, rep_perm, pos_l, lr_l);
     const T h_l = (pos_l >= 0) ? hs[pos_l] : T(0);
-    const int cnt = min(64, nv - w);
+    const int cnt = min(64, vs.nv - w);
     for (int t = 0; t < cnt; ++t) {
       const int pos = rl(pos_l, t);
       if (pos < 0) continue;  // padding slot (wave-uniform)
@@ -374,60 +446,220 @@ __device__ double sweep_direct(Chain<T, G>& ch, bool active, const T* hs, const 
       const bool up = (rl(ch.bits, pl) >> ps) & 1;
       const T fh = rl(ch.pick(ps), pl) + rl(h_l, t);
       double dn;
-      if (decide<T, AIS>(c.ptype, up, fh, lr, (double)beta, c.ref, c.lratio, dn)) {
+      if (decide<T, false>(c.ptype, up, fh, lr, (double)beta, c.ref, c.lratio, dn)) {
         sum += -dn;
         ++acc;
-        od += up ? -1 : 1;
-        if (lane == pl) ch.bits ^= (typename Chain<T, G>::B(1) << ps);
+        ch.flip(pos);
         const T dS = (c.ptype == 0) ? (up ? T(-2) : T(2)) : (up ? T(-1) : T(1));
-        if constexpr (SP)
-          ch.add_ell(c.ell_cols + (size_t)pos * c.ell_d,
-                     static_cast<const T*>(c.ell_vals) + (size_t)pos * c.ell_d, c.ell_d, dS);
-        else
-          ch.add_row_padded(Jp + (size_t)pos * ldp, ldp, dS);
+        ch.add_ell(c.ell_cols + (size_t)pos * c.ell_d,
+                   static_cast<const T*>(c.ell_vals) + (size_t)pos * c.ell_d, c.ell_d, dS);
       }
     }
   }
   return sum;
 }
 
-// Waves per workgroup of the PT kernel: the sparse form's update and refresh
-// need more registers per lane, so it runs half as many waves.
-template <typename T, int G, bool SP>
-constexpr int pt_waves() {
-  return SP ? (kernel_waves<T, G>() > 4 ? kernel_waves<T, G>() / 2 : 4) : kernel_waves<T, G>();
+// The spin change of a flip, -+2 (ising) or -+1 (qubo), in scalar registers.
+__device__ __forceinline__ float spin_change(int ptype, bool up, float) {
+  return __uint_as_float((ptype == 0 ? 0x40000000u : 0x3F800000u) | ((uint32_t)up << 31));
+}
+__device__ __forceinline__ double spin_change(int ptype, bool up, double) {
+  return as_double((uint64_t)((ptype == 0 ? 0x40000000u : 0x3FF00000u) | ((uint32_t)up << 31))
+                   << 32);
 }
 
-template <typename T, int G, bool SP>
-__global__ __launch_bounds__((64 * pt_waves<T, G, SP>())) void plain_pt_kernel(PTParams<T> p) {
-  const int read = blockIdx.x;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, W = blockDim.x >> 6;
-  const int R = p.R, n = p.n;
-  __shared__ T s_h[kPlainMaxN];
-  __shared__ T s_bs[kMaxR];
-  __shared__ T s_beta[kMaxR];
-  __shared__ T s_E[kMaxR];
-  __shared__ long long s_bi[kMaxR];
-  __shared__ double s_ptlu[kMaxR];
-  __shared__ double s_eoff[kMaxR];  // caller's initial energy minus its f64 recomputation
-  __shared__ int s_src;
-  __shared__ T s_gE;
-  __shared__ int s_gsw, s_improved;
+// One sweep of one chain with dense rows (see the top of the file), buf the
+// wave's LDS buffer.
+// Bound: kWide by the L1 / L2 traffic of one row per accepted flip and the
+// issue of its additions; kBlock by latency, a chain of an LDS read and an f64
+// comparison per accepted flip, then the rows' loads.  Before, every visit
+// picked its field from the registers by a select tree (~100 VALU slots a
+// proposal) and waited for the row of the last flip: 512 reads of 32 replicas
+// of 1024 spins x 40 sweeps, random order, 118.0 -> 55.9 ms (kWide); 8 reads
+// of 16 replicas of 300 spins in f64 x 100 sweeps 17.8 -> 3.4 ms, one read of
+// 100 replicas of 3072 spins x 2 sweeps 944 -> 2.4 ms (kBlock, a workgroup per
+// chain; before, one workgroup for the read).
+template <typename T, int G, bool AIS, int V>
+__device__ double sweep_dense(Chain<T, G>& ch, const T* hs, const SweepCtx& c,
+                              const T* __restrict__ Jp, int ldp, T beta, uint64_t cid,
+                              const double* rep_lr, const int* rep_perm, unsigned long long& acc,
+                              int& od, T* buf) {
+  const int lane = threadIdx.x & 63;
+  const double bd = (double)beta;
+  const Visits vs(c, cid, rep_perm != nullptr);
+  od = 0;
+  double sum = 0.0;
+  for (int w = 0, cnt; w < vs.nv; w += cnt) {
+    int pos_l;
+    double lr_l;
+    vs.at(w + lane, c, cid, rep_lr, rep_perm, pos_l, lr_l);
+    cnt = min(64, vs.nv - w);
+    if (rep_perm) {  // a replayed order may repeat a position: the window ends before it
+      bool again = false;
+      for (int t = 0; t < cnt; ++t) again = again || (t < lane && pos_l == rl(pos_l, t));
+      const uint64_t dup = __ballot(again && lane < cnt);
+      if (dup) cnt = __builtin_ctzll(dup);
+      if (lane >= cnt) pos_l = -1;
+    }
+    const int pc = max(pos_l, 0);
+    const uint64_t valid = __ballot(pos_l >= 0);
+    const T h_l = hs[pc];
+    // the fields of the visits, through LDS (element i at buf[i]), and their spins
+#pragma unroll
+    for (int g4 = 0; g4 < G / 4; ++g4) {
+      T4<T> v;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) v.v[q] = ch.f[4 * g4 + q];
+      reinterpret_cast<T4<T>*>(buf)[(g4 << 6) + lane] = v;
+    }
+    wave_sync();
+    T fv = buf[pc];
+    const bool up = (shfl_bits(ch.bits, lane_of(pc)) >> slot_of(pc)) & 1;
+    const uint64_t upm = __ballot(up);
+    wave_sync();
+    if constexpr (V == kBlock) {  // row t: the couplings of visit t to every visit
+      for (int t0 = 0; t0 < cnt; t0 += 16) {
+        T v[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u)
+          v[u] = Jp[(uint32_t)max(rl(pos_l, t0 + u), 0) * (uint32_t)ldp + (uint32_t)pc];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) buf[(t0 + u) * 64 + lane] = v[u];
+      }
+      wave_sync();
+    }
+    // dn = 2 s (F + h) (ising.py:48-49) or (2x - 1)(F + h) (qubo.py:48-49)
+    const double sg = c.ptype == 0 ? (up ? 2.0 : -2.0) : (up ? 1.0 : -1.0);
+    const double refd = (AIS && c.ref == 1) ? (up ? c.lratio : -c.lratio) : 0.0;
+    const double cref = (1.0 - bd) * refd;
+    double dn;
+    auto decisions = [&]() __attribute__((always_inline)) {  // ising.py:52 / :75-83
+      dn = sg * (double)(fv + h_l);
+      const double x = bd * dn, y = AIS ? x + cref : dn, z = AIS ? y : x;
+      return __builtin_amdgcn_ballot_w64(y >= 0) | __builtin_amdgcn_ballot_w64(lr_l < z);
+    };
+    uint64_t m = decisions() & valid, taken = 0;
+    while (m) {  // the first accepted visit t of those not yet passed
+      const int t = __builtin_ctzll(m);
+      const T dS = spin_change(c.ptype, (upm >> t) & 1, T(0));
+      const double dnt = rl(dn, t);
+      taken |= 1ull << t;
+      if constexpr (V == kBlock) {
+        fv = fma_t(buf[t * 64 + lane], dS, fv);
+      } else {
+        const int pos = rl(pos_l, t);
+        T4<T> x[G / 4];
+        ch.load_row(x, Jp, pos, ldp);
+        ch.flip(pos);
+#pragma unroll
+        for (int g4 = 0; g4 < G / 4; ++g4) reinterpret_cast<T4<T>*>(buf)[(g4 << 6) + lane] = x[g4];
+        wave_sync();
+        fv = fma_t(buf[pc], dS, fv);
+        ch.add_row(x, dS);
+        wave_sync();
+      }
+      m = decisions() & valid & (~1ull << t);
+      sum += -dnt;
+    }
+    acc += (unsigned long long)__builtin_popcountll(taken);
+    od += __builtin_popcountll(taken & ~upm) - __builtin_popcountll(taken & upm);
+    if constexpr (V == kBlock) {
+      // the accepted rows in order, NB in flight; loads past the last one
+      // repeat it, so that every path issues the same loads
+      constexpr int REG = G * (int)(sizeof(T) / 4);
+      constexpr int NB = REG >= 32 ? 2 : REG >= 16 ? 4 : 8;
+      if (taken) {
+        T4<T> x[NB][G / 4];
+        uint64_t ql = taken;  // rows to load
+        int last = 0;
+        auto load_next = [&](T4<T> (&d)[G / 4]) __attribute__((always_inline)) {
+          last = ql ? rl(pos_l, __builtin_ctzll(ql)) : last;
+          ql &= ql - 1;
+          ch.load_row(d, Jp, last, ldp);
+        };
+#pragma unroll
+        for (int b = 0; b < NB; ++b) load_next(x[b]);
+        while (taken) {
+#pragma unroll
+          for (int b = 0; b < NB; ++b) {
+            if (taken) {
+              const int t = __builtin_ctzll(taken);
+              taken &= taken - 1;
+              ch.flip(rl(pos_l, t));
+              ch.add_row(x[b], spin_change(c.ptype, (upm >> t) & 1, T(0)));
+            }
+            load_next(x[b]);
+          }
+        }
+      }
+    }
+  }
+  return sum;
+}
 
-  for (int i = tid; i < n; i += blockDim.x) s_h[i] = p.h[i];
-  for (int k = tid; k < R; k += blockDim.x) {
-    s_bi[k] = p.beta_idx[(size_t)read * R + k];
-    s_E[k] = p.energies[(size_t)read * R + k];
-    s_beta[k] = p.betas[k];
+// Replica exchange of one read by one wave (utils.py:44-58): hot end first,
+// slot a = R-1-k against b = a-1 at step k.  The replica that the last pair
+// left in slot a is carried along: an exchange moves it on to b, otherwise b's
+// occupant becomes the carried one.  Lane k holds pair k's other operands, so a
+// step is a few readlanes and no memory.  E, beta, lu, bi: shared or global
+// arrays of the read; e_of(r): the energy of replica r.
+template <typename T, typename I>
+__device__ void exchange_wave(int R, const T* E, const T* beta, const double* lu, I* bi) {
+  const int lane = threadIdx.x & 63;
+  int carry = (int)bi[R - 1];
+  T ec = E[carry];
+  for (int k0 = 0; k0 < R - 1; k0 += 64) {
+    const int cnt = min(64, R - 1 - k0);
+    const int k = k0 + min(lane, cnt - 1);
+    const int a = R - 1 - k;
+    const int rb_l = (int)bi[a - 1];
+    const T eb_l = E[rb_l], db_l = (T)(beta[a] - beta[a - 1]);
+    const double lu_l = lu[k];
+    int out = 0;
+    for (int j = 0; j < cnt; ++j) {
+      const T eb = rl(eb_l, j);
+      const int rb = rl(rb_l, j);
+      const T dd = (T)(ec - eb) * rl(db_l, j);
+      const bool x = dd >= 0 || rl(lu_l, j) < (double)dd;
+      if (lane == j) out = x ? rb : carry;
+      if (!x) {
+        carry = rb;
+        ec = eb;
+      }
+    }
+    if (lane < cnt) bi[a] = (I)out;
   }
-  if (tid == 0) {
-    s_gE = p.energies[(size_t)read * R];  // simulation.py:205
-    s_gsw = 0;
-    s_improved = 0;
+  if (lane == 0) bi[0] = (I)carry;
+}
+
+// PT log-uniform of one pair (utils.py:57): replayed or drawn.
+template <typename T>
+__device__ __forceinline__ double pt_log_uniform(const PTParams<T>& p, int read, int s, int k) {
+  if (p.rep_pt) return p.rep_pt[((size_t)read * p.S + s) * (p.R - 1) + k];
+  return log_u32(pick_word(pt_block((uint64_t)read, (uint64_t)s + p.sweep_offset, (uint32_t)k,
+                                    p.k0, p.k1),
+                           (uint32_t)k & 3u));
+}
+
+// log-omega of one sweep (ais.py:99-112) over the ascending ladder.
+template <typename T, typename I>
+__device__ double log_omega_of(int R, const int* bsort, const T* beta, const T* E, const I* bi) {
+  double lw = 0.0, bold = 0.0;
+  for (int r = 1; r < R; ++r) {
+    const int q = bsort[r];
+    const T be = beta[q];
+    const T en = E[bi[q]];
+    const T a = -be * en;
+    lw += (double)a - (-bold * (double)en);
+    bold = (double)be;
   }
-  __syncthreads();
+  return lw;
+}
+
+template <typename T>
+__device__ SweepCtx sweep_ctx(const PTParams<T>& p) {
   SweepCtx c;
-  c.n = n;
+  c.n = p.n;
   c.ptype = p.ptype;
   c.order = p.order;
   c.ref = 0;
@@ -437,7 +669,73 @@ __global__ __launch_bounds__((64 * pt_waves<T, G, SP>())) void plain_pt_kernel(P
   c.ell_cols = p.ell_cols;
   c.ell_vals = p.ell_vals;
   c.ell_d = p.ell_d;
+  return c;
+}
+
+// LDS of plain_pt_kernel (dynamic): the wave buffers, h, and the read's
+// replicas.
+template <typename T>
+struct PTLds {
+  T *buf, *h, *bs, *beta, *E, *bE;
+  double *lu, *eoff;
+  int *bi, *bsw;
+  __host__ __device__ static size_t bytes(int buf_elems, int n, int R) {
+    return (size_t)(buf_elems + ((n + 1) & ~1) + 4 * ((R + 1) & ~1)) * sizeof(T) +
+           (size_t)R * (2 * sizeof(double) + 2 * sizeof(int));
+  }
+  __device__ PTLds(char* base, int buf_elems, int n, int R) {
+    const int Re = (R + 1) & ~1;  // every array 8-byte aligned
+    buf = reinterpret_cast<T*>(base);
+    h = buf + buf_elems;
+    bs = h + ((n + 1) & ~1);
+    beta = bs + Re;
+    E = beta + Re;
+    bE = E + Re;
+    lu = reinterpret_cast<double*>(bE + Re);
+    eoff = lu + R;
+    bi = reinterpret_cast<int*>(eoff + R);
+    bsw = bi + R;
+  }
+};
+
+// All sweeps of one read: W waves carry its R replicas (each wave its own for
+// the whole run when R <= W, else one after another through global memory)
+// and meet after every sweep for the exchanges.
+template <typename T, int G, int V>
+__global__ __launch_bounds__((64 * pt_waves<T, G, V>())) void plain_pt_kernel(PTParams<T> p) {
+  const int read = blockIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63, W = blockDim.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int R = p.R, n = p.n;
+  extern __shared__ __align__(16) char lds[];
+  const PTLds<T> L(lds, W * wave_buf<G, V>(), n, R);
+  __shared__ int s_src;
+  __shared__ T s_gE;
+  __shared__ int s_gsw, s_improved;
+  T* buf = L.buf + wave * wave_buf<G, V>();
+
+  for (int i = tid; i < n; i += blockDim.x) L.h[i] = p.h[i];
+  for (int k = tid; k < R; k += blockDim.x) {
+    L.bi[k] = k;  // beta_idx = arange(R) (sa.py:325)
+    L.E[k] = p.energies[(size_t)read * R + k];
+    L.bE[k] = L.E[k];  // simulation.py:143-145
+    L.bsw[k] = 0;
+    L.beta[k] = p.betas[k];
+  }
+  if (tid == 0) {
+    s_gE = p.energies[(size_t)read * R];  // simulation.py:205
+    s_gsw = 0;
+    s_improved = 0;
+  }
+  __syncthreads();
+  SweepCtx c = sweep_ctx(p);
   unsigned long long acc = 0;
+  const bool own = R <= W;  // the wave's replica stays in registers
+  Chain<T, G> ch;
+  if (own && wave < R) {
+    const size_t off = ((size_t)read * R + wave) * n;
+    ch.load_spins(p.spins + off, n);
+  }
   for (int s = 0; s < p.S; ++s) {
     c.sw = (uint64_t)s + p.sweep_offset;
     // Local fields F = J s recomputed in f64 (rounded once) at the start and
@@ -449,70 +747,64 @@ __global__ __launch_bounds__((64 * pt_waves<T, G, SP>())) void plain_pt_kernel(P
     // other energies), so the drift of incrementally updated fields does not
     // accumulate.  Integer couplings are exact either way: the reset then
     // leaves the value unchanged.
-    if (s == 0 || (p.refresh > 0 && s % p.refresh == 0)) {
-      for (int r = wave; r < R; r += W) {
-        Chain<T, G> ch;
-        const size_t off = ((size_t)read * R + r) * n;
-        ch.load(p.fields + off, p.spins + off, n);
-        double ex;
-        if constexpr (SP)
-          ex = ch.refresh_ell(p.ell_cols, p.ell_vals, p.ell_d, s_h, n, p.ptype);
-        else
-          ex = ch.refresh(p.Jt, s_h, n, p.ptype);
-        ch.store(p.fields + off, p.spins + off, n, p.ptype);
-        if (lane == 0) {
-          if (s == 0)
-            s_eoff[r] = (double)s_E[r] - ex;
-          else
-            s_E[r] = (T)(ex + s_eoff[r]);
-        }
-      }
-    }
-    for (int k = tid; k < R; k += blockDim.x) s_bs[s_bi[k]] = s_beta[k];  // simulation.py:151-152
+    const bool fresh = s == 0 || (p.refresh > 0 && s % p.refresh == 0);
+    for (int k = tid; k < R; k += blockDim.x) L.bs[L.bi[k]] = L.beta[k];  // simulation.py:151-152
     // PT log-uniforms, one per pair, drawn in parallel ahead of the serial walk.
     if (p.use_pt)
-      for (int k = tid; k < R - 1; k += blockDim.x) {
-        double lu;
-        if (p.rep_pt)
-          lu = p.rep_pt[((size_t)read * p.S + s) * (R - 1) + k];
-        else
-          lu = log_u32(pick_word(pt_block((uint64_t)read, c.sw, (uint32_t)k, p.k0, p.k1),
-                                 (uint32_t)k & 3u));
-        s_ptlu[k] = lu;
-      }
+      for (int k = tid; k < R - 1; k += blockDim.x) L.lu[k] = pt_log_uniform(p, read, s, k);
     __syncthreads();
     for (int r = wave; r < R; r += W) {  // replicas of this read (simulation.py:154-164)
-      Chain<T, G> ch;
       const size_t off = ((size_t)read * R + r) * n;
-      ch.load(p.fields + off, p.spins + off, n);
+      if (!own) {
+        if (s == 0)
+          ch.load_spins(p.spins + off, n);
+        else
+          ch.load(p.fields + off, p.spins + off, n);
+      }
+      if (fresh) {
+        double ex;
+        if constexpr (V == kSparse)
+          ex = ch.refresh_ell(p.ell_cols, p.ell_vals, p.ell_d, L.h, n, p.ptype);
+        else
+          ex = ch.refresh(p.Jp, p.ldp, L.h, n, p.ptype);
+        if (lane == 0) {
+          if (s == 0)
+            L.eoff[r] = (double)L.E[r] - ex;
+          else
+            L.E[r] = (T)(ex + L.eoff[r]);
+        }
+        wave_sync();
+      }
       const size_t rb = (((size_t)read * p.S + s) * R + r) * (size_t)n;
+      const uint64_t cid = (uint64_t)read * R + r;
+      const double* rlr = p.rep_lr ? p.rep_lr + rb : nullptr;
+      const int* rpm = p.rep_perm ? p.rep_perm + rb : nullptr;
+      double d;
       int od;
-      const double d = sweep_direct<T, G, false, SP>(ch, true, s_h, c, p.Jp, p.ldp, s_bs[r],
-                                                 (uint64_t)read * R + r,
-                                                 p.rep_lr ? p.rep_lr + rb : nullptr,
-                                                 p.rep_perm ? p.rep_perm + rb : nullptr, acc, od);
-      ch.store(p.fields + off, p.spins + off, n, p.ptype);
-      const T en = (T)((double)s_E[r] + d);  // simulation.py:157-158
-      if (lane == 0) s_E[r] = en;
-      if (p.best_sem == 0) {
-        const size_t bi = (size_t)read * R + r;
-        if (en < p.best_rep_e[bi]) {  // simulation.py:161-164
-          ch.store_spins(p.best_rep + bi * n, n, p.ptype);
-          if (lane == 0) {
-            p.best_rep_e[bi] = en;
-            p.best_rep_sw[bi] = s;
-          }
+      if constexpr (V == kSparse)
+        d = sweep_sparse<T, G>(ch, L.h, c, L.bs[r], cid, rlr, rpm, acc);
+      else
+        d = sweep_dense<T, G, false, V>(ch, L.h, c, p.Jp, p.ldp, L.bs[r], cid, rlr, rpm, acc, od,
+                                        buf);
+      if (!own || s + 1 == p.S || p.best_sem == 1) ch.store(p.fields + off, p.spins + off, n, p.ptype);
+      const T en = (T)((double)L.E[r] + d);  // simulation.py:157-158
+      if (p.best_sem == 0 && en < L.bE[r]) {  // simulation.py:161-164
+        ch.store_spins(p.best_rep + off, n, p.ptype);
+        if (lane == 0) {
+          L.bE[r] = en;
+          L.bsw[r] = s;
         }
       }
+      if (lane == 0) L.E[r] = en;
     }
     __syncthreads();
-    if (tid == 0) {
-      if (p.best_sem == 1) {  // simulation.py:222-225 in replica order
+    if (wave == 0) {
+      if (p.best_sem == 1 && lane == 0) {  // simulation.py:222-225 in replica order
         int src = -1;
         T cur = s_gE;
         for (int k = 0; k < R; ++k)
-          if (s_E[k] < cur) {
-            cur = s_E[k];
+          if (L.E[k] < cur) {
+            cur = L.E[k];
             src = k;
           }
         if (src >= 0) {
@@ -522,28 +814,11 @@ __global__ __launch_bounds__((64 * pt_waves<T, G, SP>())) void plain_pt_kernel(P
         }
         s_src = src;
       }
-      if (p.use_pt) {  // utils.py:44-58
-        for (int k = 0; k < R - 1; ++k) {
-          const int a = R - k - 1, b = R - k - 2;
-          const T dd = (T)(s_E[s_bi[a]] - s_E[s_bi[b]]) * (T)(s_beta[a] - s_beta[b]);
-          if (dd >= 0 || s_ptlu[k] < (double)dd) {
-            const long long t = s_bi[a];
-            s_bi[a] = s_bi[b];
-            s_bi[b] = t;
-          }
-        }
-      }
-      if (p.logw && p.log_omegas) {  // ais.py:99-112 over the ascending ladder
-        double lw = 0.0, bold = 0.0;
-        for (int r = 1; r < R; ++r) {
-          const int q = p.bsort[r];
-          const T be = s_beta[q];
-          const T en = s_E[s_bi[q]];
-          const T a = -be * en;
-          lw += (double)a - (-bold * (double)en);
-          bold = (double)be;
-        }
-        p.log_omegas[(size_t)read * p.S + s] = lw;
+      if (p.use_pt) exchange_wave<T, int>(R, L.E, L.beta, L.lu, L.bi);
+      if (p.logw && p.log_omegas) {
+        wave_sync();
+        if (lane == 0)
+          p.log_omegas[(size_t)read * p.S + s] = log_omega_of<T, int>(R, p.bsort, L.beta, L.E, L.bi);
       }
     }
     __syncthreads();
@@ -555,8 +830,8 @@ __global__ __launch_bounds__((64 * pt_waves<T, G, SP>())) void plain_pt_kernel(P
 
   // Outputs.
   for (int k = tid; k < R; k += blockDim.x) {
-    p.beta_idx[(size_t)read * R + k] = s_bi[k];
-    p.energies[(size_t)read * R + k] = s_E[k];
+    p.beta_idx[(size_t)read * R + k] = L.bi[k];
+    p.energies[(size_t)read * R + k] = L.E[k];
   }
   if (lane == 0 && p.accepted) atomicAdd(p.accepted + read, acc);
   __syncthreads();
@@ -564,10 +839,10 @@ __global__ __launch_bounds__((64 * pt_waves<T, G, SP>())) void plain_pt_kernel(P
     if (tid == 0) {
       int bp = 0;
       for (int k = 1; k < R; ++k)
-        if (p.best_rep_e[(size_t)read * R + k] < p.best_rep_e[(size_t)read * R + bp]) bp = k;
+        if (L.bE[k] < L.bE[bp]) bp = k;
       s_src = bp;
-      p.best_energy[read] = p.best_rep_e[(size_t)read * R + bp];
-      p.best_sweeps[read] = p.best_rep_sw[(size_t)read * R + bp];
+      p.best_energy[read] = L.bE[bp];
+      p.best_sweeps[read] = L.bsw[bp];
     }
     __syncthreads();
     const int8_t* src = p.best_rep + ((size_t)read * R + s_src) * n;
@@ -584,21 +859,171 @@ __global__ __launch_bounds__((64 * pt_waves<T, G, SP>())) void plain_pt_kernel(P
   }
 }
 
+// ---- one workgroup (one wave) per chain ----
+
+// F = J s and the energy of a chain from its f64 sums (chain_sums_kernel), as
+// Chain::refresh makes them; s: the sweep before which this happens.
+template <typename T, int G>
+__global__ __launch_bounds__(64) void chain_refresh_kernel(PTParams<T> p, int s) {
+  const size_t chain = blockIdx.x;
+  const int lane = threadIdx.x, n = p.n;
+  Chain<T, G> ch;
+  ch.load_spins(p.spins + chain * n, n);
+  const double* sums = p.sums + chain * n;
+  double e = 0.0;
+#pragma unroll
+  for (int g4 = 0; g4 < G / 4; ++g4) {
+    double a[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int i = (g4 << 8) + (lane << 2) + q;
+      a[q] = i < n ? sums[i] : 0.0;
+    }
+    e = ch.put_fields(g4, a, p.h, n, p.ptype, e);
+  }
+  e = wave_sum(e);
+  ch.store(p.fields + chain * n, p.spins + chain * n, n, p.ptype);
+  if (lane == 0) {
+    if (s == 0)
+      p.eoff[chain] = (double)p.energies[chain] - e;
+    else
+      p.energies[chain] = (T)(e + p.eoff[chain]);
+  }
+}
+
+// Sweeps [s0, s1) of one chain (several only when nothing of a sweep's end
+// concerns other chains).
+template <typename T, int G>
+__global__ __launch_bounds__(64) void chain_sweep_kernel(PTParams<T> p, int s0, int s1) {
+  __shared__ T buf[64 * 64];
+  const int chain = blockIdx.x, lane = threadIdx.x, n = p.n;
+  const size_t off = (size_t)chain * n;
+  Chain<T, G> ch;
+  ch.load(p.fields + off, p.spins + off, n);
+  SweepCtx c = sweep_ctx(p);
+  const T beta = p.chain_beta[chain];
+  T E = p.energies[chain], bE = p.best_rep_e[chain];
+  const int read = chain / p.R, r = chain - read * p.R;
+  unsigned long long acc = 0;
+  for (int s = s0; s < s1; ++s) {
+    c.sw = (uint64_t)s + p.sweep_offset;
+    const size_t rb = (((size_t)read * p.S + s) * p.R + r) * (size_t)n;
+    int od;
+    const double d = sweep_dense<T, G, false, kBlock>(
+        ch, p.h, c, p.Jp, p.ldp, beta, (uint64_t)chain, p.rep_lr ? p.rep_lr + rb : nullptr,
+        p.rep_perm ? p.rep_perm + rb : nullptr, acc, od, buf);
+    E = (T)((double)E + d);  // simulation.py:157-158
+    if (p.best_sem == 0 && E < bE) {  // simulation.py:161-164
+      bE = E;
+      ch.store_spins(p.best_rep + off, n, p.ptype);
+      if (lane == 0) {
+        p.best_rep_e[chain] = E;
+        p.best_rep_sw[chain] = s;
+      }
+    }
+  }
+  ch.store(p.fields + off, p.spins + off, n, p.ptype);
+  if (lane == 0) {
+    p.energies[chain] = E;
+    if (p.accepted) atomicAdd(p.accepted + read, acc);
+  }
+}
+
+// The end of sweep s of a read whose chains run in workgroups of their own
+// (s < 0: before the first sweep, which only takes the betas): best state in
+// replica order, exchanges, log-omega and the chains' new betas, as in
+// plain_pt_kernel.
+template <typename T>
+__global__ __launch_bounds__(256) void chain_exchange_kernel(PTParams<T> p, int s) {
+  __shared__ T s_E[kMaxR], s_beta[kMaxR];
+  __shared__ int s_bi[kMaxR];
+  __shared__ double s_lu[kMaxR];
+  __shared__ int s_src;
+  const int read = blockIdx.x, tid = threadIdx.x, R = p.R, n = p.n;
+  const size_t c0 = (size_t)read * R;
+  for (int k = tid; k < R; k += 256) {
+    s_E[k] = p.energies[c0 + k];
+    s_beta[k] = p.betas[k];
+    s_bi[k] = s < 0 ? k : (int)p.beta_idx[c0 + k];
+    if (s >= 0 && p.use_pt && k < R - 1) s_lu[k] = pt_log_uniform(p, read, s, k);
+  }
+  __syncthreads();
+  if (tid < 64) {
+    if (tid == 0 && p.best_sem == 1) {  // simulation.py:222-225 in replica order
+      T cur = s < 0 ? s_E[0] : p.best_energy[read];
+      int src = -1;
+      if (s >= 0)
+        for (int k = 0; k < R; ++k)
+          if (s_E[k] < cur) {
+            cur = s_E[k];
+            src = k;
+          }
+      if (s < 0 || src >= 0) {
+        p.best_energy[read] = cur;
+        p.best_sweeps[read] = s < 0 ? 0 : s;
+        if (src >= 0) p.best_rep_sw[c0] = 1;  // a state has been copied
+      }
+      s_src = src;
+    }
+    if (s >= 0) {
+      if (p.use_pt) exchange_wave<T, int>(R, s_E, s_beta, s_lu, s_bi);
+      wave_sync();
+      if (p.logw && p.log_omegas && tid == 0)
+        p.log_omegas[(size_t)read * p.S + s] = log_omega_of<T, int>(R, p.bsort, s_beta, s_E, s_bi);
+    }
+  }
+  __syncthreads();
+  if (p.best_sem == 1 && s_src >= 0) {
+    const int8_t* src = p.spins + (c0 + s_src) * n;
+    for (int i = tid; i < n; i += 256) p.best_state[(size_t)read * n + i] = src[i];
+  }
+  for (int k = tid; k < R; k += 256) {
+    p.beta_idx[c0 + k] = s_bi[k];
+    p.chain_beta[c0 + s_bi[k]] = s_beta[k];  // simulation.py:151-152
+  }
+}
+
+// The best of a read after the last sweep.
+template <typename T>
+__global__ __launch_bounds__(256) void chain_best_kernel(PTParams<T> p) {
+  const int read = blockIdx.x, n = p.n, R = p.R;
+  const size_t c0 = (size_t)read * R;
+  int bp = 0;
+  const int8_t* from = p.spins;  // never improved: the view of states[0] (simulation.py:204)
+  if (p.best_sem == 0) {  // simulation.py:174-177, first minimum wins
+    for (int k = 1; k < R; ++k)
+      if (p.best_rep_e[c0 + k] < p.best_rep_e[c0 + bp]) bp = k;
+    if (threadIdx.x == 0) {
+      p.best_energy[read] = p.best_rep_e[c0 + bp];
+      p.best_sweeps[read] = p.best_rep_sw[c0 + bp];
+    }
+    from = p.best_rep;
+  } else if (p.best_rep_sw[c0]) {
+    return;
+  }
+  for (int i = threadIdx.x; i < n; i += 256)
+    p.best_state[(size_t)read * n + i] = from[(c0 + bp) * n + i];
+}
+
 // AIS: each wave carries one chain through the whole beta schedule
 // (simulation.py:266-317); chains are independent, so there are no barriers
 // after h is staged.
-template <typename T, int G>
-__global__ __launch_bounds__((64 * kernel_waves<T, G>())) void plain_ais_kernel(AISParams<T> p) {
-  __shared__ T s_h[kPlainMaxN];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, W = blockDim.x >> 6;
+template <typename T, int G, int V>
+__global__ __launch_bounds__(64 * (V == kBlock ? 1 : kernel_waves<T, G>())) void plain_ais_kernel(
+    AISParams<T> p) {
+  __shared__ T s_h[64 * G];
+  __shared__ T s_buf[(V == kBlock ? 1 : kernel_waves<T, G>()) * wave_buf<G, V>()];
+  const int tid = threadIdx.x, lane = tid & 63, W = blockDim.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = p.n;
   for (int i = tid; i < n; i += blockDim.x) s_h[i] = p.h[i];
   __syncthreads();
   const int chain = blockIdx.x * W + wave;
   if (chain >= p.chains) return;
+  T* buf = s_buf + wave * wave_buf<G, V>();
   Chain<T, G> ch;
-  ch.load(p.fields + (size_t)chain * n, p.spins + (size_t)chain * n, n);
-  double E = ch.refresh(p.Jt, s_h, n, p.ptype);
+  ch.load_spins(p.spins + (size_t)chain * n, n);
+  double E = ch.refresh(p.Jp, p.ldp, s_h, n, p.ptype);
   int ones = ch.count_up(n);
   SweepCtx c;
   c.n = n;
@@ -618,16 +1043,18 @@ __global__ __launch_bounds__((64 * kernel_waves<T, G>())) void plain_ais_kernel(
     // (simulation.py:309); here fields and energy are recomputed in f64
     // every `refresh` steps and updated by the accepted changes in between,
     // which bounds the drift of float couplings.
-    if (t > 0 && p.refresh > 0 && t % p.refresh == 0) E = ch.refresh(p.Jt, s_h, n, p.ptype);
+    if (t > 0 && p.refresh > 0 && t % p.refresh == 0)
+      E = ch.refresh(p.Jp, p.ldp, s_h, n, p.ptype);
     if (p.ordering == 1) {  // Neal's ordering: weight before the transition
       const double refE = (p.ref == 1) ? -((double)(n - ones) * p.lp + (double)ones * p.l1p) : 0.0;
       lw += (-bd * E - (1.0 - bd) * refE) - (-bold * E - (1.0 - bold) * refE);
     }
     const size_t rb = ((size_t)chain * p.nt + t) * (size_t)n;
     int od;
-    const double d = sweep_direct<T, G, true>(ch, true, s_h, c, p.Jp, p.ldp, beta, (uint64_t)chain,
-                                              p.rep_lr ? p.rep_lr + rb : nullptr,
-                                              p.rep_perm ? p.rep_perm + rb : nullptr, acc, od);
+    const double d = sweep_dense<T, G, true, V>(ch, p.h, c, p.Jp, p.ldp, beta, (uint64_t)chain,
+                                                p.rep_lr ? p.rep_lr + rb : nullptr,
+                                                p.rep_perm ? p.rep_perm + rb : nullptr, acc, od,
+                                                buf);
     E += d;
     ones += od;
     if (p.ordering == 0) {  // simulation.py:309-314, after the transition
@@ -803,26 +1230,101 @@ int regs_for(int n) {
   return g;
 }
 
+// J s in f64 of every chain (the input of chain_refresh_kernel).
+template <typename T>
+__global__ __launch_bounds__(256) void chain_sums_kernel(const T* __restrict__ Jt,
+                                                         const int8_t* __restrict__ spins, int n,
+                                                         int count, int ptype, double* sums) {
+  double f[4][1];
+  const int s0 = blockIdx.x * 4, i = blockIdx.y * 256 + threadIdx.x;
+  field_sums<T, 4, 1, false>(Jt, spins, n, count, s0, blockIdx.y * 256,
+                             ptype == 0 ? 0xBFF00000u : 0u, f);
+  if (i >= n) return;
+#pragma unroll
+  for (int b = 0; b < 4; ++b)
+    if (s0 + b < count) sums[(size_t)(s0 + b) * n + i] = f[b][0];
+}
+
+// Whether anything at the end of a sweep concerns other chains of the read.
+template <typename T>
+bool coupled_sweeps(const PTParams<T>& p) {
+  return (p.use_pt && p.R > 1) || (p.logw && p.log_omegas) || p.best_sem == 1;
+}
+
+template <typename T, int G, int V>
+hipError_t launch_pt_read(const PTParams<T>& p, hipStream_t st) {
+  const int W = min(p.R, pt_waves<T, G, V>());
+  const size_t lds = PTLds<T>::bytes(W * wave_buf<G, V>(), p.n, p.R);
+  hipLaunchKernelGGL((plain_pt_kernel<T, G, V>), dim3(p.reads), dim3(64 * W), lds, st, p);
+  return hipGetLastError();
+}
+
+template <typename T, int G>
+hipError_t launch_pt_chains(const PTParams<T>& p, hipStream_t st) {
+  const int chains = p.reads * p.R;
+  const bool coupled = coupled_sweeps(p);
+  hipLaunchKernelGGL((chain_exchange_kernel<T>), dim3(p.reads), dim3(256), 0, st, p, -1);
+  for (int s = 0; s < p.S;) {
+    if (s == 0 || (p.refresh > 0 && s % p.refresh == 0)) {
+      hipLaunchKernelGGL((chain_sums_kernel<T>), dim3((chains + 3) / 4, (p.n + 255) / 256),
+                         dim3(256), 0, st, p.Jt, p.spins, p.n, chains, p.ptype, p.sums);
+      hipLaunchKernelGGL((chain_refresh_kernel<T, G>), dim3(chains), dim3(64), 0, st, p, s);
+    }
+    int e = coupled ? s + 1 : p.S;
+    if (p.refresh > 0) e = min(e, s + p.refresh - s % p.refresh);
+    hipLaunchKernelGGL((chain_sweep_kernel<T, G>), dim3(chains), dim3(64), 0, st, p, s, e);
+    if (coupled) hipLaunchKernelGGL((chain_exchange_kernel<T>), dim3(p.reads), dim3(256), 0, st, p, s);
+    s = e;
+    const hipError_t le = hipGetLastError();
+    if (le != hipSuccess) return le;
+  }
+  hipLaunchKernelGGL((chain_best_kernel<T>), dim3(p.reads), dim3(256), 0, st, p);
+  return hipGetLastError();
+}
+
 template <typename T, int G>
 hipError_t launch_pt_shape(const PTParams<T>& p, hipStream_t st) {
-  if (p.ell_d > 0) {
-    const int W = min(p.R, pt_waves<T, G, true>());
-    hipLaunchKernelGGL((plain_pt_kernel<T, G, true>), dim3(p.reads), dim3(64 * W), 0, st, p);
+  if (p.ell_d > 0) return launch_pt_read<T, G, kSparse>(p, st);
+  if (p.plan == kPlanChains) return launch_pt_chains<T, G>(p, st);
+  return launch_pt_read<T, G, kWide>(p, st);
+}
+
+// AIS chains are independent: a workgroup each with staged windows while two
+// fit a compute unit, else kWide waves spread evenly over the device.
+template <typename T, int G>
+hipError_t launch_ais_shape(const AISParams<T>& p, hipStream_t st) {
+  const int cus = device_cus();
+  if (p.chains <= 2 * cus) {
+    hipLaunchKernelGGL((plain_ais_kernel<T, G, kBlock>), dim3(p.chains), dim3(64), 0, st, p);
   } else {
-    const int W = min(p.R, pt_waves<T, G, false>());
-    hipLaunchKernelGGL((plain_pt_kernel<T, G, false>), dim3(p.reads), dim3(64 * W), 0, st, p);
+    const int W = min(kernel_waves<T, G>(), (p.chains + cus - 1) / cus);
+    hipLaunchKernelGGL((plain_ais_kernel<T, G, kWide>), dim3((p.chains + W - 1) / W), dim3(64 * W),
+                       0, st, p);
   }
   return hipGetLastError();
 }
 
-template <typename T, int G>
-hipError_t launch_ais_shape(const AISParams<T>& p, hipStream_t st) {
-  const int W = kernel_waves<T, G>();
-  hipLaunchKernelGGL((plain_ais_kernel<T, G>), dim3((p.chains + W - 1) / W), dim3(64 * W), 0, st, p);
-  return hipGetLastError();
-}
-
 }  // namespace
+
+// A workgroup per chain when its rounds over the device (8 chains per compute
+// unit, 4 in f64, before they slow each other down) are fewer than the rounds
+// of a workgroup per read over its replicas; with one round each, when the
+// chains leave most of the device idle anyway and a sweep is long beside the
+// two launches it costs.  Microseconds a sweep, per read / per chain: f32 n =
+// 1024, 64 reads of 32: 585 / 442; 1 read of 32: 566 / 209; 32 reads of 16: 313
+// / 237, of n = 200: 40 / 46; 128 reads of 16: 323 / 436; 512 reads of 4: 259 /
+// 446; f64 n = 500, 8 reads of 16: 108 / 89.
+int plan_plain(int n, int reads, int R, int elem) {
+  const int64_t chains = (int64_t)reads * R;
+  const int G = regs_for(n);
+  const int W = elem == 8 ? waves_of(2 * G) : waves_of(G);
+  const int rounds = (R + W - 1) / W;
+  const int64_t per = (int64_t)device_cus() * (elem == 8 ? 4 : 8);
+  const int64_t crounds = (chains + per - 1) / per;
+  if (crounds < rounds) return kPlanChains;
+  return chains <= 2 * device_cus() && (int64_t)n * R * (elem / 4) >= 8000 ? kPlanChains
+                                                                           : kPlanReads;
+}
 
 template <typename T>
 hipError_t launch_plain_pt(const PTParams<T>& p, hipStream_t st) {
@@ -833,7 +1335,8 @@ hipError_t launch_plain_pt(const PTParams<T>& p, hipStream_t st) {
     case 8: return launch_pt_shape<T, 8>(p, st);
     case 16: return launch_pt_shape<T, 16>(p, st);
     case 32: return launch_pt_shape<T, 32>(p, st);
-    case 64: return launch_pt_shape<T, 64>(p, st);
+    case 64:
+      if constexpr (sizeof(T) == 4) return launch_pt_shape<T, 64>(p, st);
     default: return hipErrorInvalidValue;
   }
 }
@@ -846,7 +1349,8 @@ hipError_t launch_plain_ais(const AISParams<T>& p, hipStream_t st) {
     case 8: return launch_ais_shape<T, 8>(p, st);
     case 16: return launch_ais_shape<T, 16>(p, st);
     case 32: return launch_ais_shape<T, 32>(p, st);
-    case 64: return launch_ais_shape<T, 64>(p, st);
+    case 64:
+      if constexpr (sizeof(T) == 4) return launch_ais_shape<T, 64>(p, st);
     default: return hipErrorInvalidValue;
   }
 }
