@@ -60,14 +60,21 @@ __device__ __forceinline__ void bracket_factors(float beta, float& cb, float& c0
   cb = 0.69314718055994531f * inv_b;
   c0 = 9.62e-7f * inv_b;
 }
-__device__ __forceinline__ void accept_bounds_f(uint32_t w, float cb, float c0, float& lo,
-                                                float& hi) {
+__device__ __forceinline__ float accept_log2(uint32_t w) {
   // (w + 0.5) 2^-32 rounded as in accept_bounds (scaling by 2^-32 is exact)
   const float uf = __builtin_fmaf((float)w, 2.3283064365386963e-10f, 1.1641532182693481e-10f);
-  const float q = __builtin_amdgcn_logf(uf) * cb;
+  return __builtin_amdgcn_logf(uf);
+}
+__device__ __forceinline__ void accept_bounds_l(float log2u, float cb, float c0, float& lo,
+                                                float& hi) {
+  const float q = log2u * cb;
   const float m = __builtin_fmaf(fabsf(q), 4.27e-6f, c0);
   hi = q + m;
   lo = q - m;
+}
+__device__ __forceinline__ void accept_bounds_f(uint32_t w, float cb, float c0, float& lo,
+                                                float& hi) {
+  accept_bounds_l(accept_log2(w), cb, c0, lo, hi);
 }
 
 // The exact test (pysa/ising.py:52) for the rare dn inside the bracket.

@@ -661,27 +661,32 @@ BlockedPlan plan_blocked(const BlockedProblem& b, int n, int reads, int R, int o
   pl.groups = (reads + (64 / R) - 1) / (64 / R);
   pl.kw = 1;
   while (pl.kw < 4 && 2 * pl.kw <= pl.nblk && pl.groups * pl.kw < 1024) pl.kw *= 2;
-  // The pipelined kernel (proposal wave + six matrix waves) takes every
-  // problem of at least three blocks; PYSA_AMD_BLOCKED_SPLITK=1 selects the
-  // split-K kernel instead (kept for small problems and comparisons).
+  // The pipelined kernel takes every problem of two blocks or more;
+  // PYSA_AMD_BLOCKED_SPLITK=1 selects the split-K kernel instead (kept for one
+  // block and for comparisons).
   static const bool force_splitk = [] {
     const char* e = getenv("PYSA_AMD_BLOCKED_SPLITK");
     return e && e[0] == '1';
   }();
-  // The problem's launch shape (pysa_amd_problem_set_shape) picks the kernel
-  // where the size allows both; the split-K kernel has no block-random order.
+  // The problem's launch shape (pysa_amd_problem_set_shape) picks the kernel;
+  // the split-K kernel has no block-random order.
   const bool want_splitk = force_splitk || b.shape_kernel == 2;
-  pl.pipe = order == kBlockRandom || (pl.nblk >= kPipeMW && (b.shape_kernel == 1 || !want_splitk));
-  // Tiles of 32 replicas per workgroup of the pipelined kernel: two, unless
-  // two-tile groups leave compute units idle and a read fits one tile (one
-  // workgroup per CU either way: LDS and registers hold one).
-  const int groups2 = (reads + (64 / R) - 1) / (64 / R);
+  // It reads its schedule two steps ahead, across at most one sweep's end, so
+  // it needs two blocks.
+  pl.pipe = order == kBlockRandom || (pl.nblk >= 2 && (b.shape_kernel == 1 || !want_splitk));
+  // Tiles of 32 replicas per workgroup of the pipelined kernel (one workgroup
+  // per CU either way): the fewer rounds over the device, a one-tile block step
+  // taking about 18 / 25 of a two-tile one (n = 1024: 2.7 and 3.8 us).
   if (R > 32)
     pl.nt = 2;
   else if (b.shape_tiles == 1 || b.shape_tiles == 2)
     pl.nt = b.shape_tiles;
-  else
-    pl.nt = groups2 < device_cus() ? 1 : 2;
+  else {
+    const int cus = device_cus();
+    const int r1 = ((reads + 32 / R - 1) / (32 / R) + cus - 1) / cus;
+    const int r2 = ((reads + 64 / R - 1) / (64 / R) + cus - 1) / cus;
+    pl.nt = 18 * r1 <= 25 * r2 ? 1 : 2;
+  }
   if (pl.pipe) pl.groups = (reads + (32 * pl.nt / R) - 1) / (32 * pl.nt / R);
   pl.kbp = (pl.nblk + kPipeMW - 1) / kPipeMW;
   pl.nwp = 4;
@@ -1030,12 +1035,13 @@ int run_blocked_ais(BlockedProblem& b, const void* dJ, const void* dJt, const vo
     for (int i = 0; i < n; ++i)
       if (hh[i] != 0.f) b.h_zero = 0;
   }
-  // one chain per read (R = 1: the chain index is the oracle's), two tiles
-  // of 32 chains per workgroup on the pipelined kernel
+  // one chain per read (R = 1: the chain index is the oracle's); tiles of 32
+  // chains on the pipelined kernel, one per workgroup while each gets a compute
+  // unit of its own (its block step is the shorter one), else two
   BlockedPlan pl = plan_blocked(b, n, chains, 1, order, pieces);
   pl.pipe = true;
-  pl.nt = 2;
-  pl.groups = (chains + 63) / 64;
+  pl.nt = (chains + 31) / 32 <= device_cus() ? 1 : 2;
+  pl.groups = (chains + 32 * pl.nt - 1) / (32 * pl.nt);
   int rc = prepare_encoding(b, dJ, dJt, n, ptype, pl, st, why);
   if (rc) return rc;
   BParams p{};
@@ -1045,7 +1051,7 @@ int run_blocked_ais(BlockedProblem& b, const void* dJ, const void* dJt, const vo
   p.R = 1;
   p.reads = chains;
   p.S = nt;
-  p.rpw = 64;
+  p.rpw = 32 * pl.nt;
   p.np = pl.np;
   p.use_pt = 0;
   p.logw = 0;
@@ -1076,13 +1082,13 @@ int run_blocked_ais(BlockedProblem& b, const void* dJ, const void* dJt, const vo
   (void)hipEventRecord(ev2.a, st);
   hipError_t le;
   if (pl.i8)
-    le = launch_pipe_ais_i8(p, pl.nwp, pl.groups, st);
+    le = launch_pipe_ais_i8(p, pl.nwp, pl.nt, pl.groups, st);
   else if (pl.np == 1)
-    le = launch_pipe_ais_bf16_1(p, pl.nwp, pl.groups, st);
+    le = launch_pipe_ais_bf16_1(p, pl.nwp, pl.nt, pl.groups, st);
   else if (pl.np == 2)
-    le = launch_pipe_ais_bf16_2(p, pl.nwp, pl.groups, st);
+    le = launch_pipe_ais_bf16_2(p, pl.nwp, pl.nt, pl.groups, st);
   else
-    le = launch_pipe_ais_bf16_3(p, pl.nwp, pl.groups, st);
+    le = launch_pipe_ais_bf16_3(p, pl.nwp, pl.nt, pl.groups, st);
   (void)hipEventRecord(ev2.b, st);
   if (le != hipSuccess) {
     *why = std::string("MFMA AIS launch: ") + hipGetErrorString(le);

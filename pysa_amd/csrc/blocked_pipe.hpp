@@ -9,61 +9,92 @@ namespace blk {
 
 // ------------------------------------------------------- pipelined form --
 // Eight waves per group of 32 NT replicas (NT tiles of 32), two per SIMD.
-// Wave 0 runs the proposals with one lane per replica: the lane holds all 32
-// fields of the block, so a decision needs no cross-lane broadcast.  Three
-// matrix waves (SIMDs 1-3), a third of the K range each and every tile,
-// compute the next block's fields over every K block except c (whose spins
-// are changing) while wave 0 sweeps block c:
+// One proposal wave per tile runs the proposals, two lanes per replica: lane l
+// holds replica l % 32 of the tile and, of the block's 32 visits, those of
+// the 4-visit groups with the parity h = l / 32 -- the layout in which the
+// matrix cores deliver a product (row 8 (v / 4) + 4 h + v % 4 of column l % 32
+// in register v).  Three matrix waves (SIMDs 1-3), a third of the K range
+// each and every tile, compute the next block's fields over every K block
+// except c (whose spins are changing) while the proposal waves sweep block c:
 //     P_{c+1} = sum_{b != c} J[c+1, b] . S_b
-// When wave 0 is done with block c it adds the missing product
-// J[c+1, c] . S_c itself (one K block on SIMD 0's matrix core), so the fields
-// of block c+1 are ready at the block's barrier.  The four helper waves stage
-// the next block's J block, h and row sums and compute its acceptance
-// brackets (those on SIMDs 1-3), so the chain only compares, flips and
-// updates.  Shared state alternates between two buffers by the parity of a
-// running block counter.
+// When a proposal wave is done with block c it adds the missing product
+// J[c+1, c] . S_c itself (one K block), so the fields of block c+1 are ready
+// at the block's barrier.  The rows of every fragment are loaded in the visit
+// order of their block (row k ^ mask at place k: an XOR of the lane's address),
+// so the fields come out in visit order and nothing is permuted afterwards.
+// The helper waves stage the next blocks' J block, h and row sums and compute
+// the acceptance brackets, so the chain only compares, flips and updates.
+// Shared state alternates between two buffers by the parity of a running
+// block counter.
 // K ranges of the pipelined kernel (one matrix wave each).
 constexpr int kPipeMW = 3;
 // What the pipelined kernel runs (its MODE).
 constexpr int kModePT = 0, kModeBatched = 1, kModeAIS = 2;
-constexpr int kPipePF = 3;  // fragment stages in flight per matrix wave (slot ring)
+// Waves 4..7 but the second tile's proposal wave are helpers.  Wave w runs on
+// SIMD w % 4, so both proposal waves share SIMD 0 (with the second one on SIMD
+// 1, beside a matrix wave, N = 1024 took 129 instead of 121 us a sweep).
+constexpr int kPropWave1 = 4;
 
-// A replica's 32 fields take 32 floats; its 16-byte row groups are XOR-
-// swizzled by the replica index so that 8 lanes of a 16-byte access hit all
-// 32 banks.
+// The least float t > x for x < 0 (so x < d, d a float, is t <= d).
+__device__ __forceinline__ float float_above(double x) {
+  const float f = (float)x;
+  return (double)f > x ? f : __uint_as_float(__float_as_uint(f) - 1u);
+}
 __device__ __forceinline__ void swap2(float& a, float& b) {
   const float t = a;
   a = b;
   b = t;
 }
-// Field layout [replica][row]: the 16-byte groups of four rows are XOR
-// swizzled by the replica so that a 16-byte access by consecutive replicas
-// hits distinct banks in every aligned run of 8 lanes (32 banks) and of 16
-// lanes (64 banks: consecutive rows of 128 bytes alternate bank halves).
-__device__ __forceinline__ int fld(int q, int r) {
-  return q * 32 + 4 * ((r >> 2) ^ (q & 7) ^ ((q >> 3) & 1)) + (r & 3);
-}
 constexpr int kHL = 36;
-constexpr int kFG = 2;  // row groups per stage of the proposal wave's field sums
+// Place of visit v in a row of the staged J block: the visits of either lane
+// half together, in the order of its field registers.
+__device__ __forceinline__ int half_slot(int v) {
+  return ((v >> 2) & 1) * 16 + (v >> 3) * 4 + (v & 3);
+}
+// Counts every element of x as used here (no instruction).
+__device__ __forceinline__ void use_whole(const float4& x) {
+  asm volatile("" ::"v"(x.x), "v"(x.y), "v"(x.z), "v"(x.w));
+}
+// The value of lane l % 32 (HI = 0) or 32 + l % 32 (HI = 1) in lane l.
+template <int HI>
+__device__ __forceinline__ uint32_t half_bcast(uint32_t x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+  return HI ? r[1] : r[0];
+}
+template <int HI>
+__device__ __forceinline__ float half_bcast(float x) {
+  return __uint_as_float(half_bcast<HI>(__float_as_uint(x)));
+}
+template <int HI>
+__device__ __forceinline__ double half_bcast(double x) {
+  const uint64_t u = as_u64(x);
+  return as_double(((uint64_t)half_bcast<HI>((uint32_t)(u >> 32)) << 32) |
+                   half_bcast<HI>((uint32_t)u));
+}
 // NI: instances per workgroup (the batched form keeps one J block and h per
 // tile).
-template <int MW, int NI>
+template <int MW, int NI, int NT>
 struct __align__(16) PipeLds {
-  float part[2][MW][64 * 32];  // [parity][matrix wave][fld(replica, row)]
-  float corr[64 * 32];         // J[c+1, c] . S_c of the next block
-  float jb[2][NI][kB * kB];   // row i of J[blk][blk] right of the diagonal, shifted left:
-                              // J^T[pos0+i][pos0+i+1+t] at i*32 + t (t < 31 - i), else 0
-  float hb[2][NI][kB];
+  // [parity][matrix wave][tile][register group v / 4][lane]: partial fields
+  float4 part[2][MW][NT][4][64];
+  // visit i's couplings to the later visits v, else 0: at 32 i + half_slot(v), or
+  // (MFMA updates) those of later 4-visit groups at 32 i + v and those of its
+  // own group in ji at 4 i + v % 4
+  float jb[2][NI][kB * kB];
+  float ji[2][NI][kB * 4];
+  float hb[2][NI][kB];        // in visit order
   float rsb[2][kB];
   // acceptance brackets [parity][replica][visit index], rows padded to
   // kHL floats so that 16-byte reads of consecutive replicas hit distinct banks
-  float lo[2][64][kHL];
-  float hi[2][64][kHL];
+  float lo[2][32 * NT][kHL];
+  float hi[2][32 * NT][kHL];
   uint32_t bb[2][64];         // block spins before the block (bit k = row k ^ the visit mask)
   uint32_t bnew[2][64];       // block spins after the block (by block parity)
-  float sfp[64 * 33];         // exact rerun staging
+  float sfp[32 * NT * 33];    // exact rerun staging
   // visit schedule by pass parity: block at step t | its in-block XOR mask << 8
   uint16_t sch[2][64];
+  double ds[64];  // a replica's energy change over the sweep (dry pass: its energy)
+  uint32_t nacc[64];  // its accepted flips
   float E[64];
   float rb[64];
   float bet[64];  // the ladder by slot (batched: tile t's instance's at 32 t)
@@ -72,7 +103,7 @@ struct __align__(16) PipeLds {
   int bi[64];
   int flag[64];
   int src[64];
-  double lu[64];
+  float lu[64];  // by pair: the least float above the log-uniform of its exchange
 };
 
 // BR: block-random visit order (schedule tables in LDS); otherwise blocks are
@@ -95,11 +126,17 @@ __global__ __launch_bounds__(128 * (MW + 1)) void blocked_pipe_kernel(BParams p0
   // a local copy (the register allocation of the block loops was found to be
   // sensitive to this; the copy keeps it as measured)
   BParams p = p0;
-  static_assert(!BAT || (I8 && NP == 1 && NT == 2),
-                "the batched form multiplies int8 couplings, two tiles per workgroup");
+  static_assert(!BAT || (I8 && NP == 1), "the batched form multiplies int8 couplings");
   constexpr int NI = BAT ? NT : 1;  // instances per workgroup (coupling sets)
-  __shared__ PipeLds<MW, NI> L;
-  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), tid = threadIdx.x;
+  // How the proposal waves update the fields of later visits.  One tile per
+  // workgroup is bound by the latency of its one proposal wave, and the f32
+  // MFMA form shortens it (n = 512, us per sweep of 16 blocks: 43.8 against
+  // 45.5); two tiles are bound by instruction issue, shared by two proposal
+  // waves on SIMD 0, where the VALU form is better (n = 1024, 32 blocks: 119
+  // against 125).
+  constexpr bool MU = NT == 1;
+  __shared__ PipeLds<MW, NI, NT> L;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int read0 = blockIdx.x * p.rpw;
   const int R = p.R, n = p.n;
   const int nblk = BAT ? p.bat[blockIdx.x].nblk : p.nblk;
@@ -115,17 +152,21 @@ __global__ __launch_bounds__(128 * (MW + 1)) void blocked_pipe_kernel(BParams p0
   auto tile = [&](int tt) -> const BatTile& { return bt[tt]; };
   auto n_of = [&](int tt) { return BAT ? tile(tt).n : n; };
   const int h = lane >> 5;
-  // Two waves per SIMD (SIMD w & 3).  Wave 0 runs the proposals; matrix
-  // wave w = 1..MW computes the products of K range m = w - 1 for both tiles
-  // of 32 replicas (each coupling fragment is loaded once for both); the
-  // helper waves MW+1.. stage the next blocks' J block, h and row sums,
-  // compute the acceptance brackets (those on SIMDs 1..MW) and, wave MW+1,
-  // the visit schedule.
-  static_assert(MW == 3, "eight waves: the proposal wave, three matrix waves, four helpers");
-  const bool mw = w >= 1 && w <= MW;  // a matrix wave
-  const bool hw = w > MW;             // a helper wave
+  // Two waves per SIMD (SIMD w & 3).  Waves 0 and (two tiles) kPropWave1 run
+  // the proposals of a tile each; matrix wave w = 1..MW computes the products
+  // of K range m = w - 1 for both tiles of 32 replicas (each coupling fragment
+  // is loaded once for both); the helper waves stage the next blocks' J block,
+  // h and row sums and compute the acceptance brackets, wave 4 the visit
+  // schedule, wave 7 the exchange uniforms.  Wave 0 also ends the sweeps.
+  static_assert(MW == 3, "eight waves: up to two proposal waves, three matrix waves, helpers");
+  const bool mw = w >= 1 && w <= MW;                          // a matrix wave
+  const bool pw = w == 0 || (NT == 2 && w == kPropWave1);     // a proposal wave
+  const bool hw = !mw && !pw;                                 // a helper wave
   const int m = mw ? w - 1 : 0;
-  const int hl = hw ? (w - MW - 1) * 64 + lane : -1;  // helper-lane index 0..64 (MW+1) - 1
+  constexpr int NH = NT == 2 ? 3 : 4;  // helpers
+  // helper index
+  const int hx = !hw ? 0 : w - (8 - NH);
+  const int hl = hw ? hx * 64 + lane : -1;  // helper-lane index 0..64 NH - 1
   // Operand role (matrix waves): replica qtt[tt] of tile tt.
   static_assert(NT == 1 || NT == 2, "one or two tiles of 32 replicas");
   // gtt: its read within the workgroup (recomputed where needed: kept in
@@ -164,17 +205,25 @@ __global__ __launch_bounds__(128 * (MW + 1)) void blocked_pipe_kernel(BParams p0
   // within the workgroup, tq its tile in the batched form (whose instance's
   // size, scale and ladder the lane uses).
   const int q = lane;
-  const int tq = BAT ? (q >> 5) : 0;
+  const int tq = BAT && NT == 2 ? (q >> 5) : 0;
   const int gl = BAT ? (q & 31) / R : 0;  // batched: its read within the tile
   const int g = BAT ? tq * p.rpw + gl : q / R;
   const int rr = BAT ? (q & 31) - gl * R : q - g * R;
-  const int read = BAT ? (tq ? tile(1).read0 : tile(0).read0) + gl : read0 + g;
-  const bool act = BAT ? gl < p.rpw && read < (tq ? tile(1).read_end : tile(0).read_end)
+  const int read = BAT ? (tq ? tile(NI - 1).read0 : tile(0).read0) + gl : read0 + g;
+  const bool act = BAT ? (NT == 2 || q < 32) && gl < p.rpw &&
+                             read < (tq ? tile(NI - 1).read_end : tile(0).read_end)
                        : (g < p.rpw) && (read < p.reads);
-  const int nq = BAT ? (tq ? tile(1).n : tile(0).n) : n;
+  const int nq = BAT ? (tq ? tile(NI - 1).n : tile(0).n) : n;
   const float* betas_q =
-      BAT ? p.betas + (size_t)(tq ? tile(1).inst : tile(0).inst) * R : p.betas;
+      BAT ? p.betas + (size_t)(tq ? tile(NI - 1).inst : tile(0).inst) * R : p.betas;
   const uint64_t cid = (uint64_t)read * R + rr;
+  // the same of replica qx of a workgroup with one tile
+  auto chain_of = [&](int qx) -> uint64_t {
+    return (uint64_t)(BAT ? tile(0).read0 : read0) * R + qx;
+  };
+  auto act_of = [&](int qx) {
+    return qx < p.rpw * R && (BAT ? tile(0).read0 : read0) + qx / R < (BAT ? tile(0).read_end : p.reads);
+  };
   const int c0 = mw ? m * kb : 0;
   const int jn = mw ? max(0, min(kb, nblk - c0)) : 0;
 
@@ -221,20 +270,16 @@ __global__ __launch_bounds__(128 * (MW + 1)) void blocked_pipe_kernel(BParams p0
       p.best_rep_sw[(size_t)read * R + rr] = 0;
     }
   }
-  // Fields of replicas no tile covers (NT = 1: lanes 32-63 of the proposal
-  // wave) stay zero, so their idle decisions see finite values.
-  for (int i = tid; i < 64 * 32; i += 128 * (MW + 1)) L.corr[i] = 0.f;
-  for (int i = tid; i < 2 * MW * 64 * 32; i += 128 * (MW + 1)) (&L.part[0][0][0])[i] = 0.f;
-
-  constexpr int PF = kPipePF;
+  // fragment stages in flight per matrix wave (slot ring), within the registers
+  constexpr int PF = I8 || NP == 1 ? 6 : NT == 1 ? (NP == 2 ? 6 : 4) : 3;
   const uint32_t emul = p.ptype == 0 ? 0xFEu : 1u;
   const uint32_t exr = p.ptype == 0 ? 0xFFFFFFFFu : 0u;
   // operand-expansion constants in vector registers (see spins_bf16_r)
   uint32_t vmask = 0x80008000u, vone = 0x3F803F80u;
   asm volatile("" : "+v"(vmask), "+v"(vone));
   constexpr int NST = I8 ? 1 : 2;
-  constexpr int NHL = 64 * (MW + 1);  // helper lanes
-  constexpr int NJB = (kB * kB + NHL - 1) / NHL;
+  constexpr int NHL = 64 * NH;  // helper lanes, NHL / 32 rows of the J block at a time
+  constexpr int NJB = (kB * 32 + NHL - 1) / NHL;
   typedef typename std::conditional<I8, i32x4, bf16x8>::type Frag;
   Frag ring[NI][PF][NST][NP];  // by instance (tile in the batched form)
   float jb_reg[NI][NJB], h_reg[NI] = {}, rs_reg = 0.f;
@@ -246,8 +291,8 @@ __global__ __launch_bounds__(128 * (MW + 1)) void blocked_pipe_kernel(BParams p0
     return reinterpret_cast<const Frag*>(p.frag);
   };
   auto frag_ptr = [&](int ti, int c, int j, int st, int pc) -> const Frag* {
-    if (I8) return frag_base(ti) + ((size_t)c * nblk + c0 + j) * 64 + lane;
-    return frag_base(ti) + (((size_t)c * (2 * nblk) + 2 * (c0 + j) + st) * NP + pc) * 64 + lane;
+    if (I8) return frag_base(ti) + ((size_t)c * nblk + c0 + j) * 64;
+    return frag_base(ti) + (((size_t)c * (2 * nblk) + 2 * (c0 + j) + st) * NP + pc) * 64;
   };
   // Stage j of this wave's K range; stages past the range reload the
   // range's last K block (recently read, so a cache hit), so every path
@@ -255,7 +300,8 @@ __global__ __launch_bounds__(128 * (MW + 1)) void blocked_pipe_kernel(BParams p0
   // would make the compiler wait for all of them).
   // One K block of fragments: NST * NP * 64 of them, consecutive.
   constexpr int kStage = NST * NP * 64;
-  auto load_stage = [&](int c, int j, Frag (&dst)[NST][NP], int ti) {
+  // lx: the lane, its row (low five bits) XORed by the row block's visit mask.
+  auto load_stage = [&](int c, int lx, int j, Frag (&dst)[NST][NP], int ti) {
     // jn passes through an empty asm so that the per-stage offsets are
     // recomputed (a few scalar ops) rather than hoisted out of the block
     // loop into registers that would spill
@@ -263,63 +309,55 @@ __global__ __launch_bounds__(128 * (MW + 1)) void blocked_pipe_kernel(BParams p0
     asm volatile("" : "+s"(jnl));
     const int jc = jnl > 0 ? min(j, jnl - 1) : nblk - 1 - c0;
     // wave-uniform base of the stage, then a per-lane 16-byte offset
-    const Frag* base = frag_ptr(ti, c, 0, 0, 0) - lane + (size_t)jc * kStage;
+    const Frag* base = frag_ptr(ti, c, 0, 0, 0) + (size_t)jc * kStage;
 #pragma unroll
     for (int st = 0; st < NST; ++st)
 #pragma unroll
-      for (int pc = 0; pc < NP; ++pc) dst[st][pc] = base[(st * NP + pc) * 64 + lane];
+      for (int pc = 0; pc < NP; ++pc) dst[st][pc] = base[(st * NP + pc) * 64 + lx];
   };
-  // Request row block c: the first PF fragment stages of this wave's K range
-  // (matrix waves).
-  auto prefetch_frags = [&](int c) {
+  // Request row block c (visit mask xm): the first PF fragment stages of this
+  // wave's K range (matrix waves).
+  auto prefetch_frags = [&](int c, uint32_t xm) {
+    const int lx = lane ^ (int)xm;
 #pragma unroll
     for (int u = 0; u < PF; ++u)
 #pragma unroll
-      for (int ti = 0; ti < NI; ++ti) load_stage(c, u, ring[ti][u], ti);
+      for (int ti = 0; ti < NI; ++ti) load_stage(c, lx, u, ring[ti][u], ti);
   };
   // Request row block c, visited with in-block mask xm, spread over the
-  // helper lanes: J[blk][blk] in visit order, h and row sums.
+  // helper lanes: J[blk][blk] in visit order, h and row sums.  Lane hl takes
+  // visit column v = hl % 32 of the visit rows hl / 32 + e2 NHL / 32.
+  const int jv = hl & 31, ji0 = hl >> 5;
   auto prefetch_jb = [&](int c, uint32_t xm) {
     const int pos0 = 32 * c;
     // Every lane loads (an in-bounds address when its element is padding)
     // and publish_block zeroes the padding: no register is written here
     // except by these loads, which keeps them from waiting on older loads.
-    if constexpr (!BAT) {
-      jb_ok[0] = 0;
+#pragma unroll
+    for (int ti = 0; ti < NI; ++ti) {
+      const int ni = n_of(ti);
+      const int col = pos0 + (jv ^ (int)xm);
+      const bool cok = hl >= 0 && col < ni;
+      jb_ok[ti] = 0;
 #pragma unroll
       for (int e2 = 0; e2 < NJB; ++e2) {
-        const int e = hl + e2 * NHL;
-        // slot t = e & 31 of visit row i holds visit column k = i + 1 + t;
-        // visit index v is block row v ^ xm
-        const int i = e >> 5, k = i + 1 + (e & 31);
-        const int ri = i ^ (int)xm, rk = k ^ (int)xm;
-        const bool ok = e >= 0 && e < kB * kB && k < kB && pos0 + ri < n && pos0 + rk < n;
-        jb_ok[0] |= (uint32_t)ok << e2;
-        jb_reg[0][e2] = p.Jt[ok ? (size_t)(pos0 + ri) * n + pos0 + rk : 0];
+        const int i = ji0 + e2 * (NHL / 32);  // visit row
+        const int row = pos0 + (i ^ (int)xm);
+        const bool ok = cok && i < jv && row < ni;  // i < jv <= 31: later visits only
+        jb_ok[ti] |= (uint32_t)ok << e2;
+        if constexpr (BAT)  // S symmetric: S^T = S
+          jb_reg[ti][e2] = (float)(p.sgn + tile(ti).sgn)[ok ? (size_t)row * tile(ti).ld + col : 0];
+        else
+          jb_reg[ti][e2] = p.Jt[ok ? (size_t)row * ni + col : 0];
       }
-      const bool hok = hl >= 0 && hl < kB && pos0 + hl < n;
-      jb_ok[0] |= (uint32_t)hok << 31;
-      h_reg[0] = p.h[hok ? pos0 + hl : 0];
-      if (!I8 && p.rowsum) rs_reg = p.rowsum[hok ? pos0 + hl : 0];
-    } else {  // each tile's instance (S symmetric: S^T = S; no row sums with int8)
-#pragma unroll
-      for (int ti = 0; ti < NI; ++ti) {
-        const int ni = tile(ti).n;
-        const int8_t* sg = p.sgn + tile(ti).sgn;
-        jb_ok[ti] = 0;
-#pragma unroll
-        for (int e2 = 0; e2 < NJB; ++e2) {
-          const int e = hl + e2 * NHL;
-          const int i = e >> 5, k = i + 1 + (e & 31);
-          const int ri = i ^ (int)xm, rk = k ^ (int)xm;
-          const bool ok = e >= 0 && e < kB * kB && k < kB && pos0 + ri < ni && pos0 + rk < ni;
-          jb_ok[ti] |= (uint32_t)ok << e2;
-          jb_reg[ti][e2] = (float)sg[ok ? (size_t)(pos0 + ri) * tile(ti).ld + pos0 + rk : 0];
-        }
-        const bool hok = hl >= 0 && hl < kB && pos0 + hl < ni;
-        jb_ok[ti] |= (uint32_t)hok << 31;
+      const bool hok = cok && hl < kB;
+      jb_ok[ti] |= (uint32_t)hok << 31;
+      if constexpr (BAT) {  // no row sums with int8
         const int64_t ho = tile(ti).h;
-        h_reg[ti] = ho >= 0 ? p.h[ho + (hok ? pos0 + hl : 0)] : 0.f;
+        h_reg[ti] = ho >= 0 ? p.h[ho + (hok ? col : 0)] : 0.f;
+      } else {
+        h_reg[ti] = p.h[hok ? col : 0];
+        if (!I8 && p.rowsum) rs_reg = p.rowsum[hok ? col : 0];
       }
     }
   };
@@ -328,8 +366,17 @@ __global__ __launch_bounds__(128 * (MW + 1)) void blocked_pipe_kernel(BParams p0
     for (int ti = 0; ti < NI; ++ti)
 #pragma unroll
       for (int e2 = 0; e2 < NJB; ++e2) {
-        const int e = hl + e2 * NHL;
-        if (hl >= 0 && e < kB * kB) L.jb[pb][ti][e] = ((jb_ok[ti] >> e2) & 1u) ? jb_reg[ti][e2] : 0.f;
+        const int i = ji0 + e2 * (NHL / 32);
+        if (hl >= 0 && i < kB) {
+          const float x = ((jb_ok[ti] >> e2) & 1u) ? jb_reg[ti][e2] : 0.f;
+          if constexpr (MU) {
+            const bool own = (i >> 2) == (jv >> 2);
+            L.jb[pb][ti][hl + e2 * NHL] = own ? 0.f : x;
+            if (own) L.ji[pb][ti][4 * i + (jv & 3)] = x;
+          } else {
+            L.jb[pb][ti][32 * i + half_slot(jv)] = x;
+          }
+        }
       }
     if (hl >= 0 && hl < kB) {
 #pragma unroll
@@ -365,26 +412,12 @@ __global__ __launch_bounds__(128 * (MW + 1)) void blocked_pipe_kernel(BParams p0
       }
     }
   };
-  // Fields from the C layout (register v: row 8(v/4) + 4h + v%4 of column
-  // lane%32) into [replica][row], four consecutive rows per 16-byte store.
-  auto write_fields_col = [&](float* dst, const f32x16& acc, const i32x16& iacc, int qcol) {
-#pragma unroll
-    for (int g4 = 0; g4 < 4; ++g4) {
-      const int i = 8 * g4 + 4 * h;
-      float4 x;
-      if (I8)
-        x = make_float4((float)iacc[4 * g4], (float)iacc[4 * g4 + 1], (float)iacc[4 * g4 + 2],
-                        (float)iacc[4 * g4 + 3]);
-      else
-        x = make_float4(acc[4 * g4], acc[4 * g4 + 1], acc[4 * g4 + 2], acc[4 * g4 + 3]);
-      *reinterpret_cast<float4*>(&dst[fld(qcol, i)]) = x;
-    }
-  };
-
   // Partial fields of row block cr over this wave's K range, skipping K block
   // ex (its product is added by the proposal wave once the block's spins are
-  // final); ring holds the first PF stages of row block cr on entry.
-  auto compute_part = [&](int cr, int ex, float* dst) {
+  // final), into the buffers of parity pb; ring holds the first PF stages of
+  // row block cr (visit mask xm) on entry.
+  auto compute_part = [&](int cr, uint32_t xm, int ex, int pb) {
+    const int lx = lane ^ (int)xm;
     f32x16 acc[NT] = {};
     i32x16 iacc[NT] = {};
     const int jx = ex - c0;  // the skipped stage, if it is in this wave's range
@@ -409,28 +442,67 @@ __global__ __launch_bounds__(128 * (MW + 1)) void blocked_pipe_kernel(BParams p0
             mfma_step(ring[BAT ? tt : 0][u], get_half<NW>(sa[tt], j), acc[tt], iacc[tt]);
         }
 #pragma unroll
-        for (int ti = 0; ti < NI; ++ti) load_stage(cr, j + PF, ring[ti][u], ti);
+        for (int ti = 0; ti < NI; ++ti) load_stage(cr, lx, j + PF, ring[ti][u], ti);
       }
     }
 #pragma unroll
-    for (int tt = 0; tt < NT; ++tt) write_fields_col(dst, acc[tt], iacc[tt], qtt[tt]);
+    for (int tt = 0; tt < NT; ++tt)
+#pragma unroll
+      for (int g4 = 0; g4 < 4; ++g4) {
+        float4 x;
+        if (I8)
+          x = make_float4((float)iacc[tt][4 * g4], (float)iacc[tt][4 * g4 + 1],
+                          (float)iacc[tt][4 * g4 + 2], (float)iacc[tt][4 * g4 + 3]);
+        else
+          x = make_float4(acc[tt][4 * g4], acc[tt][4 * g4 + 1], acc[tt][4 * g4 + 2],
+                          acc[tt][4 * g4 + 3]);
+        L.part[pb][m][tt][g4][lane] = x;
+      }
   };
   // Acceptance brackets of row block cr (in-block mask xm) for sweep counter
-  // sw, stored by visit index, lane = replica (beta from L.rb): groups of 4
-  // rows (one Philox block each) dealt over the helpers on SIMDs 1..MW, so
-  // that none lands on the SIMD of the proposal chain.
-  auto brackets = [&](int cr, uint32_t xm, uint64_t sw, int pb) {
-    float cb, cz;
-    bracket_factors(L.rb[q], cb, cz);
+  // sw, stored by visit index: groups of 4 rows (one Philox block each) dealt
+  // over the helpers, beta from L.rb.  Two tiles: lane = replica; one tile:
+  // lanes l and l + 32 hold replica l and take groups 2 hx and 2 hx + 1.
+  const int qb = NT == 2 ? q : (lane & 31);
+  const uint64_t cidb = NT == 2 ? cid : chain_of(qb);
+  const bool actb = NT == 2 ? act : act_of(qb);
+  const SweepStream stream(cidb, p.k0, p.k1);
+  const bool idle_any = __ballot(!actb) != 0;
+  float cb = 0.f, cz = 0.f;  // of the pass (sweep_factors)
+  auto sweep_factors = [&]() { bracket_factors(L.rb[qb], cb, cz); };
+  // a lane's groups side by side (their Philox rounds are one dependent chain
+  // each); with two tiles the third helper's last one repeats its first
+  constexpr int NG = NT == 2 ? 3 : 1;
+  static_assert(NT == 2 ? NH == 3 : NH == 4, "8 groups over the helpers");
+  auto group_of = [&](int i) {
+    const int g4 = NT == 2 ? hx + 3 * i : 2 * hx + h;
+    return g4 < kB / 4 ? g4 : hx;
+  };
+  // the logarithms (base 2) of row block cr's uniforms, which need no beta
+  auto draw = [&](int cr, uint64_t sw, float (&lg)[NG][4]) {
+    const auto sws = stream.sweep(sw);
+    u32x4 blk[NG];
+#pragma unroll
+    for (int i = 0; i < NG; ++i) blk[i] = stream.block(sws, (uint32_t)(8 * cr + group_of(i)));
+#pragma unroll
+    for (int i = 0; i < NG; ++i) {
+      lg[i][0] = accept_log2(blk[i].x), lg[i][1] = accept_log2(blk[i].y);
+      lg[i][2] = accept_log2(blk[i].z), lg[i][3] = accept_log2(blk[i].w);
+    }
+  };
+  auto finish = [&](int cr, uint32_t xm, const float (&lg)[NG][4], int pb) {
     const int pos0 = 32 * cr;
-    for (int g4 = w - MW - 2; g4 < kB / 4; g4 += MW) {
-      const u32x4 blk = sweep_block(cid, sw, (uint32_t)(pos0 + 4 * g4), p.k0, p.k1);
-      const uint32_t wd[4] = {blk.x, blk.y, blk.z, blk.w};
+    const bool partial = pos0 + kB > (BAT ? min(tile(0).n, tile(NI - 1).n) : n);
+#pragma unroll
+    for (int i = 0; i < NG; ++i) {
+      const int g4 = group_of(i);
       float lo[4], hi[4];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        accept_bounds_f(wd[e], cb, cz, lo[e], hi[e]);
-        if (pos0 + 4 * g4 + e >= nq || !act) lo[e] = hi[e] = INFINITY;  // padding, idle lanes
+      for (int e = 0; e < 4; ++e) accept_bounds_l(lg[i][e], cb, cz, lo[e], hi[e]);
+      if (partial || idle_any) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (pos0 + 4 * g4 + e >= nq || !actb) lo[e] = hi[e] = INFINITY;  // padding, idle lanes
       }
       // rows 4 g4 + e are visits 4 (g4 ^ xm / 4) + (e ^ xm % 4): one 16-byte
       // store each, its entries exchanged by the uniform low bits of xm
@@ -443,9 +515,15 @@ __global__ __launch_bounds__(128 * (MW + 1)) void blocked_pipe_kernel(BParams p0
         swap2(hi[0], hi[2]), swap2(hi[1], hi[3]);
       }
       const int v4 = 4 * (g4 ^ (int)(xm >> 2));
-      *reinterpret_cast<float4*>(&L.lo[pb][q][v4]) = make_float4(lo[0], lo[1], lo[2], lo[3]);
-      *reinterpret_cast<float4*>(&L.hi[pb][q][v4]) = make_float4(hi[0], hi[1], hi[2], hi[3]);
+      *reinterpret_cast<float4*>(&L.lo[pb][qb][v4]) = make_float4(lo[0], lo[1], lo[2], lo[3]);
+      *reinterpret_cast<float4*>(&L.hi[pb][qb][v4]) = make_float4(hi[0], hi[1], hi[2], hi[3]);
     }
+  };
+  float lgn[NG][4];  // drawn for the next pass's first block during this pass's last
+  auto brackets = [&](int cr, uint32_t xm, uint64_t sw, int pb) {
+    float lg[NG][4];
+    draw(cr, sw, lg);
+    finish(cr, xm, lg, pb);
   };
   auto owner_of = [&](int c) { return 1 + c / kb; };  // matrix wave owning K block c
   // by the owner of block c, in the visit order of its next visit (mask xm),
@@ -525,9 +603,9 @@ __global__ __launch_bounds__(128 * (MW + 1)) void blocked_pipe_kernel(BParams p0
   {
     int s0;
     const bool dry0 = pass_info(0, s0);
-    if (BR && w == 4) fill_sched(0, (uint64_t)s0 + p.sweep_offset, dry0);
+    if (BR && w == 7) fill_sched(0, (uint64_t)s0 + p.sweep_offset, dry0);
   }
-  __syncthreads();  // wave 0's betas (L.rb), the zeroed L.corr and the schedule are visible
+  __syncthreads();  // wave 0's betas (L.rb) and the schedule are visible
   {
     int s0;
     (void)pass_info(0, s0);
@@ -536,16 +614,17 @@ __global__ __launch_bounds__(128 * (MW + 1)) void blocked_pipe_kernel(BParams p0
     const int cf = entry_block(ef), cs = entry_block(es);
     const uint32_t mf = entry_mask(ef), ms = entry_mask(es);
     if (mw) {
-      prefetch_frags(cf);
-      compute_part(cf, -1, L.part[0][m]);
-      prefetch_frags(cs);
+      prefetch_frags(cf, mf);
+      compute_part(cf, mf, -1, 0);
+      prefetch_frags(cs, ms);
       if (w == owner_of(cf)) publish_bits(cf, 0, mf);
     }
     if (hw) {
       prefetch_jb(cf, mf);
       publish_block(0);
       prefetch_jb(cs, ms);
-      if (w > MW + 1) brackets(cf, mf, sw0, 0);
+      sweep_factors();
+      brackets(cf, mf, sw0, 0);
     }
   }
   __syncthreads();
@@ -556,67 +635,52 @@ __global__ __launch_bounds__(128 * (MW + 1)) void blocked_pipe_kernel(BParams p0
   // rsb (zero otherwise); fsc is a power of two, so the fma rounds like the add
   const bool qsum = !I8 && p.ptype == 1;
   const float fsc = qsum ? 0.5f : 1.f;
-  // batched: field = bsc * count + h, the scale of the lane's instance
-  const float bsc = BAT ? (tq ? tile(1).scale : tile(0).scale) : 1.f;
+  // batched: field = bsc * count + h, the scale of the proposal wave's instance
+  const float bsc = BAT ? (w == 0 ? tile(0).scale : tile(NI - 1).scale) : 1.f;
   double eoff = 0.0;  // wave 0: caller's initial energy minus its recomputation
 
-  // The correction J[c1, c] . S_c of the next block c1 by the proposal wave,
-  // once block c's spins are final (on SIMD 0's matrix core, idle otherwise):
-  // bits = block c's spins of replica `lane` in block-row order; the A
-  // fragments of row block c1, K block c were loaded into fa at the block's
-  // start.  Result to L.corr (read by this wave at the next block's start).
-  typedef Frag FragSet[NI][NST][NP];  // by instance
-  auto load_corr_frags = [&](int c1, int c, FragSet& fa) {
+  // The correction J[c1, c] . S_c of the next block c1 by a proposal wave,
+  // once block c's spins are final: the A fragments of row block c1, K block
+  // c (rows in the visit order of c1, lx as in load_stage) were loaded into fa
+  // at the block's start, and the product stays in its registers.
+  typedef Frag FragSet[NST][NP];
+  auto load_corr_frags = [&](int c1, int c, int lx, int ti, FragSet& fa) {
+    const Frag* fb = frag_base(ti);
 #pragma unroll
-    for (int ti = 0; ti < NI; ++ti) {
-      const Frag* fb = frag_base(ti);
+    for (int st = 0; st < NST; ++st)
 #pragma unroll
-      for (int st = 0; st < NST; ++st)
-#pragma unroll
-        for (int pc = 0; pc < NP; ++pc) {
-          const size_t f = I8 ? (size_t)c1 * nblk + c
-                              : ((size_t)c1 * (2 * nblk) + 2 * c + st) * NP + pc;
-          fa[ti][st][pc] = fb[f * 64 + lane];
-        }
-    }
-  };
-  auto corr_products = [&](const FragSet& fa, uint32_t bits, int ql) {  // ql: lane
-#pragma unroll
-    for (int tl = 0; tl < NT; ++tl) {
-      // column lane % 32 of tile tl is replica 32 tl + lane % 32
-      const uint32_t bt = (uint32_t)__shfl((int)bits, 32 * tl + (ql & 31), 64);
-      f32x16 a = {};
-      i32x16 ia = {};
-      mfma_step(fa[BAT ? tl : 0], half_of<I8>(bt, h), a, ia);
-      write_fields_col(L.corr, a, ia, 32 * tl + (ql & 31));
-    }
+      for (int pc = 0; pc < NP; ++pc) {
+        const size_t f = I8 ? (size_t)c1 * nblk + c
+                            : ((size_t)c1 * (2 * nblk) + 2 * c + st) * NP + pc;
+        fa[st][pc] = fb[f * 64 + lx];
+      }
   };
 
   uint32_t t = 0;                               // running block counter
-  // The two roles run separate copies of the block loop (so that each keeps
-  // only its own state in registers); both pass the same barriers: one after
-  // the block's work (B), and at the end of a pass one more (three after a
-  // sweep).
-  if (w == 0) {
+  // The roles run separate copies of the block loop (so that each keeps only
+  // its own state in registers); all pass the same barriers: one after the
+  // block's work (B), and at the end of a pass one more (three after a sweep).
+  if (pw) {
     // schedule entries of the current step, each read one block ahead
     const uint32_t e0 = sched_entry(0, 0);
     int c_nx = entry_block(e0);
     uint32_t xm_nx = entry_mask(e0);
+    const int tw = w == 0 ? 0 : NT - 1;    // the wave's tile
+    const int ti = BAT ? tw : 0;           // its instance
+    const int qp = 32 * tw + (lane & 31);  // the lane's replica of the group
+    const int np = n_of(ti);
+    float corr[16];  // J[c, c_prev] . S of the block before
+#pragma unroll
+    for (int v = 0; v < 16; ++v) corr[v] = 0.f;
     for (int ps = 0; ps < npass; ++ps) {
       int s;
       const bool dry = pass_info(ps, s);
       const uint64_t sw = (uint64_t)s + p.sweep_offset;
       const int sp = ps & 1;
-      const float beta = act ? L.rb[q] : 0.f;
       double dsum = 0.0, eacc = 0.0;
       uint32_t nacc = 0;
       for (int tb = 0; tb < nblk; ++tb, ++t) {
         const int pb = t & 1;
-        // The lane's LDS offsets are recomputed each block from an opaque
-        // copy of its index (a few VALU ops): hoisted out of the loop they
-        // would stay live across the chain, where registers are scarce.
-        int qo = q;
-        asm volatile("" : "+v"(qo));
         // block c of this step, its visit k being block row k ^ xm; c1 the next
         const int c = c_nx;
         const uint32_t xm = xm_nx;
@@ -627,265 +691,356 @@ __global__ __launch_bounds__(128 * (MW + 1)) void blocked_pipe_kernel(BParams p0
         xm_nx = entry_mask(e1);
         c_nx = c1;
         FragSet fcorr;
-        load_corr_frags(c1, c, fcorr);
+        load_corr_frags(c1, c, lane ^ (int)xm_nx, ti, fcorr);
+        // the spins of the block's visits, in either half of the wave
+        uint32_t mb = L.bb[pb][qp];
         if (dry) {
           // ---- dry pass: f64 energy of the block's rows from its full fields
-          // (a dry pass visits every block with mask 0: bits in row order)
-          const uint32_t bits = L.bb[pb][qo];
-          for (int i = 0; i < kB; ++i) {
-            if (pos0 + i < nq) {
-              const int o = fld(qo, i);
-              double f = (double)L.part[pb][0][o];
-              for (int mm = 1; mm < MW; ++mm) f += (double)L.part[pb][mm][o];
-              f += (double)L.corr[o];
-              if (qsum) f = 0.5 * (f + (double)L.rsb[pb][i]);
-              if (BAT) f *= (double)bsc;
-              const double si = ((bits >> i) & 1u) ? 1.0 : (p.ptype == 0 ? -1.0 : 0.0);
-              eacc += si * (0.5 * f + (double)L.hb[pb][tq][i]);
+          // (a dry pass visits every block with mask 0: visits are rows), the
+          // rows' terms added in order, passed between the lane halves
+          static_for<kB / 4>([&](auto gc) __attribute__((always_inline)) {
+            constexpr int gr = decltype(gc)::value, g4 = gr >> 1;
+            float4 x[MW];
+#pragma unroll
+            for (int mm = 0; mm < MW; ++mm) x[mm] = L.part[pb][mm][tw][g4][lane];
+            for (int e = 0; e < 4; ++e) {
+              const int i = 4 * gr + e;
+              if (pos0 + i < np) {
+                auto el = [&](const float4& y) { return e == 0 ? y.x : e == 1 ? y.y : e == 2 ? y.z : y.w; };
+                double f = (double)el(x[0]);
+#pragma unroll
+                for (int mm = 1; mm < MW; ++mm) f += (double)el(x[mm]);
+                f += (double)(e == 0   ? corr[4 * g4]
+                              : e == 1 ? corr[4 * g4 + 1]
+                              : e == 2 ? corr[4 * g4 + 2]
+                                       : corr[4 * g4 + 3]);
+                if (qsum) f = 0.5 * (f + (double)L.rsb[pb][i]);
+                if (BAT) f *= (double)bsc;
+                const double si = ((mb >> i) & 1u) ? 1.0 : (p.ptype == 0 ? -1.0 : 0.0);
+                eacc += si * (0.5 * f + (double)L.hb[pb][ti][i]);
+              }
+            }
+            eacc = half_bcast<gr & 1>(eacc);
+          });
+        } else {
+          // ---- proposals of block c: slot j = 4 m + e of a lane is visit
+          // 8 m + 4 h + e
+          // brackets of the lane's visits, read first (their latency overlaps
+          // the field sums and they leave the chain free of LDS waits)
+          float hib[16], lob[16];
+#pragma unroll
+          for (int g4 = 0; g4 < 4; ++g4) {
+            const float4 a = *reinterpret_cast<const float4*>(&L.hi[pb][qp][8 * g4 + 4 * h]);
+            const float4 b = *reinterpret_cast<const float4*>(&L.lo[pb][qp][8 * g4 + 4 * h]);
+            hib[4 * g4] = a.x, hib[4 * g4 + 1] = a.y, hib[4 * g4 + 2] = a.z, hib[4 * g4 + 3] = a.w;
+            lob[4 * g4] = b.x, lob[4 * g4 + 1] = b.y, lob[4 * g4 + 2] = b.z, lob[4 * g4 + 3] = b.w;
+          }
+          // fields: the partials in order, the correction, (QUBO with bf16
+          // operands) the row sums, then h (batched: the integer counts, with
+          // h in hk)
+          f32x16 fp;
+          float hk[16];
+          {
+            float4 x[4][MW];
+#pragma unroll
+            for (int g4 = 0; g4 < 4; ++g4)
+#pragma unroll
+              for (int mm = 0; mm < MW; ++mm) x[g4][mm] = L.part[pb][mm][tw][g4][lane];
+#pragma unroll
+            for (int g4 = 0; g4 < 4; ++g4) {
+              float4 sm = x[g4][0];
+#pragma unroll
+              for (int mm = 1; mm < MW; ++mm) {
+                sm.x = sm.x + x[g4][mm].x;
+                sm.y = sm.y + x[g4][mm].y;
+                sm.z = sm.z + x[g4][mm].z;
+                sm.w = sm.w + x[g4][mm].w;
+              }
+              fp[4 * g4] = sm.x + corr[4 * g4];
+              fp[4 * g4 + 1] = sm.y + corr[4 * g4 + 1];
+              fp[4 * g4 + 2] = sm.z + corr[4 * g4 + 2];
+              fp[4 * g4 + 3] = sm.w + corr[4 * g4 + 3];
+            }
+            if (qsum) {
+#pragma unroll
+              for (int g4 = 0; g4 < 4; ++g4) {
+                const float4 r = *reinterpret_cast<const float4*>(&L.rsb[pb][8 * g4 + 4 * h]);
+                fp[4 * g4] += r.x, fp[4 * g4 + 1] += r.y, fp[4 * g4 + 2] += r.z, fp[4 * g4 + 3] += r.w;
+              }
+            }
+            // every h zero: adding +0 would only turn a -0 into +0, which no
+            // decision or sum distinguishes
+            if (BAT || qsum || !p.hzero) {
+#pragma unroll
+              for (int g4 = 0; g4 < 4; ++g4) {
+                const float4 r = *reinterpret_cast<const float4*>(&L.hb[pb][ti][8 * g4 + 4 * h]);
+                const float hv[4] = {r.x, r.y, r.z, r.w};
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                  if constexpr (BAT)
+                    hk[4 * g4 + e] = hv[e];
+                  else
+                    fp[4 * g4 + e] = __builtin_fmaf(fsc, fp[4 * g4 + e], hv[e]);
+                }
+              }
             }
           }
-          L.bnew[pb][qo] = bits;
-          // the same block next (the owners skip it), in its next visit order
-          if (c1 == c) L.bb[pb ^ 1][qo] = BR ? xor_permute_bits(bits, xm_nx) : bits;
-          corr_products(fcorr, bits, qo);
+          const uint32_t mb0 = mb;
+          // accepted flips and decisions not below their bracket, step k at bit
+          // 31 - k: one add with carry each per step (tn: only the bits of the
+          // lane's own visits mean anything)
+          uint32_t tk = 0, tn = 0;
+          // bit k of mb is only changed at step k, so every step reads its
+          // spin from the block's initial bits: sign bit = !spin, magnitude cu
+          const uint32_t nmb = ~mb0, cub = __float_as_uint(cu);
+          uint32_t vsgn = 0x80000000u;  // kept in a register (not a literal operand)
+          asm volatile("" : "+v"(vsgn));
+          float dpart = 0.f;
+          const double dsum0 = dsum;  // batched: the sum before the block (for a rerun)
+          // The field updates of the later visits, one of two ways (MU):
+          // * VALU: every decision updates the lane's later slots, rows of
+          //   J[blk][blk] streaming from LDS through a ring JR rows ahead, from
+          //   the first slot group a lane of either half needs.
+          // * MFMA: within a 4-visit group each decision updates the fields
+          //   behind it on the VALU (ff); the later groups take two visits at a
+          //   time as one f32 MFMA: row v of A = J[visits][v], B = the two spin
+          //   changes per replica, C = the fields, which lie in this layout
+          //   already.  The instruction adds its two products one after the
+          //   other, each as an fma (checked on the device against both orders
+          //   and against one rounding), and the products are exact (changes
+          //   are 0, +-1 or +-2), so the fields round as with one VALU update
+          //   per visit.
+          constexpr int JR = 2;
+          const float4* jb4 = reinterpret_cast<const float4*>(L.jb[pb][ti]) + 4 * h;
+          float4 jring[JR][4];
+          auto load_j = [&](auto kc) __attribute__((always_inline)) {
+            constexpr int k = decltype(kc)::value;
+            // k = 8 m + 7 is done with slot group m
+            if constexpr (!MU && k + 1 < kB)
+              static_for<4>([&](auto mc) __attribute__((always_inline)) {
+                constexpr int m4 = decltype(mc)::value;
+                if constexpr (m4 >= (k + 1) >> 3) jring[k % JR][m4] = jb4[k * (kB / 4) + m4];
+              });
+          };
+          static_for<JR>([&](auto dc) __attribute__((always_inline)) { load_j(dc); });
+          const float* ja = &L.jb[pb][ti][lane];
+          const float4* jg = reinterpret_cast<const float4*>(L.ji[pb][ti]);
+          float a_rg[2][2];  // one group ahead of the chain
+          float4 j_rg[2][3];
+          auto load_group = [&](auto gc) __attribute__((always_inline)) {
+            constexpr int g = decltype(gc)::value;
+            if constexpr (MU && g < kB / 4) {
+              if constexpr (g + 1 < kB / 4) {
+                a_rg[g & 1][0] = ja[(4 * g) * kB];
+                a_rg[g & 1][1] = ja[(4 * g + 2) * kB];
+              }
+              j_rg[g & 1][0] = jg[4 * g];
+              j_rg[g & 1][1] = jg[4 * g + 1];
+              j_rg[g & 1][2] = jg[4 * g + 2];
+            }
+          };
+          load_group(std::integral_constant<int, 0>{});
+          // sg = 2 s or 2x - 1 of visit k: one bit insert
+          auto sign_of = [&](int k) __attribute__((always_inline)) {
+            const uint32_t shk = nmb << (31 - k);
+            return __uint_as_float((shk & vsgn) | (cub & ~vsgn));
+          };
+          static_for<kB / 4>([&](auto gc) __attribute__((always_inline)) {
+            constexpr int g = decltype(gc)::value;
+            constexpr int H = g & 1, j0 = 4 * (g >> 1);  // the half that holds the group, its first slot
+            load_group(std::integral_constant<int, g + 1>{});
+            float ff[4] = {fp[j0], fp[j0 + 1], fp[j0 + 2], fp[j0 + 3]}, dS[4];
+            static_for<4>([&](auto ec) __attribute__((always_inline)) {
+              constexpr int e = decltype(ec)::value, k = 4 * g + e;
+              const float f = MU ? ff[e] : fp[j0 + e];
+              // batched: scale * c + h of the count, a product, then a sum
+              const float fk = BAT ? f * bsc + hk[j0 + e] : f;
+              const float sg = sign_of(k);
+              // dn = 2 s (F + h) (ising) or (2x - 1)(F + h) (qubo), exact in f32
+              const float dn = fk * sg;
+              // The half without visit k compares another slot; only the
+              // other's word counts.  Idle lanes and padding rows have lo = hi
+              // = +inf (and finite dn): never taken, never inside their bracket.
+              const uint64_t tb64 = __builtin_amdgcn_ballot_w64(dn > hib[j0 + e]);
+              const uint64_t ib64 = __builtin_amdgcn_ballot_w64(!(dn < lob[j0 + e]));
+              const uint32_t tm = H ? (uint32_t)(tb64 >> 32) : (uint32_t)tb64;
+              // the decisions as the lane mask of both halves (the vector type
+              // keeps it to one scalar move)
+              typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+              const uint64_t tmm = __builtin_bit_cast(uint64_t, (u32x2){tm, tm});
+              // taken ? -sg : 0
+              asm("v_cndmask_b32_e64 %0, 0, -%1, %2" : "=v"(dS[e]) : "v"(sg), "s"(tmm));
+              if constexpr (MU) {
+                if constexpr (e < 3) {
+                  const float4 j4 = j_rg[g & 1][e];
+                  const float jv4[4] = {j4.x, j4.y, j4.z, j4.w};
+                  static_for<4>([&](auto rc) __attribute__((always_inline)) {
+                    constexpr int r = decltype(rc)::value;
+                    if constexpr (r > e) ff[r] = __builtin_fmaf(jv4[r], dS[e], ff[r]);
+                  });
+                }
+                if constexpr (g + 1 < kB / 4 && (e & 1) == 1) {
+                  const float b = h ? dS[e] : dS[e - 1];
+                  fp = __builtin_amdgcn_mfma_f32_32x32x2f32(a_rg[g & 1][e >> 1], b, fp, 0, 0, 0);
+                }
+              } else {
+                // every element of the row's loads counts as used, or the
+                // compiler splits them into narrow ones
+                static_for<4>([&](auto mc) __attribute__((always_inline)) {
+                  constexpr int m4 = decltype(mc)::value;
+                  if constexpr (k + 1 < kB && m4 >= (k + 1) >> 3) use_whole(jring[k % JR][m4]);
+                });
+                static_for<16>([&](auto rc) __attribute__((always_inline)) {
+                  constexpr int r = decltype(rc)::value;
+                  // slot r is a later visit in one half at least (the high
+                  // one's visit is the later)
+                  if constexpr (8 * (r >> 2) + 4 + (r & 3) > k) {
+                    const float4 j4 = jring[k % JR][r >> 2];
+                    const float jv4[4] = {j4.x, j4.y, j4.z, j4.w};
+                    fp[r] = __builtin_fmaf(jv4[r & 3], dS[e], fp[r]);
+                  }
+                });
+                load_j(std::integral_constant<int, k + JR>{});
+              }
+              {
+                uint64_t co;  // tk = 2 tk + taken (the mask as carry-in)
+                asm("v_addc_co_u32_e64 %0, %1, %2, %2, %3"
+                    : "=v"(tk), "=s"(co)
+                    : "v"(tk), "s"(tmm));
+                asm("v_addc_co_u32_e64 %0, %1, %2, %2, %3"
+                    : "=v"(tn), "=s"(co)
+                    : "v"(tn), "s"(ib64));
+                (void)co;
+              }
+              // dS * fk is exactly -dn or 0, so this rounds like dpart - dn
+              // (batched: summed in f64 in visit order, as the oracle sums)
+              if constexpr (BAT)
+                dsum += (double)(dS[e] * fk);
+              else
+                dpart = __builtin_fmaf(dS[e], fk, dpart);
+            });
+            // the sum so far goes to the half of the next group's visits
+            if constexpr (BAT)
+              dsum = half_bcast<H>(dsum);
+            else
+              dpart = half_bcast<H>(dpart);
+          });
+          // a decision not below its bracket and not taken is inside; bits of the
+          // lane's own visits (k / 4 even or odd, bit 31 - k)
+          const uint32_t own = h ? 0x0F0F0F0Fu : 0xF0F0F0F0u;
+          const bool inside = __builtin_amdgcn_ballot_w64(((tn & ~tk) & own) != 0) != 0;
+          mb = mb0 ^ __builtin_bitreverse32(tk);
+          if (__builtin_expect(inside, 0)) {
+            // A decision fell inside its bracket: rerun the block, taking the
+            // exact test for the decisions inside their brackets (rolled loop,
+            // fields staged in LDS; both lanes of a replica do the same).
+            float* sf = &L.sfp[qp * 33];
+#pragma unroll
+            for (int g4 = 0; g4 < 4; ++g4) {
+              float4 v = L.part[pb][0][tw][g4][lane];
+#pragma unroll
+              for (int mm = 1; mm < MW; ++mm) {
+                const float4 y = L.part[pb][mm][tw][g4][lane];
+                v.x = v.x + y.x, v.y = v.y + y.y, v.z = v.z + y.z, v.w = v.w + y.w;
+              }
+              const float vs[4] = {v.x + corr[4 * g4], v.y + corr[4 * g4 + 1], v.z + corr[4 * g4 + 2],
+                                   v.w + corr[4 * g4 + 3]};
+#pragma unroll
+              for (int e = 0; e < 4; ++e) {
+                const int r = 8 * g4 + 4 * h + e;
+                sf[r] = BAT ? vs[e] : __builtin_fmaf(fsc, vs[e] + L.rsb[pb][r], L.hb[pb][ti][r]);
+              }
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            const float beta = L.rb[qp];
+            const int glp = BAT ? (lane & 31) / R : qp / R;  // its read of the tile / group
+            const int rdp = BAT ? tile(ti).read0 + glp : read0 + glp;
+            const bool actp = glp < p.rpw && rdp < (BAT ? tile(ti).read_end : p.reads);
+            const uint64_t cidp = (uint64_t)rdp * R + (BAT ? (lane & 31) - glp * R : qp - glp * R);
+            mb = mb0;
+            dpart = 0.f;
+            if constexpr (BAT) dsum = dsum0;
+            for (int k = 0; k < kB; ++k) {
+              const bool up = (mb >> k) & 1u;
+              const float sg = up ? cu : -cu;
+              const float fk = BAT ? sf[k] * bsc + L.hb[pb][ti][k] : sf[k];
+              const float dn = fk * sg;
+              // idle lanes and padding rows have lo = hi = +inf: never taken
+              bool take = actp & (dn > L.hi[pb][qp][k]);
+              if (actp && !take && !(dn < L.lo[pb][qp][k])) {
+                const uint32_t pk = (uint32_t)(pos0 + (k ^ (int)xm));
+                const uint32_t wd = pick_word(sweep_block(cidp, sw, pk, p.k0, p.k1), pk & 3u);
+                take = accept_exact(wd, beta, dn);
+              }
+              mb ^= (uint32_t)take << k;
+              if constexpr (BAT)
+                dsum += take ? (double)(-dn) : 0.0;
+              else
+                dpart += take ? -dn : 0.f;
+              const float dS = take ? -sg : 0.f;
+              for (int r = k + 1; r < kB; ++r)
+                sf[r] = __builtin_fmaf(!MU                    ? L.jb[pb][ti][k * kB + half_slot(r)]
+                                       : (r >> 2) == (k >> 2) ? L.ji[pb][ti][4 * k + (r & 3)]
+                                                              : L.jb[pb][ti][k * kB + r],
+                                       dS, sf[r]);
+              __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            }
+          }
+          if constexpr (!BAT) dsum += (double)dpart;
+          nacc += (uint32_t)__builtin_popcount(mb ^ mb0);
+        }
+        {
+          const uint32_t mbr = BR ? xor_permute_bits(mb, xm) : mb;  // back to block-row order
+          if (lane < 32) {
+            L.bnew[pb][qp] = mbr;
+            // the same block next (at a pass boundary): its spins are these,
+            // in its next visit order (the owners, whose copy is older, skip it)
+            if (c1 == c) L.bb[pb ^ 1][qp] = BR ? xor_permute_bits(mbr, xm_nx) : mbr;
+          }
+          f32x16 a = {};
+          i32x16 ia = {};
+          mfma_step(fcorr, half_of<I8>(mbr, h), a, ia);
+#pragma unroll
+          for (int v = 0; v < 16; ++v) corr[v] = I8 ? (float)ia[v] : a[v];
+        }
+        if (lastb && lane < 32) {
+          L.ds[qp] = dry ? eacc : dsum;
+          L.nacc[qp] = nacc;
+        }
+        if (dry) {
           __syncthreads();  // B
           if (lastb) {
-            if (act) {
+            if (w == 0 && act) {
               if constexpr (AIS) {
                 if (ps == 0)
-                  eoff = Ed - eacc;
+                  eoff = Ed - L.ds[q];
                 else
-                  Ed = eacc + eoff;
+                  Ed = L.ds[q] + eoff;
               } else {
                 if (ps == 0)
-                  eoff = (double)E - eacc;
+                  eoff = (double)E - L.ds[q];
                 else
-                  E = (float)(eacc + eoff);
+                  E = (float)(L.ds[q] + eoff);
               }
             }
             __syncthreads();  // the next pass's first brackets
           }
           continue;
         }
-        // ---- proposals of block c, one lane per replica
-        // brackets of the block's 32 visits, read first (their latency
-        // overlaps the field sums and they leave the chain free of LDS waits)
-        float hib[kB], lob[kB];
-#pragma unroll
-        for (int t4 = 0; t4 < kB / 4; ++t4) {
-          const float4 a = *reinterpret_cast<const float4*>(&L.hi[pb][qo][4 * t4]);
-          const float4 b = *reinterpret_cast<const float4*>(&L.lo[pb][qo][4 * t4]);
-          hib[4 * t4] = a.x, hib[4 * t4 + 1] = a.y, hib[4 * t4 + 2] = a.z, hib[4 * t4 + 3] = a.w;
-          lob[4 * t4] = b.x, lob[4 * t4 + 1] = b.y, lob[4 * t4 + 2] = b.z, lob[4 * t4 + 3] = b.w;
-        }
-        // fields in visit order (batched: the integer counts, with h in hk)
-        float fp[kB], hk[kB];
-        {
-          const int xg = (int)(xm >> 2);
-          // visit group r4 holds block rows 4 (r4 ^ xg) + (e ^ (xm & 3)); the
-          // in-group part is a compile-time permutation per uniform branch
-          // FM: 0 = sums + h; 1 = (sums + row sums) / 2 + h (QUBO with bf16
-          // operands); 2 = the sums alone (every h zero: adding +0 would only
-          // turn a -0 into +0, which no decision or sum distinguishes)
-          auto load_fields = [&](auto pc, auto fmc) __attribute__((always_inline)) {
-            constexpr int P = decltype(pc)::value;
-            constexpr int FM = decltype(fmc)::value;
-            constexpr bool RS = FM == 1;
-            // kFG groups of 4 rows per stage: every LDS read of a stage is
-            // issued before its first sum, so a stage costs one LDS latency
-#pragma unroll
-            for (int g0 = 0; g0 < kB / 4; g0 += kFG) {
-              float4 ld[kFG][MW + 3];
-#pragma unroll
-              for (int j = 0; j < kFG; ++j) {
-                const int gr = (g0 + j) ^ xg;
-                const int o = fld(qo, 4 * gr);
-#pragma unroll
-                for (int mm = 0; mm < MW; ++mm)
-                  ld[j][mm] = *reinterpret_cast<const float4*>(&L.part[pb][mm][o]);
-                ld[j][MW] = *reinterpret_cast<const float4*>(&L.corr[o]);
-                if constexpr (FM != 2) ld[j][MW + 1] = *reinterpret_cast<const float4*>(&L.hb[pb][tq][4 * gr]);
-                if constexpr (RS) ld[j][MW + 2] = *reinterpret_cast<const float4*>(&L.rsb[pb][4 * gr]);
-              }
-              __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-              for (int j = 0; j < kFG; ++j) {
-                float4 sm = ld[j][0];
-#pragma unroll
-                for (int mm = 1; mm < MW; ++mm) {
-                  sm.x = sm.x + ld[j][mm].x;
-                  sm.y = sm.y + ld[j][mm].y;
-                  sm.z = sm.z + ld[j][mm].z;
-                  sm.w = sm.w + ld[j][mm].w;
-                }
-                const float4 cr = ld[j][MW];
-                const float4 h4 = FM != 2 ? ld[j][MW + 1] : make_float4(0.f, 0.f, 0.f, 0.f);
-                float vs[4] = {sm.x + cr.x, sm.y + cr.y, sm.z + cr.z, sm.w + cr.w};
-                if constexpr (RS) {
-                  const float4 s4 = ld[j][MW + 2];
-                  vs[0] = vs[0] + s4.x, vs[1] = vs[1] + s4.y, vs[2] = vs[2] + s4.z, vs[3] = vs[3] + s4.w;
-                }
-                const float hv[4] = {h4.x, h4.y, h4.z, h4.w};
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                  if constexpr (BAT) {
-                    fp[4 * (g0 + j) + e] = vs[e ^ P];
-                    hk[4 * (g0 + j) + e] = hv[e ^ P];
-                  } else {
-                    if constexpr (FM == 2)
-                      fp[4 * (g0 + j) + e] = vs[e ^ P];
-                    else
-                      fp[4 * (g0 + j) + e] = __builtin_fmaf(fsc, vs[e ^ P], hv[e ^ P]);
-                  }
-                }
-              }
-              __builtin_amdgcn_sched_barrier(0);
-            }
-          };
-          auto load_fm = [&](auto fmc) __attribute__((always_inline)) {
-            switch (xm & 3u) {
-              case 0: load_fields(std::integral_constant<int, 0>{}, fmc); break;
-              case 1: load_fields(std::integral_constant<int, 1>{}, fmc); break;
-              case 2: load_fields(std::integral_constant<int, 2>{}, fmc); break;
-              default: load_fields(std::integral_constant<int, 3>{}, fmc); break;
-            }
-          };
-          if (qsum)
-            load_fm(std::integral_constant<int, 1>{});
-          else if (!BAT && p.hzero)
-            load_fm(std::integral_constant<int, 2>{});
-          else
-            load_fm(std::integral_constant<int, 0>{});
-
-        }
-        // spins in visit order (bit k = block row k ^ xm), as published
-        uint32_t mb = L.bb[pb][qo];
-        const uint32_t mb0 = mb;
-        // accepted flips, step k at bit 31 - k: one add with carry per step
-        uint32_t tk = 0;
-        // bit k of mb is only changed at step k, so every step reads its
-        // spin from the block's initial bits: sign bit = !spin, magnitude cu
-        const uint32_t nmb = ~mb0, cub = __float_as_uint(cu);
-        uint32_t vsgn = 0x80000000u;  // kept in a register (not a literal operand)
-        asm volatile("" : "+v"(vsgn));
-        float dpart = 0.f;
-        const double dsum0 = dsum;  // batched: the sum before the block (for a rerun)
-        uint64_t amb = 0;  // lanes with a decision inside its bracket
-        // Rows of J[blk][blk] (the same for every lane) stream from LDS
-        // through a ring JR rows ahead of the chain.  Row k holds only the
-        // columns right of the diagonal, shifted to the start of the row, so
-        // the ceil((31 - k) / 4) 16-byte loads of a row carry no dead lanes.
-        constexpr int JR = 2;
-        const float4* jb4 = reinterpret_cast<const float4*>(L.jb[pb][tq]);
-        float4 jring[JR][kB / 4];
-        static_for<JR>([&](auto dc) __attribute__((always_inline)) {
-          constexpr int d = decltype(dc)::value;
-          static_for<(kB - 1 - d + 3) / 4>([&](auto tc) __attribute__((always_inline)) {
-            constexpr int t4 = decltype(tc)::value;
-            jring[d][t4] = jb4[d * (kB / 4) + t4];
-          });
-        });
-        static_for<kB>([&](auto kc) __attribute__((always_inline)) {
-          constexpr int k = decltype(kc)::value;
-          // dn = 2 s (F + h) (ising) or (2x - 1)(F + h) (qubo), exact in f32
-          const uint32_t shk = nmb << (31 - k);
-          const float sg = __uint_as_float((shk & vsgn) | (cub & ~vsgn));  // one bit insert
-          // batched: the field scale * c + h of the count (a product, then a sum)
-          const float fk = BAT ? fp[k] * bsc + hk[k] : fp[k];
-          const float dn = fk * sg;
-          const float hik = hib[k], lok = lob[k];
-          // idle lanes and padding rows have lo = hi = +inf (and finite dn):
-          // never taken, never inside their bracket
-          const bool take = dn > hik;
-          // the decision's lane mask, used as it is by the two selects below
-          const uint64_t tm = __builtin_amdgcn_ballot_w64(take);
-          amb |= __builtin_amdgcn_ballot_w64(!(dn < lok)) & ~tm;
-          float dS;  // take ? -sg : 0
-          asm("v_cndmask_b32_e64 %0, 0, -%1, %2" : "=v"(dS) : "v"(sg), "s"(tm));
-          {
-            uint64_t co;  // tk = 2 tk + take (the mask as carry-in)
-            asm("v_addc_co_u32_e64 %0, %1, %2, %2, %3" : "=v"(tk), "=s"(co) : "v"(tk), "s"(tm));
-            (void)co;
-          }
-          // dS * fk is exactly -dn or 0, so this rounds like dpart - dn
-          // (batched: summed in f64 in visit order, as the oracle sums)
-          if constexpr (BAT)
-            dsum += (double)(dS * fk);
-          else
-            dpart = __builtin_fmaf(dS, fp[k], dpart);
-          static_for<(kB - 1 - k + 3) / 4>([&](auto tc) __attribute__((always_inline)) {
-            constexpr int t4 = decltype(tc)::value;
-            const float4 j4 = jring[k % JR][t4];
-            const float jv[4] = {j4.x, j4.y, j4.z, j4.w};
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              const int r = k + 1 + 4 * t4 + e;
-              // dS is 0, +-1 or +-2, so the fused form rounds like mul + add
-              if (r < kB) fp[r] = __builtin_fmaf(jv[e], dS, fp[r]);
-            }
-          });
-          if (k + JR < kB)
-            static_for<(kB - 1 - (k + JR) + 3) / 4>([&](auto tc) __attribute__((always_inline)) {
-              constexpr int t4 = decltype(tc)::value;
-              jring[k % JR][t4] = jb4[(k + JR) * (kB / 4) + t4];
-            });
-        });
-        mb = mb0 ^ __builtin_bitreverse32(tk);
-        if (__builtin_expect(amb != 0, 0)) {
-          // A decision fell inside its bracket: rerun the block, taking the
-          // exact test for the decisions inside their brackets (rolled loop,
-          // fields staged in LDS).
-          float* sf = &L.sfp[qo * 33];
-          for (int r = 0; r < kB; ++r) {  // visit order, as fp
-            const int br = r ^ (int)xm;
-            float v = L.part[pb][0][fld(qo, br)];
-            for (int mm = 1; mm < MW; ++mm) v = v + L.part[pb][mm][fld(qo, br)];
-            v = v + L.corr[fld(qo, br)];
-            sf[r] = BAT ? v : __builtin_fmaf(fsc, v + L.rsb[pb][br], L.hb[pb][tq][br]);
-          }
-          mb = mb0;
-          dpart = 0.f;
-          if constexpr (BAT) dsum = dsum0;
-          for (int k = 0; k < kB; ++k) {
-            const bool up = (mb >> k) & 1u;
-            const float sg = up ? cu : -cu;
-            const float fk = BAT ? sf[k] * bsc + L.hb[pb][tq][k ^ (int)xm] : sf[k];
-            const float dn = fk * sg;
-            // idle lanes and padding rows have lo = hi = +inf: never taken
-            bool take = act & (dn > L.hi[pb][qo][k]);
-            if (act && !take && !(dn < L.lo[pb][qo][k])) {
-              const uint32_t pk = (uint32_t)(pos0 + (k ^ (int)xm));
-              const uint32_t wd = pick_word(sweep_block(cid, sw, pk, p.k0, p.k1), pk & 3u);
-              take = accept_exact(wd, beta, dn);
-            }
-            mb ^= (uint32_t)take << k;
-            if constexpr (BAT)
-              dsum += take ? (double)(-dn) : 0.0;
-            else
-              dpart += take ? -dn : 0.f;
-            const float dS = take ? -sg : 0.f;
-            for (int r = k + 1; r < kB; ++r)
-              sf[r] = __builtin_fmaf(L.jb[pb][tq][k * kB + (r - k - 1)], dS, sf[r]);
-          }
-        }
-        {
-          const uint32_t mbr = BR ? xor_permute_bits(mb, xm) : mb;  // back to block-row order
-          L.bnew[pb][qo] = mbr;
-          // the same block next (at a pass boundary): its spins are these,
-          // in its next visit order (the owners, whose copy is older, skip it)
-          if (c1 == c) L.bb[pb ^ 1][qo] = BR ? xor_permute_bits(mbr, xm_nx) : mbr;
-          corr_products(fcorr, mbr, qo);
-        }
-        if constexpr (!BAT) dsum += (double)dpart;
-        nacc += (uint32_t)__builtin_popcount(mb ^ mb0);
         __syncthreads();  // B
         if (AIS && lastb) {
+          if (w != 0) {
+            __syncthreads();
+            __syncthreads();
+            __syncthreads();
+            continue;
+          }
           // ---- end of an AIS step (simulation.py:305-316 with the uniform
           // reference: its log-density is 0): the energy after the sweep, the
           // weight of this step (ordering 0) or of the next one before its
           // sweep (ordering 1), and the next step's beta for every chain
-          acc += nacc;
-          Ed = Ed + dsum;
+          acc += L.nacc[q];
+          Ed = Ed + L.ds[q];
           const double bt = (double)p.temps[s];
           if (act && p.ordering == 0) lw = lw + ((-bt * Ed) - (-bold * Ed));
           bold = bt;
@@ -897,9 +1052,16 @@ __global__ __launch_bounds__(128 * (MW + 1)) void blocked_pipe_kernel(BParams p0
           __syncthreads();
           __syncthreads();  // the next pass's first brackets
         } else if (lastb) {
+          if (w != 0) {
+            __syncthreads();
+            __syncthreads();
+            __syncthreads();
+            continue;
+          }
           // ---- end of sweep: energy (simulation.py:157-158), best states, PT
-          acc += nacc;
-          E = (float)((double)E + dsum);
+          // (lane = replica)
+          acc += L.nacc[q];
+          E = (float)((double)E + L.ds[q]);
           L.E[q] = E;
           if (p.best_sem == 0) {  // simulation.py:161-164
             const bool imp = act && (E < bestE);
@@ -917,7 +1079,7 @@ __global__ __launch_bounds__(128 * (MW + 1)) void blocked_pipe_kernel(BParams p0
           // index: hoisted to the kernel start they were kept in scratch.
           int qx = q;
           asm volatile("" : "+v"(qx));
-          const int tx = BAT ? (qx >> 5) : 0;
+          const int tx = BAT && NT == 2 ? (qx >> 5) : 0;
           const int b0 = BAT ? 32 * tx + ((qx & 31) / R) * R : (qx / R) * R;  // the read's first lane
           const int slot = qx - b0;
           const float* bet = &L.bet[32 * tx];
@@ -951,12 +1113,12 @@ __global__ __launch_bounds__(128 * (MW + 1)) void blocked_pipe_kernel(BParams p0
               float ec = L.Es[b0 + R - 1], ba = bet[R - 1];
               int rbn = L.bi[b0 + R - 2];
               float ebn = L.Es[b0 + R - 2], bbn = bet[R - 2];
-              double lun = L.lu[b0];
+              float lun = L.lu[b0];
               for (int k = 0; k < R - 1; ++k) {
                 const int a = R - k - 1, b = a - 1;
                 const int rb = rbn;
                 const float eb = ebn, bb = bbn;
-                const double luk = lun;
+                const float luk = lun;
                 if (b > 0) {
                   rbn = L.bi[b0 + b - 1];
                   ebn = L.Es[b0 + b - 1];
@@ -964,7 +1126,7 @@ __global__ __launch_bounds__(128 * (MW + 1)) void blocked_pipe_kernel(BParams p0
                   lun = L.lu[b0 + k + 1];
                 }
                 const float dd = (ec - eb) * (ba - bb);
-                const bool x = dd >= 0.f || luk < (double)dd;
+                const bool x = dd >= luk;  // dd >= 0 or log u < dd (log u < 0)
                 L.bi[b0 + a] = x ? rb : carry;
                 if (!x) {
                   carry = rb;
@@ -974,23 +1136,28 @@ __global__ __launch_bounds__(128 * (MW + 1)) void blocked_pipe_kernel(BParams p0
               }
               L.bi[b0] = carry;
             }
-            if (p.logw && p.log_omegas) {  // ais.py:99-112 over the ascending ladder
-              double lw = 0.0, bold = 0.0;
-              for (int r = 1; r < R; ++r) {
-                const int k = L.bso[r];
-                const float be = bet[k];
-                const float en = L.E[b0 + L.bi[b0 + k]];
-                const float a = -be * en;
-                lw += (double)a - (-bold * (double)en);
-                bold = (double)be;
-              }
-              p.log_omegas[(size_t)read * p.S + s] = lw;
-            }
             L.src[g] = src;
           }
           // every slot's new beta to the replica now in it (after the
           // leader's exchanges: the same wave, in order)
           if (act) L.rb[b0 + L.bi[qx]] = bet[slot];
+          if (p.logw && p.log_omegas) {  // ais.py:99-112 over the ascending ladder
+            // lane r: its term, then the leader adds them in order
+            if (act && slot > 0) {
+              const int k = L.bso[slot];
+              const float en = L.E[b0 + L.bi[b0 + k]];
+              const float a = -bet[k] * en;
+              const double bold = slot > 1 ? (double)bet[L.bso[slot - 1]] : 0.0;
+              L.ds[qx] = (double)a - (-bold * (double)en);
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            if (act && rr == 0) {
+              double lw = 0.0;
+#pragma unroll 4
+              for (int r = 1; r < R; ++r) lw += L.ds[b0 + r];
+              p.log_omegas[(size_t)read * p.S + s] = lw;
+            }
+          }
           __syncthreads();
           __syncthreads();  // the next pass's first brackets
         }
@@ -1012,7 +1179,7 @@ __global__ __launch_bounds__(128 * (MW + 1)) void blocked_pipe_kernel(BParams p0
       for (int tb = 0; tb < nblk; ++tb, ++t) {
         const int pb = t & 1, pn = pb ^ 1;
         // the schedule of the next pass, needed from step nblk - 2 on
-        if (BR && w == 4 && tb == 0) fill_sched(sp ^ 1, sw_next, dry_next);
+        if (BR && w == 7 && tb == 0) fill_sched(sp ^ 1, sw_next, dry_next);
         const bool last = tb + 1 == nblk;
         const int p2 = tb + 2 < nblk ? sp : sp ^ 1, i2 = tb + 2 < nblk ? tb + 2 : tb + 2 - nblk;
         // The entry two steps ahead is read here and made wave-uniform where
@@ -1029,24 +1196,28 @@ __global__ __launch_bounds__(128 * (MW + 1)) void blocked_pipe_kernel(BParams p0
           // c1's spins have not changed since its last visit unless c1 == c
           // (a pass boundary), which the proposal wave publishes itself
           if (w == owner_of(c1) && c1 != c) publish_bits(c1, pn, m1);
-          compute_part(c1, c, L.part[pn][m]);
+          compute_part(c1, m1, c, pn);
           const uint32_t en2 = entry2();
           c2 = entry_block(en2);
           m2 = entry_mask(en2);
-          prefetch_frags(c2);
+          prefetch_frags(c2, m2);
         }
         if (hw) {
           publish_block(pn);
-          if (w > MW + 1 && !last && !dry) brackets(c1, m1, sw, pn);
+          if (!last) {
+            if (!dry) brackets(c1, m1, sw, pn);
+          } else if (!dry_next) {
+            draw(c1, sw_next, lgn);
+          }
           const uint32_t en2 = entry2();
           c2 = entry_block(en2);
           m2 = entry_mask(en2);
           prefetch_jb(c2, m2);
           // the sweep's exchange uniforms (utils.py:57), by a helper that has
           // no brackets to compute during the last block
-          if (w == MW + 2 && last && !dry && p.use_pt && act && rr < R - 1)
-            L.lu[q] = log_u32(pick_word(pt_block((uint64_t)read, sw, (uint32_t)rr, p.k0, p.k1),
-                                        (uint32_t)rr & 3u));
+          if (w == 7 && last && !dry && p.use_pt && act && rr < R - 1)
+            L.lu[q] = float_above(log_u32(pick_word(
+                pt_block((uint64_t)read, sw, (uint32_t)rr, p.k0, p.k1), (uint32_t)rr & 3u)));
         }
         __syncthreads();  // B
         // ---- the owners of block c take its new spins
@@ -1071,7 +1242,10 @@ __global__ __launch_bounds__(128 * (MW + 1)) void blocked_pipe_kernel(BParams p0
                 store_range<NW, I8>(sa[tt], c0, kb, nblk, n_of(tt), p.ptype, best_of(tt));
           }
           // the next pass's first block (after the exchanges: new betas)
-          if (hw && w > MW + 1 && !dry_next) brackets(c1, m1, sw_next, pn);
+          if (hw && !dry_next) {
+            sweep_factors();
+            finish(c1, m1, lgn, pn);
+          }
           __syncthreads();
         }
         c = c1;
@@ -1134,12 +1308,15 @@ hipError_t launch_pipe_enc(const BParams& p, int nw, int nt, int groups, hipStre
                  : launch_pipe_o<NP, I8, false, 1>(p, nw, groups, st);
 }
 
-// AIS (kModeAIS) with one coupling encoding: two tiles of 32 chains per
+// AIS (kModeAIS) with one coupling encoding: nt tiles of 32 chains per
 // workgroup, the order from p.
 template <int NP, bool I8>
-hipError_t launch_pipe_ais_enc(const BParams& p, int nw, int groups, hipStream_t st) {
-  return p.order == kBlockRandom ? launch_pipe_o<NP, I8, true, 2, kModeAIS>(p, nw, groups, st)
-                                 : launch_pipe_o<NP, I8, false, 2, kModeAIS>(p, nw, groups, st);
+hipError_t launch_pipe_ais_enc(const BParams& p, int nw, int nt, int groups, hipStream_t st) {
+  if (p.order == kBlockRandom)
+    return nt == 2 ? launch_pipe_o<NP, I8, true, 2, kModeAIS>(p, nw, groups, st)
+                   : launch_pipe_o<NP, I8, true, 1, kModeAIS>(p, nw, groups, st);
+  return nt == 2 ? launch_pipe_o<NP, I8, false, 2, kModeAIS>(p, nw, groups, st)
+                 : launch_pipe_o<NP, I8, false, 1, kModeAIS>(p, nw, groups, st);
 }
 
 // One per translation unit (blocked_pipe_i8.hip, blocked_pipe_bf16_{1,2,3}.hip).
@@ -1147,12 +1324,12 @@ hipError_t launch_pipe_i8(const BParams& p, int nw, int nt, int groups, hipStrea
 hipError_t launch_pipe_bf16_1(const BParams& p, int nw, int nt, int groups, hipStream_t st);
 hipError_t launch_pipe_bf16_2(const BParams& p, int nw, int nt, int groups, hipStream_t st);
 hipError_t launch_pipe_bf16_3(const BParams& p, int nw, int nt, int groups, hipStream_t st);
-hipError_t launch_pipe_ais_i8(const BParams& p, int nw, int groups, hipStream_t st);
-hipError_t launch_pipe_ais_bf16_1(const BParams& p, int nw, int groups, hipStream_t st);
-hipError_t launch_pipe_ais_bf16_2(const BParams& p, int nw, int groups, hipStream_t st);
-hipError_t launch_pipe_ais_bf16_3(const BParams& p, int nw, int groups, hipStream_t st);
+hipError_t launch_pipe_ais_i8(const BParams& p, int nw, int nt, int groups, hipStream_t st);
+hipError_t launch_pipe_ais_bf16_1(const BParams& p, int nw, int nt, int groups, hipStream_t st);
+hipError_t launch_pipe_ais_bf16_2(const BParams& p, int nw, int nt, int groups, hipStream_t st);
+hipError_t launch_pipe_ais_bf16_3(const BParams& p, int nw, int nt, int groups, hipStream_t st);
 // The batched form (blocked_pipe_bat.hip): one workgroup per entry of p.bat.
-hipError_t launch_pipe_bat(const BParams& p, int nw, int groups, hipStream_t st);
+hipError_t launch_pipe_bat(const BParams& p, int nw, int nt, int groups, hipStream_t st);
 
 }  // namespace blk
 }  // namespace pysa

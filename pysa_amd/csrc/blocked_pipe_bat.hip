@@ -15,9 +15,12 @@
 namespace pysa {
 namespace blk {
 
-hipError_t launch_pipe_bat(const BParams& p, int nw, int groups, hipStream_t st) {
-  return p.order == kBlockRandom ? launch_pipe_o<1, true, true, 2, kModeBatched>(p, nw, groups, st)
-                                 : launch_pipe_o<1, true, false, 2, kModeBatched>(p, nw, groups, st);
+hipError_t launch_pipe_bat(const BParams& p, int nw, int nt, int groups, hipStream_t st) {
+  if (p.order == kBlockRandom)
+    return nt == 2 ? launch_pipe_o<1, true, true, 2, kModeBatched>(p, nw, groups, st)
+                   : launch_pipe_o<1, true, true, 1, kModeBatched>(p, nw, groups, st);
+  return nt == 2 ? launch_pipe_o<1, true, false, 2, kModeBatched>(p, nw, groups, st)
+                 : launch_pipe_o<1, true, false, 1, kModeBatched>(p, nw, groups, st);
 }
 
 namespace {
@@ -140,13 +143,16 @@ hipError_t BatchedMfmaRun::enqueue(const BatchParams& bp, const std::vector<int>
     }
     foff += (int64_t)nblk * nblk * 64 * 16;
   }
+  // One tile per workgroup while each gets a compute unit of its own (its
+  // block step is the shorter one), else two.
+  const int nt = (int)tiles.size() <= device_cus() ? 1 : 2;
   for (size_t i = 0; i < tiles.size();) {
     BatWG g;
     g.nblk = tnb[i];
     g.kb = (g.nblk + kPipeMW - 1) / kPipeMW;
     g.pad0 = g.pad1 = 0;
     g.t[0] = tiles[i];
-    const bool pair = i + 1 < tiles.size() && tnb[i + 1] == tnb[i];
+    const bool pair = nt == 2 && i + 1 < tiles.size() && tnb[i + 1] == tnb[i];
     g.t[1] = pair ? tiles[i + 1] : tiles[i];
     if (!pair) g.t[1].read_end = g.t[1].read0;  // an empty tile (valid pointers, no reads)
     wg.push_back(g);
@@ -199,7 +205,7 @@ hipError_t BatchedMfmaRun::enqueue(const BatchParams& bp, const std::vector<int>
   p.accepted = bp.accepted;
   p.bat = (const BatWG*)tab;
   p.sgn = bp.signs;
-  e = launch_pipe_bat(p, nw, (int)wg.size(), st);
+  e = launch_pipe_bat(p, nw, nt, (int)wg.size(), st);
   if (e == hipSuccess && bp.best_sem == 0) e = bat_best_argmin(p, (int)wg.size(), st);
   return e;
 }

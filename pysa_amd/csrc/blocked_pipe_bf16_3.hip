@@ -8,8 +8,8 @@ hipError_t launch_pipe_bf16_3(const BParams& p, int nw, int nt, int groups, hipS
   return launch_pipe_enc<3, false>(p, nw, nt, groups, st);
 }
 
-hipError_t launch_pipe_ais_bf16_3(const BParams& p, int nw, int groups, hipStream_t st) {
-  return launch_pipe_ais_enc<3, false>(p, nw, groups, st);
+hipError_t launch_pipe_ais_bf16_3(const BParams& p, int nw, int nt, int groups, hipStream_t st) {
+  return launch_pipe_ais_enc<3, false>(p, nw, nt, groups, st);
 }
 
 }  // namespace blk

@@ -20,8 +20,10 @@
 
 #if defined(__HIPCC__)
 #define PYSA_HD __host__ __device__ __forceinline__
+#define PYSA_HD_M __host__ __device__ __forceinline__
 #else
 #define PYSA_HD static inline
+#define PYSA_HD_M inline
 #endif
 
 namespace pysa {
@@ -49,6 +51,15 @@ PYSA_HD void mulhilo32(uint32_t a, uint32_t b, uint32_t* hi, uint32_t* lo) {
   *lo = (uint32_t)p;
 }
 
+// a ^ b ^ c: one instruction on the device.
+PYSA_HD uint32_t xor3(uint32_t a, uint32_t b, uint32_t c) {
+#if defined(__HIP_DEVICE_COMPILE__) && defined(__gfx950__)
+  return __builtin_amdgcn_bitop3_b32(a, b, c, 0x96);
+#else
+  return a ^ b ^ c;
+#endif
+}
+
 PYSA_HD u32x4 philox4x32_10(u32x4 c, uint32_t k0, uint32_t k1) {
   const uint32_t M0 = 0xD2511F53u, M1 = 0xCD9E8D57u;
   const uint32_t W0 = 0x9E3779B9u, W1 = 0xBB67AE85u;
@@ -60,9 +71,9 @@ PYSA_HD u32x4 philox4x32_10(u32x4 c, uint32_t k0, uint32_t k1) {
     mulhilo32(M0, c.x, &hi0, &lo0);
     mulhilo32(M1, c.z, &hi1, &lo1);
     u32x4 n;
-    n.x = hi1 ^ c.y ^ k0;
+    n.x = xor3(hi1, c.y, k0);
     n.y = lo1;
-    n.z = hi0 ^ c.w ^ k1;
+    n.z = xor3(hi0, c.w, k1);
     n.w = lo0;
     c = n;
     k0 += W0;
@@ -204,6 +215,54 @@ PYSA_HD u32x4 sweep_block(uint64_t chain, uint64_t sweep, uint32_t pos, uint32_t
   c.w = chain_sweep_hi(chain, sweep);
   return philox4x32_10(c, k0, k1);
 }
+
+// sweep_block of one chain for many positions: what the first two rounds share
+// over positions (and over a sweep) is computed once.
+struct SweepStream {
+  uint32_t hi1, lo1, chain_hi, k0, k1;  // M1 times counter word 2 (the chain's)
+  PYSA_HD_M explicit SweepStream(uint64_t chain, uint32_t key0, uint32_t key1) : k0(key0), k1(key1) {
+    mulhilo32(0xCD9E8D57u, ((uint32_t)chain & 0x00FFFFFFu) | (kStreamSweep << 24), &hi1, &lo1);
+    chain_hi = (uint32_t)((chain >> 24) & 0xFFFFu);
+  }
+  struct Sweep {
+    uint32_t hi, lo, w;  // round 2: M0 times word 0; counter word 3
+  };
+  PYSA_HD_M Sweep sweep(uint64_t sw) const {
+    Sweep s;
+    s.w = chain_hi | ((uint32_t)((sw >> 32) & 0xFFFFu) << 16);
+    mulhilo32(0xD2511F53u, hi1 ^ (uint32_t)sw ^ k0, &s.hi, &s.lo);
+    return s;
+  }
+  // The block of positions 4 x .. 4 x + 3.
+  PYSA_HD_M u32x4 block(const Sweep& s, uint32_t x) const {
+    const uint32_t M0 = 0xD2511F53u, M1 = 0xCD9E8D57u, W0 = 0x9E3779B9u, W1 = 0xBB67AE85u;
+    uint32_t h, l, h0, l0, h1, l1;
+    mulhilo32(M0, x, &h, &l);                     // round 1: words (hi1 ^ .., lo1, h ^ .., l)
+    mulhilo32(M1, xor3(h, s.w, k1), &h1, &l1);        // round 2
+    u32x4 c;
+    c.x = xor3(h1, lo1, k0 + W0);
+    c.y = l1;
+    c.z = xor3(s.hi, l, k1 + W1);
+    c.w = s.lo;
+    uint32_t a = k0 + 2 * W0, b = k1 + 2 * W1;
+#if defined(__HIP_DEVICE_COMPILE__)
+#pragma unroll
+#endif
+    for (int r = 2; r < 10; ++r) {
+      mulhilo32(M0, c.x, &h0, &l0);
+      mulhilo32(M1, c.z, &h1, &l1);
+      u32x4 n;
+      n.x = xor3(h1, c.y, a);
+      n.y = l1;
+      n.z = xor3(h0, c.w, b);
+      n.w = l0;
+      c = n;
+      a += W0;
+      b += W1;
+    }
+    return c;
+  }
+};
 
 PYSA_HD u32x4 pt_block(uint64_t read, uint64_t sweep, uint32_t pair, uint32_t k0, uint32_t k1) {
   u32x4 c;

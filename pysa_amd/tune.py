@@ -54,7 +54,7 @@ def device_key():
 
 
 def shape_key(n, R, reads, order, float_type="float32"):
-    return f"n={n}/{float_type}/R={R}/reads={reads}/order={order}/{device_key()}"
+    return f"v2/n={n}/{float_type}/R={R}/reads={reads}/order={order}/{device_key()}"
 
 
 def candidates(n, R, order):
@@ -62,7 +62,7 @@ def candidates(n, R, order):
     nblk = (n + 31) // 32
     tiles = (1, 2) if R <= 32 else (2,)
     out = []
-    if nblk >= 3 or order == _lib.ORDER["block_random"]:
+    if nblk >= 2 or order == _lib.ORDER["block_random"]:
         out += [(1, t) for t in tiles]
     if order == _lib.ORDER["sequential"]:
         out.append((2, 0))
