@@ -48,6 +48,24 @@ struct DevBuf {
   }
 };
 
+// Pinned host memory.
+struct HostBuf {
+  void* p = nullptr;
+  size_t bytes = 0;
+  hipError_t ensure(size_t b) {
+    if (b <= bytes) return hipSuccess;
+    if (p) (void)hipHostFree(p);
+    p = nullptr;
+    bytes = 0;
+    hipError_t e = hipHostMalloc(&p, b, hipHostMallocDefault);
+    if (e == hipSuccess) bytes = b;
+    return e;
+  }
+  ~HostBuf() {
+    if (p) (void)hipHostFree(p);
+  }
+};
+
 struct Problem {
   int n = 0, ptype = 0, dtype = 0, device = 0;
   bool symmetric = true;
@@ -65,6 +83,8 @@ struct Problem {
   std::mutex mu;  // calls on one problem are serialised
   // scratch reused across calls
   DevBuf fields, best_rep, best_rep_e, best_rep_sw, work;
+  DevBuf stage;  // device arrays of the host-pointer entry points (Arena)
+  HostBuf pin;   // their copies on the way, when small
   pysa::BlockedProblem blocked;
   ~Problem() {
     (void)hipSetDevice(device);
@@ -269,22 +289,104 @@ int run_device(Problem* P, const RunArgs& a, hipStream_t st, double* ms) {
   return run_plain<T>(P, b, st, ms);
 }
 
-int metropolis_device(int64_t handle, const RunArgs& a, double* kernel_ms, void* stream) {
-  Problem* P = get(handle);
-  int rc = check_run(P, a);
-  if (rc) return rc;
-  std::lock_guard<std::mutex> lk(P->mu);
-  HIP_TRY(hipSetDevice(P->device));
-  hipStream_t st = stream ? (hipStream_t)stream : P->stream;
+// A checked run on device arrays, the problem locked.
+int metropolis_locked(Problem* P, const RunArgs& a, double* kernel_ms, hipStream_t st) {
   double ms = 0.0;
-  rc = (P->dtype == 0) ? run_device<float>(P, a, st, &ms) : run_device<double>(P, a, st, &ms);
+  const int rc = (P->dtype == 0) ? run_device<float>(P, a, st, &ms) : run_device<double>(P, a, st, &ms);
   if (rc) return rc;
   HIP_TRY(hipStreamSynchronize(st));
   if (kernel_ms) *kernel_ms = ms;
   return 0;
 }
 
-// Device copies of host arrays for the host-pointer entry points.
+int metropolis_device(int64_t handle, const RunArgs& a, double* kernel_ms, void* stream) {
+  Problem* P = get(handle);
+  int rc = check_run(P, a);
+  if (rc) return rc;
+  std::lock_guard<std::mutex> lk(P->mu);
+  HIP_TRY(hipSetDevice(P->device));
+  return metropolis_locked(P, a, kernel_ms, stream ? (hipStream_t)stream : P->stream);
+}
+
+// The device arrays of one host-pointer call in one block of memory that the
+// problem keeps for the next call (up to kKeep bytes; a larger block lives for
+// the call).  Arrays are added in the order inputs, inputs that are also
+// outputs, outputs, scratch, so the copies in and out cover one range each:
+// below kPin bytes each is a single copy through pinned memory.  (Before, a call
+// made and freed a buffer per array and copied each by itself: about 1 ms a
+// call, of which a short run of a small problem is a fraction.)
+struct Arena {
+  static constexpr size_t kKeep = size_t(256) << 20, kPin = size_t(1) << 20;
+  struct Item {
+    const void* src;
+    void* dst;
+    size_t bytes, off;
+  };
+  std::vector<Item> items;
+  size_t total = 0;
+  Problem* P;
+  DevBuf own;
+  char* base = nullptr;
+  explicit Arena(Problem* p) : P(p) { items.reserve(16); }
+  int add(const void* src, void* dst, size_t bytes) {
+    items.push_back({src, dst, bytes, total});
+    total += (bytes + 255) & ~size_t(255);
+    return (int)items.size() - 1;
+  }
+  template <typename T>
+  T* at(int i) const {
+    return reinterpret_cast<T*>(base + items[i].off);
+  }
+  // Allocates and copies the inputs in.
+  hipError_t up(hipStream_t st) {
+    DevBuf& b = total <= kKeep ? P->stage : own;
+    hipError_t e = b.ensure(total ? total : 1);
+    if (e != hipSuccess) return e;
+    base = (char*)b.p;
+    size_t end = 0;
+    for (const Item& it : items)
+      if (it.src) end = it.off + it.bytes;
+    if (end == 0) return hipSuccess;
+    if (end <= kPin && (e = P->pin.ensure(kPin)) == hipSuccess) {
+      for (const Item& it : items)
+        if (it.src) memcpy((char*)P->pin.p + it.off, it.src, it.bytes);
+      return hipMemcpyAsync(base, P->pin.p, end, hipMemcpyHostToDevice, st);
+    }
+    for (const Item& it : items)
+      if (it.src && it.bytes) {
+        e = hipMemcpyAsync(base + it.off, it.src, it.bytes, hipMemcpyHostToDevice, st);
+        if (e != hipSuccess) return e;
+      }
+    return hipSuccess;
+  }
+  // Copies the outputs back and waits for them.
+  hipError_t down(hipStream_t st) {
+    size_t lo = total, hi = 0;
+    for (const Item& it : items)
+      if (it.dst) {
+        lo = it.off < lo ? it.off : lo;
+        hi = it.off + it.bytes;
+      }
+    if (hi <= lo) return hipStreamSynchronize(st);
+    hipError_t e;
+    if (hi - lo <= kPin && (e = P->pin.ensure(kPin)) == hipSuccess) {
+      e = hipMemcpyAsync(P->pin.p, base + lo, hi - lo, hipMemcpyDeviceToHost, st);
+      if (e == hipSuccess) e = hipStreamSynchronize(st);
+      if (e != hipSuccess) return e;
+      for (const Item& it : items)
+        if (it.dst) memcpy(it.dst, (const char*)P->pin.p + (it.off - lo), it.bytes);
+      return hipSuccess;
+    }
+    for (const Item& it : items)
+      if (it.dst && it.bytes) {
+        e = hipMemcpyAsync(it.dst, base + it.off, it.bytes, hipMemcpyDeviceToHost, st);
+        if (e != hipSuccess) return e;
+      }
+    return hipStreamSynchronize(st);
+  }
+};
+
+// Device copies of the replay arrays, freed after the call.
 struct Staged {
   std::vector<void*> ptrs;
   ~Staged() {
@@ -567,6 +669,7 @@ int pysa_amd_metropolis(int64_t handle, int32_t reads, int32_t R, int32_t S, int
                energies, beta_idx, best_state, best_energy, best_sweeps, log_omegas, accepted};
   int rc = check_run(P, a);
   if (rc) return rc;
+  std::lock_guard<std::mutex> lk(P->mu);
   HIP_TRY(hipSetDevice(P->device));
   const size_t es = esize(P->dtype), n = P->n, cnt = (size_t)reads * R;
   const size_t rep = (size_t)reads * S * R * n;
@@ -574,51 +677,41 @@ int pysa_amd_metropolis(int64_t handle, int32_t reads, int32_t R, int32_t S, int
   Staged sg;
   RunArgs d = a;
   void* t;
-  HIP_TRY(sg.up(betas, R * es, &t, st));
-  d.betas = t;
-  HIP_TRY(sg.up(beta_sort, R * sizeof(int32_t), &t, st));
-  d.bsort = (const int32_t*)t;
   HIP_TRY(sg.up(replay_log_r, rep * sizeof(double), &t, st));
   d.rep_lr = (const double*)t;
   HIP_TRY(sg.up(replay_perm, rep * sizeof(int32_t), &t, st));
   d.rep_perm = (const int32_t*)t;
   HIP_TRY(sg.up(replay_pt_logu, (size_t)reads * S * (R > 1 ? R - 1 : 1) * sizeof(double), &t, st));
   d.rep_pt = (const double*)t;
-  HIP_TRY(sg.up(states, cnt * n, &t, st));
-  d.states = (int8_t*)t;
-  HIP_TRY(sg.up(energies, cnt * es, &t, st));
-  d.energies = t;
-  HIP_TRY(sg.alloc(cnt * sizeof(int64_t), &t));
-  d.beta_idx = (int64_t*)t;
-  HIP_TRY(sg.alloc((size_t)reads * n, &t));
-  d.best_state = (int8_t*)t;
-  HIP_TRY(sg.alloc((size_t)reads * es, &t));
-  d.best_energy = t;
-  HIP_TRY(sg.alloc((size_t)reads * sizeof(int32_t), &t));
-  d.best_sweeps = (int32_t*)t;
-  d.log_omegas = nullptr;
-  if (log_omega && log_omegas) {
-    HIP_TRY(sg.alloc((size_t)reads * S * sizeof(double), &t));
-    d.log_omegas = (double*)t;
+  const bool lo = log_omega && log_omegas;
+  Arena ar(P);
+  const int i_be = ar.add(betas, nullptr, R * es);
+  const int i_bs = beta_sort ? ar.add(beta_sort, nullptr, R * sizeof(int32_t)) : -1;
+  const int i_st = ar.add(states, states, cnt * n);
+  const int i_en = ar.add(energies, energies, cnt * es);
+  const int i_bi = ar.add(nullptr, beta_idx, cnt * sizeof(int64_t));
+  const int i_bst = ar.add(nullptr, best_state, (size_t)reads * n);
+  const int i_ben = ar.add(nullptr, best_energy, (size_t)reads * es);
+  const int i_bsw = ar.add(nullptr, best_sweeps, (size_t)reads * sizeof(int32_t));
+  const int i_lo = lo ? ar.add(nullptr, log_omegas, (size_t)reads * S * sizeof(double)) : -1;
+  const int i_ac = accepted ? ar.add(nullptr, accepted, (size_t)reads * sizeof(uint64_t)) : -1;
+  HIP_TRY(ar.up(st));
+  d.betas = ar.at<void>(i_be);
+  d.bsort = i_bs >= 0 ? ar.at<const int32_t>(i_bs) : nullptr;
+  d.states = ar.at<int8_t>(i_st);
+  d.energies = ar.at<void>(i_en);
+  d.beta_idx = ar.at<int64_t>(i_bi);
+  d.best_state = ar.at<int8_t>(i_bst);
+  d.best_energy = ar.at<void>(i_ben);
+  d.best_sweeps = ar.at<int32_t>(i_bsw);
+  d.log_omegas = lo ? ar.at<double>(i_lo) : nullptr;
+  d.accepted = accepted ? ar.at<uint64_t>(i_ac) : nullptr;
+  rc = metropolis_locked(P, d, kernel_ms, st);
+  if (rc) {
+    (void)hipStreamSynchronize(st);  // nothing in flight when the replay arrays are freed
+    return rc;
   }
-  d.accepted = nullptr;
-  if (accepted) {
-    HIP_TRY(sg.alloc((size_t)reads * sizeof(uint64_t), &t));
-    d.accepted = (uint64_t*)t;
-  }
-  HIP_TRY(hipStreamSynchronize(st));
-  rc = metropolis_device(handle, d, kernel_ms, st);
-  if (rc) return rc;
-  HIP_TRY(hipMemcpy(states, d.states, cnt * n, hipMemcpyDeviceToHost));
-  HIP_TRY(hipMemcpy(energies, d.energies, cnt * es, hipMemcpyDeviceToHost));
-  HIP_TRY(hipMemcpy(beta_idx, d.beta_idx, cnt * sizeof(int64_t), hipMemcpyDeviceToHost));
-  HIP_TRY(hipMemcpy(best_state, d.best_state, (size_t)reads * n, hipMemcpyDeviceToHost));
-  HIP_TRY(hipMemcpy(best_energy, d.best_energy, (size_t)reads * es, hipMemcpyDeviceToHost));
-  HIP_TRY(hipMemcpy(best_sweeps, d.best_sweeps, (size_t)reads * sizeof(int32_t), hipMemcpyDeviceToHost));
-  if (d.log_omegas)
-    HIP_TRY(hipMemcpy(log_omegas, d.log_omegas, (size_t)reads * S * sizeof(double), hipMemcpyDeviceToHost));
-  if (d.accepted)
-    HIP_TRY(hipMemcpy(accepted, d.accepted, (size_t)reads * sizeof(uint64_t), hipMemcpyDeviceToHost));
+  HIP_TRY(ar.down(st));
   return 0;
 }
 
@@ -651,19 +744,18 @@ int pysa_amd_ais(int64_t handle, const void* temps, int32_t nt, int32_t chains, 
     HIP_TRY(hipSetDevice(P->device));
     hipStream_t st = P->stream;
     const size_t n = P->n;
-    Staged sg;
-    void *dT, *dS, *dE, *dW;
-    HIP_TRY(sg.up(temps, (size_t)nt * sizeof(float), &dT, st));
-    HIP_TRY(sg.up(states, (size_t)chains * n, &dS, st));
-    HIP_TRY(sg.alloc((size_t)chains * sizeof(double), &dE));
-    HIP_TRY(sg.alloc((size_t)chains * sizeof(double), &dW));
-    void* dX = nullptr;
-    const size_t xb = pysa::energy_scratch_bytes((int)n, chains);
-    if (xb) HIP_TRY(sg.alloc(xb, &dX));
+    Arena ar(P);
+    const int i_t = ar.add(temps, nullptr, (size_t)nt * sizeof(float));
+    const int i_s = ar.add(states, states, (size_t)chains * n);
+    const int i_e = ar.add(nullptr, energies, (size_t)chains * sizeof(double));
+    const int i_w = ar.add(nullptr, log_w, (size_t)chains * sizeof(double));
+    const int i_x = ar.add(nullptr, nullptr, pysa::energy_scratch_bytes((int)n, chains));
+    HIP_TRY(ar.up(st));
+    int8_t* dS = ar.at<int8_t>(i_s);
+    double* dE = ar.at<double>(i_e);
     // the initial energies in f64 (simulation.py:301)
-    hipError_t le = pysa::launch_energy_f64<float>((const float*)P->dJt, (const float*)P->dh,
-                                                   (const int8_t*)dS, (double*)dE, (int)n, chains,
-                                                   (double*)dX, st);
+    hipError_t le = pysa::launch_energy_f64<float>((const float*)P->dJt, (const float*)P->dh, dS, dE,
+                                                   (int)n, chains, ar.at<double>(i_x), st);
     if (le != hipSuccess) {
       (void)hipStreamSynchronize(st);
       return fail(PYSA_AMD_EHIP, std::string("energy launch: ") + hipGetErrorString(le));
@@ -671,15 +763,15 @@ int pysa_amd_ais(int64_t handle, const void* temps, int32_t nt, int32_t chains, 
     std::string why;
     double ms = 0.0;
     const int rc = pysa::run_blocked_ais(P->blocked, P->dJ, P->dJt, P->dh, (int)n, P->ptype, chains,
-                                         nt, (const float*)dT, order, ordering,
-                                         form == PYSA_AMD_FORM_BLOCKED_EXACT ? 3 : 0, seed,
-                                         (int8_t*)dS, (double*)dE, (double*)dW, st, &ms, &why);
-    if (rc != 0) return fail(rc, why);
+                                         nt, ar.at<const float>(i_t), order, ordering,
+                                         form == PYSA_AMD_FORM_BLOCKED_EXACT ? 3 : 0, seed, dS, dE,
+                                         ar.at<double>(i_w), st, &ms, &why);
+    if (rc != 0) {
+      (void)hipStreamSynchronize(st);
+      return fail(rc, why);
+    }
     if (kernel_ms) *kernel_ms = ms;
-    HIP_TRY(hipMemcpy(states, dS, (size_t)chains * n, hipMemcpyDeviceToHost));
-    HIP_TRY(hipMemcpy(log_w, dW, (size_t)chains * sizeof(double), hipMemcpyDeviceToHost));
-    if (energies)
-      HIP_TRY(hipMemcpy(energies, dE, (size_t)chains * sizeof(double), hipMemcpyDeviceToHost));
+    HIP_TRY(ar.down(st));
     return 0;
   }
   if (P->n > pysa::kPlainMaxN) return fail(PYSA_AMD_ENOTSUP, "n above 4096");
@@ -820,22 +912,24 @@ int pysa_amd_energy(int64_t handle, const int8_t* states, int64_t count, double*
   std::lock_guard<std::mutex> lk(P->mu);
   HIP_TRY(hipSetDevice(P->device));
   hipStream_t st = P->stream;
-  Staged sg;
-  void *dS, *dO, *dX = nullptr;
-  HIP_TRY(sg.up(states, (size_t)count * P->n, &dS, st));
-  HIP_TRY(sg.alloc((size_t)count * sizeof(double), &dO));
-  const size_t xb = pysa::energy_scratch_bytes(P->n, count);
-  if (xb) HIP_TRY(sg.alloc(xb, &dX));
-  hipError_t le = (P->dtype == 0)
-                      ? pysa::launch_energy_f64<float>((const float*)P->dJt, (const float*)P->dh,
-                                                       (const int8_t*)dS, (double*)dO, P->n, count,
-                                                       (double*)dX, st)
-                      : pysa::launch_energy_f64<double>((const double*)P->dJt, (const double*)P->dh,
-                                                        (const int8_t*)dS, (double*)dO, P->n, count,
-                                                        (double*)dX, st);
-  if (le != hipSuccess) return fail(PYSA_AMD_EHIP, std::string("energy launch: ") + hipGetErrorString(le));
-  HIP_TRY(hipMemcpyAsync(out, dO, (size_t)count * sizeof(double), hipMemcpyDeviceToHost, st));
-  HIP_TRY(hipStreamSynchronize(st));
+  Arena ar(P);
+  const int i_s = ar.add(states, nullptr, (size_t)count * P->n);
+  const int i_o = ar.add(nullptr, out, (size_t)count * sizeof(double));
+  const int i_x = ar.add(nullptr, nullptr, pysa::energy_scratch_bytes(P->n, count));
+  HIP_TRY(ar.up(st));
+  const int8_t* dS = ar.at<const int8_t>(i_s);
+  double *dO = ar.at<double>(i_o), *dX = ar.at<double>(i_x);
+  hipError_t le =
+      P->dtype == 0
+          ? pysa::launch_energy_f64<float>((const float*)P->dJt, (const float*)P->dh, dS, dO, P->n,
+                                           count, dX, st)
+          : pysa::launch_energy_f64<double>((const double*)P->dJt, (const double*)P->dh, dS, dO, P->n,
+                                            count, dX, st);
+  if (le != hipSuccess) {
+    (void)hipStreamSynchronize(st);
+    return fail(PYSA_AMD_EHIP, std::string("energy launch: ") + hipGetErrorString(le));
+  }
+  HIP_TRY(ar.down(st));
   return 0;
 }
 

@@ -105,9 +105,23 @@ class Solver(object):
         e = self._problem(dt).energy(self._spins(np.asarray(conf).astype(dt))[None, :])[0]
         return dt.type(e)
 
-    def _energies(self, states, dtype):
+    def _energies(self, states, dtype, spins=False):
+        """Energies of float states, or (spins) of states in the engine's
+        encoding, as get_energy gives them one by one."""
         dt = np.dtype(dtype)
-        return self._problem(dt).energy(self._spins(states)).astype(dt)
+        return self._problem(dt).energy(states if spins else self._spins(states)).astype(dt)
+
+    def _random_spins(self, states):
+        """Random states into the last axis' rows, from the global NumPy RNG: the
+        draws and their order are those of one np.random.randint(2) call per
+        read (pysa/sa.py:213-243), whose values one larger call repeats."""
+        flat = states.reshape(-1)
+        step = 1 << 20  # draws are 64-bit: 8 MB at a time
+        for k in range(0, flat.size, step):
+            flat[k:k + step] = np.random.randint(2, size=min(step, flat.size - k))
+        if self.problem_type == 'ising':
+            flat *= 2
+            flat -= 1
 
     def metropolis_update_async(self, **kwargs):
         kwargs['send_background'] = False
@@ -166,11 +180,8 @@ class Solver(object):
         betas = self._ladder(num_replicas, temps, min_temp, max_temp, beta0)
         num_replicas = len(betas)
         ft = np.dtype(self.float_type)
-        couplings = self.couplings.astype(self.float_type)
-        local_fields = self.local_fields.astype(self.float_type)
 
-        init = self._init_strategy(initialize_strategy, init_energies, num_replicas, couplings,
-                                   local_fields)
+        init = self._init_strategy(initialize_strategy, init_energies, num_replicas)
         if update_strategy not in ('random', 'sequential', 'block_random'):
             raise ValueError(f"update_strategy='{update_strategy}' not recognized.")
         if int(num_sweeps) < 1:
@@ -191,11 +202,15 @@ class Solver(object):
         R, N = num_replicas, self.n_vars
         t0 = time()
         states = np.empty((num_reads, R, N), dtype=np.int8)
-        energies = np.empty((num_reads, R), dtype=ft)
-        for r in range(num_reads):
-            s, e = init()
-            states[r] = self._spins(s)
-            energies[r] = e
+        if init is None:  # random: spins straight into the engine's encoding
+            self._random_spins(states)
+            energies = self._energies(states.reshape(-1, N), ft, spins=True).reshape(num_reads, R)
+        else:
+            energies = np.empty((num_reads, R), dtype=ft)
+            for r in range(num_reads):
+                s, e = init()
+                states[r] = self._spins(s)
+                energies[r] = e
         init_time = (time() - t0) / num_reads
 
         form_code, order = self._resolve_form(form, update_strategy, ft, R, replay)
@@ -263,15 +278,20 @@ class Solver(object):
                 'updates_per_s': upd / (kms.value * 1e-3) if kms.value > 0 else float('nan'),
             })
 
+        if recompute_energy:  # pysa/sa.py:372-377, original problem dtype
+            dt = self.couplings.dtype
+            energies64 = self._energies(states.reshape(-1, N), dt, spins=True).reshape(num_reads, R)
+            best64 = self._energies(best_state, dt, spins=True)
+
         def _read_result(r):
             out_states = states[r].astype(ft)
             out_energies = energies[r].copy()
             bstate = best_state[r].astype(ft)
             benergy = best_energy[r]
             out_beta_idx = beta_idx[r]
-            if recompute_energy:  # pysa/sa.py:372-377, original problem dtype
-                benergy = self.get_energy(bstate)
-                out_energies = np.array([self.get_energy(s) for s in out_states])
+            if recompute_energy:
+                benergy = best64[r]
+                out_energies = energies64[r].copy()
             if sort_output_temps:  # pysa/sa.py:380-387
                 out_betas = betas
                 out_states = out_states[out_beta_idx]
@@ -332,28 +352,24 @@ class Solver(object):
             betas = 1 / np.array(temps, dtype=self.float_type)
         return np.asarray(betas).astype(self.float_type)
 
-    def _init_strategy(self, initialize_strategy, init_energies, num_replicas, couplings,
-                       local_fields):
-        """Per-read initial states and energies (pysa/sa.py:213-313)."""
+    def _init_strategy(self, initialize_strategy, init_energies, num_replicas):
+        """Per-read initial states and energies (pysa/sa.py:213-313); None for
+        random ones (_random_spins)."""
         ft = self.float_type
         n = self.n_vars
         if type(initialize_strategy) == str:
             if initialize_strategy == 'random':
-                if self.problem_type == 'qubo':
-                    def _init():
-                        states = np.random.randint(2, size=(num_replicas, n)).astype(ft)
-                        return states, self._energies(states, ft)
-                elif self.problem_type == 'ising':
-                    def _init():
-                        states = 2 * np.random.randint(2, size=(num_replicas, n)).astype(ft) - 1
-                        return states, self._energies(states, ft)
-                else:
+                if self.problem_type not in ('qubo', 'ising'):
                     raise ValueError(f"self.problem_type=='{self.problem_type}' not supported.")
+                return None
             elif initialize_strategy == 'zeros' and self.problem_type == 'qubo':
                 def _init():
                     return (np.zeros((num_replicas, n), dtype=ft),
                             np.zeros(num_replicas, dtype=ft))
             elif initialize_strategy == 'ones':
+                couplings = self.couplings.astype(ft)
+                local_fields = self.local_fields.astype(ft)
+
                 def _init():
                     states = np.ones((num_replicas, n), dtype=ft)
                     energies = np.ones(num_replicas, dtype=ft) * (np.sum(couplings) / 2 +
@@ -446,14 +462,10 @@ class Solver(object):
         order (as in metropolis_update)."""
         if reference_prob == "uniform":
             logZ0 = _ais.uniform_partition_fun(self.n_vars)
-            initialize_prob = _ais.uniform_prob_initialization
-            initial_args = None
             ref_code, p = 0, 0.5
         elif reference_prob == "bernoulli":
             logZ0 = _ais.bernoulli_partition_fun(self.n_vars)
-            initialize_prob = _ais.bernoulli_prob_initialization
-            initial_args = reference_args
-            ref_code, p = 1, float(initial_args[0])
+            ref_code, p = 1, float(reference_args[0])
         else:
             raise ValueError("Reference Probability not recognized.")
         if update_strategy == 'random':
@@ -469,16 +481,18 @@ class Solver(object):
 
         ft = np.dtype(self.float_type)
         temps = np.array([(i + 1) / (num_temps) for i in range(num_temps)], dtype=self.float_type)
-        couplings = beta * self.couplings.astype(self.float_type)
-        local_fields = beta * self.local_fields.astype(self.float_type)
 
-        initial_states = []
-        for _ in range(num_samps):
-            initial_states += [
-                initialize_prob(self.n_vars, self.problem_type, initial_args).astype(self.float_type)
-            ]
-        initial_states = np.array(initial_states)
-        spins = np.ascontiguousarray(self._spins(initial_states))
+        # the initial states (pysa/ais.py:137-149, :175-195), drawn chain after
+        # chain as uniform_/bernoulli_prob_initialization would, in one array
+        spins = np.empty((num_samps, self.n_vars), dtype=np.int8)
+        if ref_code == 0:
+            self._random_spins(spins)
+        else:
+            for k in range(num_samps):
+                spins[k] = np.random.binomial(1, 1 - reference_args[0], size=self.n_vars)
+            if self.problem_type == 'ising':
+                spins *= 2
+                spins -= 1
         rep_lr = rep_perm = None
         if replay is not None:
             rep_lr = np.ascontiguousarray(replay['log_r'], dtype=np.float64)
@@ -503,7 +517,8 @@ class Solver(object):
         if mfma and order == _lib.ORDER['random']:
             order = _lib.ORDER['block_random']
 
-        prob = _lib.Problem(np.asarray(couplings, dtype=ft), np.asarray(local_fields, dtype=ft),
+        prob = _lib.Problem(np.asarray(beta * self.couplings.astype(self.float_type), dtype=ft),
+                            np.asarray(beta * self.local_fields.astype(self.float_type), dtype=ft),
                             self.problem_type, ft)
         log_omegas = np.empty(num_samps, dtype=np.float64)
         kms = _lib._c_dbl(0.0)
@@ -522,6 +537,6 @@ class Solver(object):
         samples = spins.astype(ft)
         logZf = _ais.omegas_to_partition(np.array(log_omegas), logZ0)
         lomax = log_omegas.max()
-        normalization = np.sum(np.exp(log_omegas - lomax))
-        omegas = [np.exp(log_omegas[i] - lomax) / normalization for i in range(num_samps)]
+        weights = np.exp(log_omegas - lomax)
+        omegas = list(weights / np.sum(weights))
         return logZf, samples, omegas
