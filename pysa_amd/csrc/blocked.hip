@@ -207,16 +207,8 @@ __global__ __launch_bounds__(64 * KW) void blocked_pt_kernel(BParams p) {
   for (int j = 0; j < kb; ++j) {
     const int c = c0 + j;
     if (c >= nblk) break;
-    uint32_t va = 0, vb = 0;
-#pragma unroll
-    for (int b = 0; b < 16; ++b) {
-      const int rel = I8 ? (16 * h + b) : ((b < 8) ? (8 * h + b) : (16 + 8 * h + (b - 8)));
-      const int pos = 32 * c + rel;
-      if (pos < n) {
-        if (acta && p.spins[base_a + pos] == 1) va |= 1u << b;
-        if (actb && p.spins[base_b + pos] == 1) vb |= 1u << b;
-      }
-    }
+    const uint32_t va = acta ? load_half<I8>(p.spins + base_a, c, h, n) : 0u;
+    const uint32_t vb = actb ? load_half<I8>(p.spins + base_b, c, h, n) : 0u;
     set_half<NW>(sa, j, va);
     set_half<NW>(sb, j, vb);
   }
@@ -551,18 +543,12 @@ __global__ __launch_bounds__(64 * KW) void blocked_pt_kernel(BParams p) {
   }
 }
 
-// Final argmin over per-replica bests (simulation.py:174-177), one thread per read.
-__global__ void best_argmin_kernel(BParams p) {
-  const int read = blockIdx.x * blockDim.x + threadIdx.x;
-  if (read >= p.reads) return;
-  const int R = p.R;
-  int bp = 0;
-  for (int k = 1; k < R; ++k)
-    if (p.best_rep_e[(size_t)read * R + k] < p.best_rep_e[(size_t)read * R + bp]) bp = k;
-  p.best_energy[read] = p.best_rep_e[(size_t)read * R + bp];
-  p.best_sweeps[read] = p.best_rep_sw[(size_t)read * R + bp];
-  const int8_t* src = p.best_rep + ((size_t)read * R + bp) * p.n;
-  for (int i = 0; i < p.n; ++i) p.best_state[(size_t)read * p.n + i] = src[i];
+// Each read's best over its replicas' bests, one wave per read (128 reads of
+// 32 replicas of 512 spins: 4.2 us; 100 us with a thread per read).
+__global__ __launch_bounds__(64) void best_argmin_kernel(BParams p) {
+  const size_t read = blockIdx.x, c0 = read * p.R;
+  take_best(p.R, p.n, p.best_rep_e + c0, p.best_rep_sw + c0, p.best_rep + c0 * p.n,
+            p.best_energy + read, p.best_sweeps + read, p.best_state + read * p.n);
 }
 
 template <int NP, bool I8, int KW>
@@ -946,7 +932,7 @@ hipError_t launch_blocked(const BlockedProblem& b, const BlockedPlan& pl, const 
   else
     e = launch_np<3, false>(p, pl.nw, pl.kw, pl.groups, st);
   if (e == hipSuccess && best_sem == 0) {
-    hipLaunchKernelGGL(best_argmin_kernel, dim3((reads + 63) / 64), dim3(64), 0, st, p);
+    hipLaunchKernelGGL(best_argmin_kernel, dim3(reads), dim3(64), 0, st, p);
     e = hipGetLastError();
   }
   return e;

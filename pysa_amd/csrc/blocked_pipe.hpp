@@ -17,9 +17,11 @@ namespace blk {
 // each and every tile, compute the next block's fields over every K block
 // except c (whose spins are changing) while the proposal waves sweep block c:
 //     P_{c+1} = sum_{b != c} J[c+1, b] . S_b
-// When a proposal wave is done with block c it adds the missing product
-// J[c+1, c] . S_c itself (one K block), so the fields of block c+1 are ready
-// at the block's barrier.  The rows of every fragment are loaded in the visit
+// The missing product J[c+1, c] . S_c (one K block) a proposal wave takes itself
+// at the start of block c+1, behind its reads of the partials and brackets,
+// whose latency it covers (behind the chain of block c, before the barrier:
+// 41.4 instead of 40.8 us a sweep at n = 512, 113.7 instead of 112.5 with two
+// tiles at n = 1024).  The rows of every fragment are loaded in the visit
 // order of their block (row k ^ mask at place k: an XOR of the lane's address),
 // so the fields come out in visit order and nothing is permuted afterwards.
 // The helper waves stage the next blocks' J block, h and row sums and compute
@@ -98,12 +100,15 @@ struct __align__(16) PipeLds {
   float E[64];
   float rb[64];
   float bet[64];  // the ladder by slot (batched: tile t's instance's at 32 t)
-  float Es[64];   // energy of the replica in each slot, before the exchanges
-  int bso[64];    // its ascending order (log-omega)
+  // by slot a (the exchange with slot a - 1): the energy of the replica in slot
+  // a - 1, beta[a] - beta[a - 1], the exchange's log-uniform
+  // (behind four entries that are only read ahead)
+  float4 wl[4 + 64];
+  int bso[64];    // the ladder's ascending order (log-omega)
   int bi[64];
   int flag[64];
   int src[64];
-  float lu[64];  // by pair: the least float above the log-uniform of its exchange
+  float lu[64];  // by slot a: the least float above the log-uniform of its exchange with a - 1
 };
 
 // BR: block-random visit order (schedule tables in LDS); otherwise blocks are
@@ -233,13 +238,8 @@ __global__ __launch_bounds__(128 * (MW + 1)) void blocked_pipe_kernel(BParams p0
     sa[tt].w = 0;
     for (int j = 0; j < jn; ++j) {
       const int c = c0 + j;
-      uint32_t va = 0;
-#pragma unroll
-      for (int b = 0; b < 16; ++b) {
-        const int rel = I8 ? (16 * h + b) : ((b < 8) ? (8 * h + b) : (16 + 8 * h + (b - 8)));
-        const int pos = 32 * c + rel;
-        if (pos < n_of(tt) && actt[tt] && p.spins[base_t[tt] + pos] == 1) va |= 1u << b;
-      }
+      const uint32_t va =
+          actt[tt] ? load_half<I8>(p.spins + base_t[tt], c, h, n_of(tt)) : 0u;
       set_half<NW>(sa[tt], j, va);
     }
   }
@@ -661,17 +661,23 @@ __global__ __launch_bounds__(128 * (MW + 1)) void blocked_pipe_kernel(BParams p0
   // its own state in registers); all pass the same barriers: one after the
   // block's work (B), and at the end of a pass one more (three after a sweep).
   if (pw) {
-    // schedule entries of the current step, each read one block ahead
-    const uint32_t e0 = sched_entry(0, 0);
-    int c_nx = entry_block(e0);
-    uint32_t xm_nx = entry_mask(e0);
+    // schedule entries of this step and the next; the one after is read each
+    // block and made wave-uniform at the block's end
+    const uint32_t e0 = sched_entry(0, 0), e1 = sched_entry(0, 1);
+    int c = entry_block(e0), c1 = entry_block(e1);
+    uint32_t xm = entry_mask(e0), xm1 = entry_mask(e1);
     const int tw = w == 0 ? 0 : NT - 1;    // the wave's tile
     const int ti = BAT ? tw : 0;           // its instance
     const int qp = 32 * tw + (lane & 31);  // the lane's replica of the group
     const int np = n_of(ti);
-    float corr[16];  // J[c, c_prev] . S of the block before
+    // the block before: its fragments of J[c, c_prev] and its final spins (block
+    // rows); their product, the correction, is taken while the partials are read
+    FragSet fcorr;
 #pragma unroll
-    for (int v = 0; v < 16; ++v) corr[v] = 0.f;
+    for (int st = 0; st < NST; ++st)
+#pragma unroll
+      for (int pc = 0; pc < NP; ++pc) fcorr[st][pc] = Frag{};
+    uint32_t mbr = 0;
     for (int ps = 0; ps < npass; ++ps) {
       int s;
       const bool dry = pass_info(ps, s);
@@ -682,34 +688,50 @@ __global__ __launch_bounds__(128 * (MW + 1)) void blocked_pipe_kernel(BParams p0
       for (int tb = 0; tb < nblk; ++tb, ++t) {
         const int pb = t & 1;
         // block c of this step, its visit k being block row k ^ xm; c1 the next
-        const int c = c_nx;
-        const uint32_t xm = xm_nx;
         const int pos0 = 32 * c;
         const bool lastb = tb + 1 == nblk;
-        const uint32_t e1 = sched_entry(lastb ? sp ^ 1 : sp, lastb ? 0 : tb + 1);
-        const int c1 = entry_block(e1);
-        xm_nx = entry_mask(e1);
-        c_nx = c1;
-        FragSet fcorr;
-        load_corr_frags(c1, c, lane ^ (int)xm_nx, ti, fcorr);
+        const int p2 = tb + 2 < nblk ? sp : sp ^ 1, i2 = tb + 2 < nblk ? tb + 2 : tb + 2 - nblk;
+        const uint32_t raw2 = BR ? (uint32_t)*(volatile uint16_t*)&L.sch[p2][i2] : (uint32_t)i2;
         // the spins of the block's visits, in either half of the wave
         uint32_t mb = L.bb[pb][qp];
+        // the partial fields and the brackets of the lane's visits (slot 4 m + e
+        // is visit 8 m + 4 h + e)
+        float hib[16], lob[16];
+        float4 x[4][MW];
+#pragma unroll
+        for (int g4 = 0; g4 < 4; ++g4)
+#pragma unroll
+          for (int mm = 0; mm < MW; ++mm) x[g4][mm] = L.part[pb][mm][tw][g4][lane];
+#pragma unroll
+        for (int g4 = 0; g4 < 4; ++g4) {
+          const float4 a = *reinterpret_cast<const float4*>(&L.hi[pb][qp][8 * g4 + 4 * h]);
+          const float4 b = *reinterpret_cast<const float4*>(&L.lo[pb][qp][8 * g4 + 4 * h]);
+          hib[4 * g4] = a.x, hib[4 * g4 + 1] = a.y, hib[4 * g4 + 2] = a.z, hib[4 * g4 + 3] = a.w;
+          lob[4 * g4] = b.x, lob[4 * g4 + 1] = b.y, lob[4 * g4 + 2] = b.z, lob[4 * g4 + 3] = b.w;
+        }
+        __builtin_amdgcn_sched_barrier(0);  // the reads first: the product covers their latency
+        float corr[16];
+        {
+          f32x16 a = {};
+          i32x16 ia = {};
+          mfma_step(fcorr, half_of<I8>(mbr, h), a, ia);
+#pragma unroll
+          for (int v = 0; v < 16; ++v) corr[v] = I8 ? (float)ia[v] : a[v];
+        }
+        load_corr_frags(c1, c, lane ^ (int)xm1, ti, fcorr);
         if (dry) {
           // ---- dry pass: f64 energy of the block's rows from its full fields
           // (a dry pass visits every block with mask 0: visits are rows), the
           // rows' terms added in order, passed between the lane halves
           static_for<kB / 4>([&](auto gc) __attribute__((always_inline)) {
             constexpr int gr = decltype(gc)::value, g4 = gr >> 1;
-            float4 x[MW];
-#pragma unroll
-            for (int mm = 0; mm < MW; ++mm) x[mm] = L.part[pb][mm][tw][g4][lane];
             for (int e = 0; e < 4; ++e) {
               const int i = 4 * gr + e;
               if (pos0 + i < np) {
                 auto el = [&](const float4& y) { return e == 0 ? y.x : e == 1 ? y.y : e == 2 ? y.z : y.w; };
-                double f = (double)el(x[0]);
+                double f = (double)el(x[g4][0]);
 #pragma unroll
-                for (int mm = 1; mm < MW; ++mm) f += (double)el(x[mm]);
+                for (int mm = 1; mm < MW; ++mm) f += (double)el(x[g4][mm]);
                 f += (double)(e == 0   ? corr[4 * g4]
                               : e == 1 ? corr[4 * g4 + 1]
                               : e == 2 ? corr[4 * g4 + 2]
@@ -723,29 +745,13 @@ __global__ __launch_bounds__(128 * (MW + 1)) void blocked_pipe_kernel(BParams p0
             eacc = half_bcast<gr & 1>(eacc);
           });
         } else {
-          // ---- proposals of block c: slot j = 4 m + e of a lane is visit
-          // 8 m + 4 h + e
-          // brackets of the lane's visits, read first (their latency overlaps
-          // the field sums and they leave the chain free of LDS waits)
-          float hib[16], lob[16];
-#pragma unroll
-          for (int g4 = 0; g4 < 4; ++g4) {
-            const float4 a = *reinterpret_cast<const float4*>(&L.hi[pb][qp][8 * g4 + 4 * h]);
-            const float4 b = *reinterpret_cast<const float4*>(&L.lo[pb][qp][8 * g4 + 4 * h]);
-            hib[4 * g4] = a.x, hib[4 * g4 + 1] = a.y, hib[4 * g4 + 2] = a.z, hib[4 * g4 + 3] = a.w;
-            lob[4 * g4] = b.x, lob[4 * g4 + 1] = b.y, lob[4 * g4 + 2] = b.z, lob[4 * g4 + 3] = b.w;
-          }
+          // ---- proposals of block c
           // fields: the partials in order, the correction, (QUBO with bf16
           // operands) the row sums, then h (batched: the integer counts, with
           // h in hk)
           f32x16 fp;
           float hk[16];
           {
-            float4 x[4][MW];
-#pragma unroll
-            for (int g4 = 0; g4 < 4; ++g4)
-#pragma unroll
-              for (int mm = 0; mm < MW; ++mm) x[g4][mm] = L.part[pb][mm][tw][g4][lane];
 #pragma unroll
             for (int g4 = 0; g4 < 4; ++g4) {
               float4 sm = x[g4][0];
@@ -989,20 +995,17 @@ __global__ __launch_bounds__(128 * (MW + 1)) void blocked_pipe_kernel(BParams p0
           if constexpr (!BAT) dsum += (double)dpart;
           nacc += (uint32_t)__builtin_popcount(mb ^ mb0);
         }
-        {
-          const uint32_t mbr = BR ? xor_permute_bits(mb, xm) : mb;  // back to block-row order
-          if (lane < 32) {
-            L.bnew[pb][qp] = mbr;
-            // the same block next (at a pass boundary): its spins are these,
-            // in its next visit order (the owners, whose copy is older, skip it)
-            if (c1 == c) L.bb[pb ^ 1][qp] = BR ? xor_permute_bits(mbr, xm_nx) : mbr;
-          }
-          f32x16 a = {};
-          i32x16 ia = {};
-          mfma_step(fcorr, half_of<I8>(mbr, h), a, ia);
-#pragma unroll
-          for (int v = 0; v < 16; ++v) corr[v] = I8 ? (float)ia[v] : a[v];
+        mbr = BR ? xor_permute_bits(mb, xm) : mb;  // back to block-row order
+        if (lane < 32) {
+          L.bnew[pb][qp] = mbr;
+          // the same block next (at a pass boundary): its spins are these, in
+          // its next visit order (the owners, whose copy is older, skip it)
+          if (c1 == c) L.bb[pb ^ 1][qp] = BR ? xor_permute_bits(mbr, xm1) : mbr;
         }
+        // the next step's block and the one after it
+        c = c1, xm = xm1;
+        const uint32_t e2 = BR ? (uint32_t)__builtin_amdgcn_readfirstlane((int)raw2) : raw2;
+        c1 = entry_block(e2), xm1 = entry_mask(e2);
         if (lastb && lane < 32) {
           L.ds[qp] = dry ? eacc : dsum;
           L.nacc[qp] = nacc;
@@ -1083,65 +1086,80 @@ __global__ __launch_bounds__(128 * (MW + 1)) void blocked_pipe_kernel(BParams p0
           const int b0 = BAT ? 32 * tx + ((qx & 31) / R) * R : (qx / R) * R;  // the read's first lane
           const int slot = qx - b0;
           const float* bet = &L.bet[32 * tx];
-          if (act) L.Es[qx] = L.E[b0 + L.bi[qx]];
-          if (act && rr == 0) {  // read leader
+          int occ = L.bi[qx];  // the replica in the lane's slot
+          if (p.best_sem == 1 && act && rr == 0) {  // simulation.py:222-225 in replica order
             int src = -1;
-            if (p.best_sem == 1) {  // simulation.py:222-225 in replica order
-              float cur = gE;
-              float en = L.E[b0];
-              for (int k = 0; k < R; ++k) {
-                const float ek = en;
-                if (k + 1 < R) en = L.E[b0 + k + 1];  // the next one, read ahead
-                if (ek < cur) {
-                  cur = ek;
-                  src = k;
-                }
-              }
-              if (src >= 0) {
-                gE = cur;
-                gsw = s;
-                gimp = 1;
+            float cur = gE;
+            float en = L.E[b0];
+            for (int k = 0; k < R; ++k) {
+              const float ek = en;
+              if (k + 1 < R) en = L.E[b0 + k + 1];  // the next one, read ahead
+              if (ek < cur) {
+                cur = ek;
+                src = k;
               }
             }
-            if (p.use_pt && R > 1) {  // utils.py:44-58
-              // Hot end first: slot a = R-k-1 holds the carried replica (the one
-              // the previous pair left there), slot b = a-1 still its occupant
-              // from before the walk.  An exchange moves the carried replica on
-              // to b; otherwise b's occupant becomes the carried one.  Every
-              // operand but the carried one is read one step ahead.
-              int carry = L.bi[b0 + R - 1];
-              float ec = L.Es[b0 + R - 1], ba = bet[R - 1];
-              int rbn = L.bi[b0 + R - 2];
-              float ebn = L.Es[b0 + R - 2], bbn = bet[R - 2];
-              float lun = L.lu[b0];
-              for (int k = 0; k < R - 1; ++k) {
-                const int a = R - k - 1, b = a - 1;
-                const int rb = rbn;
-                const float eb = ebn, bb = bbn;
-                const float luk = lun;
-                if (b > 0) {
-                  rbn = L.bi[b0 + b - 1];
-                  ebn = L.Es[b0 + b - 1];
-                  bbn = bet[b - 1];
-                  lun = L.lu[b0 + k + 1];
-                }
-                const float dd = (ec - eb) * (ba - bb);
-                const bool x = dd >= luk;  // dd >= 0 or log u < dd (log u < 0)
-                L.bi[b0 + a] = x ? rb : carry;
-                if (!x) {
-                  carry = rb;
-                  ec = eb;
-                }
-                ba = bb;
-              }
-              L.bi[b0] = carry;
+            if (src >= 0) {
+              gE = cur;
+              gsw = s;
+              gimp = 1;
             }
             L.src[g] = src;
           }
-          // every slot's new beta to the replica now in it (after the
-          // leader's exchanges: the same wave, in order)
-          if (act) L.rb[b0 + L.bi[qx]] = bet[slot];
+          if (p.use_pt && R > 1) {  // utils.py:44-58
+            // Hot end first: at slot a the carried replica (at first slot R - 1's)
+            // meets the occupant of slot a - 1 from before the walk; exchanged,
+            // it is carried on to a - 1, otherwise it stays in a and that
+            // occupant becomes the carried one.  Which replica is carried at a
+            // slot is serial, but not how far each would be carried if it
+            // were: every lane walks its slot's replica to where it would
+            // stay (to), four slots at a time, and then the carried ones are
+            // read off from the hot end, S = slots where one is picked up (a
+            // read's last one leads on to the read below it; idle lanes stay
+            // where they are).  R = 32: 6.6 -> 2.3 k cycles a sweep (one lane
+            // per read walking all slots before).
+            const int below = L.bi[max(qx - 1, 0)];  // of the slot below
+            const float es = L.E[b0 + occ];
+            // (a read's last slot and idle lanes: no exchange)
+            L.wl[4 + qx] = make_float4(L.E[b0 + below], bet[slot] - bet[max(slot - 1, 0)],
+                                       act && slot > 0 ? L.lu[qx] : __builtin_nanf(""), 0.f);
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            int to = qx;
+            uint64_t go = ~0ull;  // lanes still carried, kept as a mask: no branches inside
+            do {
+              float4 y[4];
+#pragma unroll
+              for (int i = 0; i < 4; ++i) y[i] = L.wl[4 + to - i];
+              int d = 0;
+#pragma unroll
+              for (int i = 0; i < 4; ++i) {
+                const float dd = (es - y[i].x) * y[i].y;
+                go &= __builtin_amdgcn_ballot_w64(dd >= y[i].z);  // dd >= 0 or log u < dd (log u < 0)
+                uint64_t co;
+                asm("v_addc_co_u32_e64 %0, %1, 0, %2, %3" : "=v"(d), "=s"(co) : "v"(d), "s"(go));
+                (void)co;
+              }
+              to -= d;
+            } while (go != 0);
+            // S starts as every slot; a replica carried down takes out the ones
+            // it passes
+            uint64_t S = ~0ull, mv = __builtin_amdgcn_ballot_w64(to != qx);
+            while (mv != 0) {
+              const int c = 63 - __builtin_clzll(mv), d = __builtin_amdgcn_readlane(to, c);
+              S &= ~((1ull << c) - (1ull << d));
+              mv &= (1ull << d) - 1ull;
+            }
+            // the slot below one that is picked up (or below none) ends a walk
+            const bool end = qx == 0 || ((S >> (qx - 1)) & 1ull) != 0;
+            const int from = L.bi[qx + (int)__builtin_ctzll(S >> qx)];
+            occ = end ? from : below;
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            if (act) L.bi[qx] = occ;
+          }
+          // every slot's new beta to the replica now in it
+          if (act) L.rb[b0 + occ] = bet[slot];
           if (p.logw && p.log_omegas) {  // ais.py:99-112 over the ascending ladder
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
             // lane r: its term, then the leader adds them in order
             if (act && slot > 0) {
               const int k = L.bso[slot];
@@ -1216,7 +1234,7 @@ __global__ __launch_bounds__(128 * (MW + 1)) void blocked_pipe_kernel(BParams p0
           // the sweep's exchange uniforms (utils.py:57), by a helper that has
           // no brackets to compute during the last block
           if (w == 7 && last && !dry && p.use_pt && act && rr < R - 1)
-            L.lu[q] = float_above(log_u32(pick_word(
+            L.lu[q + R - 1 - 2 * rr] = float_above(log_u32(pick_word(  // pair rr: slot R - 1 - rr
                 pt_block((uint64_t)read, sw, (uint32_t)rr, p.k0, p.k1), (uint32_t)rr & 3u)));
         }
         __syncthreads();  // B

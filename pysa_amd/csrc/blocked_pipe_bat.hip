@@ -46,25 +46,19 @@ __global__ void pack_i8_batched_kernel(const int8_t* __restrict__ signs,
   *reinterpret_cast<int4*>(out + t.frag + gid * 16) = v;
 }
 
-// Per-read minimum over the replicas' bests (simulation.py:174-177, first
-// minimum wins), one thread per read slot of a workgroup's tiles.
-__global__ void bat_best_argmin_kernel(BParams p, int groups) {
-  const int gw = blockIdx.x * blockDim.x + threadIdx.x;
+// Each read's best over its replicas' bests, one wave per read slot of a
+// workgroup's tiles.
+__global__ __launch_bounds__(64) void bat_best_argmin_kernel(BParams p) {
+  const int gw = blockIdx.x;
   const int per = 2 * p.rpw;
   const int wg = gw / per, tt = (gw - wg * per) / p.rpw, j = gw - wg * per - tt * p.rpw;
-  if (wg >= groups) return;
   const BatTile& b = p.bat[wg].t[tt];
   const int read = b.read0 + j;
   if (read >= b.read_end) return;
-  const int R = p.R, n = b.n;
-  int bp = 0;
-  for (int k = 1; k < R; ++k)
-    if (p.best_rep_e[(size_t)read * R + k] < p.best_rep_e[(size_t)read * R + bp]) bp = k;
-  p.best_energy[read] = p.best_rep_e[(size_t)read * R + bp];
-  p.best_sweeps[read] = p.best_rep_sw[(size_t)read * R + bp];
-  const int8_t* src = p.best_rep + (b.spin_adj + ((int64_t)read * R + bp) * n);
-  int8_t* dst = p.best_state + (b.best_adj + (int64_t)read * n);
-  for (int i = 0; i < n; ++i) dst[i] = src[i];
+  const size_t c0 = (size_t)read * p.R;
+  take_best(p.R, b.n, p.best_rep_e + c0, p.best_rep_sw + c0,
+            p.best_rep + (b.spin_adj + (int64_t)c0 * b.n), p.best_energy + read,
+            p.best_sweeps + read, p.best_state + (b.best_adj + (int64_t)read * b.n));
 }
 
 }  // namespace
@@ -83,9 +77,8 @@ hipError_t pack_batched_frags(const int8_t* signs, const BatPack* tab, int count
 }
 
 hipError_t bat_best_argmin(const BParams& p, int groups, hipStream_t st) {
-  const long long threads = (long long)groups * 2 * p.rpw;
-  hipLaunchKernelGGL(bat_best_argmin_kernel, dim3((unsigned)((threads + 63) / 64)), dim3(64), 0, st,
-                     p, groups);
+  hipLaunchKernelGGL(bat_best_argmin_kernel, dim3((unsigned)groups * 2u * (unsigned)p.rpw), dim3(64),
+                     0, st, p);
   return hipGetLastError();
 }
 
