@@ -223,7 +223,7 @@ int pysa_amd_plain_fields(int64_t handle, int64_t count, void* out);
  * Launch shape of the MFMA form on this problem, for the autotuner
  * (pysa_amd/tune.py).  No counterpart in the reference, whose numba loop has
  * no launch shape.  Results do not depend on the shape, only the speed.
- *   kernel  0 = by size (the pipelined kernel from three 32-spin blocks up),
+ *   kernel  0 = by size (the pipelined kernel from two 32-spin blocks up),
  *           1 = pipelined, 2 = split-K (the block-random order always runs
  *           the pipelined kernel)
  *   tiles   replicas per workgroup of the pipelined kernel in tiles of 32:

@@ -9,8 +9,9 @@ whole sweep loop (sweeps, exchanges, best tracking) runs in one persistent
 launch, so there is no sweeps-per-graph count either.  What the tuner
 chooses is how a batch is laid on the device:
 
-  kernel  the pipelined kernel (proposal wave, three matrix waves, four
-          helper waves) or the split-K kernel (sequential order only);
+  kernel  the pipelined kernel (a proposal wave per tile, three matrix waves,
+          the rest helpers; two blocks of spins or more) or the split-K kernel
+          (sequential order only);
   tiles   replicas per workgroup of the pipelined kernel, one or two tiles
           of 32: two tiles share each coupling fragment between 64 replicas,
           one tile doubles the workgroups when a batch would leave compute
@@ -24,8 +25,8 @@ every valid shape on the caller's problem and batch size (random spins, a
 few sweeps, device time of the engine call, best of two), keeps the fastest
 and stores it in a JSON cache: $PYSA_AMD_TUNE_CACHE, else
 ~/.cache/pysa_amd/tune.json.  PYSA_AMD_TUNE=0 skips tuning and leaves the
-library's occupancy rule (one tile when two-tile workgroups would leave
-compute units idle).
+library's rule (two tiles once one-tile workgroups would take more rounds
+over the compute units than they save).
 """
 
 import json
