@@ -586,8 +586,9 @@ void blocked_release(BlockedProblem& b) {
 }
 
 bool blocked_eligible(int n, int dtype, int R, int reads, int order, bool replay) {
-  // the block-random order runs on the pipelined kernel (at least 3 blocks)
-  const bool ord_ok = order == kSequential || (order == kBlockRandom && n > 2 * kB);
+  // the block-random order runs on the pipelined kernel alone
+  const bool ord_ok = order == kSequential ||
+                      (order == kBlockRandom && pipe_takes(order, (n + kB - 1) / kB));
   return dtype == 0 && n >= 32 && n <= kBlockedMaxN && R >= 1 && R <= 64 && reads >= 1 &&
          ord_ok && !replay;
 }
@@ -717,7 +718,7 @@ BlockedPlan plan_blocked(const BlockedProblem& b, int n, int reads, int R, int o
   pl.groups = (reads + (64 / R) - 1) / (64 / R);
   pl.kw = 1;
   while (pl.kw < 4 && 2 * pl.kw <= pl.nblk && pl.groups * pl.kw < 1024) pl.kw *= 2;
-  // The pipelined kernel takes every problem of two blocks or more;
+  // The pipelined kernel takes every problem it can (pipe_takes);
   // PYSA_AMD_BLOCKED_SPLITK=1 selects the split-K kernel instead (kept for one
   // block and for comparisons).
   static const bool force_splitk = [] {
@@ -727,9 +728,8 @@ BlockedPlan plan_blocked(const BlockedProblem& b, int n, int reads, int R, int o
   // The problem's launch shape (pysa_amd_problem_set_shape) picks the kernel;
   // the split-K kernel has no block-random order.
   const bool want_splitk = force_splitk || b.shape_kernel == 2;
-  // It reads its schedule two steps ahead, across at most one sweep's end, so
-  // it needs two blocks.
-  pl.pipe = order == kBlockRandom || (pl.nblk >= 2 && (b.shape_kernel == 1 || !want_splitk));
+  pl.pipe = order == kBlockRandom ||
+            (pipe_takes(order, pl.nblk) && (b.shape_kernel == 1 || !want_splitk));
   // Tiles of 32 replicas per workgroup of the pipelined kernel (one workgroup
   // per CU either way): the fewer rounds over the device, a one-tile block step
   // taking about 18 / 25 of a two-tile one (n = 1024: 2.7 and 3.8 us).

@@ -129,6 +129,12 @@ __device__ __forceinline__ void set_half(Bits<NW>& s, int c, uint32_t v) {
   s.w[c >> 1] = (s.w[c >> 1] & ~(0xFFFFu << sh)) | ((v & 0xFFFFu) << sh);
 }
 
+// Whether the pipelined kernel runs nblk blocks in this order.  It reads its
+// schedule two steps ahead, across at most one sweep's end: two blocks.  In
+// block-random order the next sweep's schedule is written during step 0 and
+// read from step nblk - 2 on, so that one has to be a later step: three.
+constexpr bool pipe_takes(int order, int nblk) { return nblk >= (order == kBlockRandom ? 3 : 2); }
+
 struct BParams {
   int n, nblk, ptype, R, reads, S, rpw, np, use_pt, logw, best_sem;
   int order;  // kSequential or kBlockRandom (pipelined kernel only)

@@ -161,8 +161,8 @@ __global__ __launch_bounds__(128 * (MW + 1)) void blocked_pipe_kernel(BParams p0
   // the proposals of a tile each; matrix wave w = 1..MW computes the products
   // of K range m = w - 1 for both tiles of 32 replicas (each coupling fragment
   // is loaded once for both); the helper waves stage the next blocks' J block,
-  // h and row sums and compute the acceptance brackets, wave 4 the visit
-  // schedule, wave 7 the exchange uniforms.  Wave 0 also ends the sweeps.
+  // h and row sums and compute the acceptance brackets, wave 7 also the
+  // visit schedule and the exchange uniforms.  Wave 0 also ends the sweeps.
   static_assert(MW == 3, "eight waves: up to two proposal waves, three matrix waves, helpers");
   const bool mw = w >= 1 && w <= MW;                          // a matrix wave
   const bool pw = w == 0 || (NT == 2 && w == kPropWave1);     // a proposal wave
@@ -541,7 +541,7 @@ __global__ __launch_bounds__(128 * (MW + 1)) void blocked_pipe_kernel(BParams p0
     }
   };
 
-  // Visit schedule of sweep counter swn into parity par (wave 4, one lane
+  // Visit schedule of sweep counter swn into parity par (wave 7, one lane
   // per step): the block visited at step t and that block's in-block mask.
   auto fill_sched = [&](int par, uint64_t swn, bool dry) {
     if (lane < nblk) {
@@ -1306,6 +1306,9 @@ __global__ __launch_bounds__(128 * (MW + 1)) void blocked_pipe_kernel(BParams p0
 
 template <int NP, bool I8, bool BR, int NT, int MODE = kModePT>
 hipError_t launch_pipe_o(const BParams& p, int nw, int groups, hipStream_t st) {
+  // (batched: the sizes are checked where the workgroups' table is built)
+  if (MODE != kModeBatched && !pipe_takes(BR ? kBlockRandom : kSequential, p.nblk))
+    return hipErrorInvalidValue;
   dim3 grid(groups), block(128 * (kPipeMW + 1));
   switch (nw) {
     case 4: hipLaunchKernelGGL((blocked_pipe_kernel<NP, I8, 4, kPipeMW, BR, NT, MODE>), grid, block, 0, st, p); break;

@@ -94,6 +94,7 @@ hipError_t BatchedMfmaRun::enqueue(const BatchParams& bp, const std::vector<int>
                                    const int64_t* hs, const int64_t* hh_off, const float* hscale,
                                    hipStream_t st) {
   using namespace blk;
+  static_assert(pipe_takes(kBlockRandom, (kBatchedMfmaMinN + kB - 1) / kB), "schedule of a tile");
   if (inst.empty()) return hipSuccess;
   const int R = bp.R, reads = bp.reads;
   if (R < 1 || R > 32) return hipErrorInvalidValue;

@@ -983,7 +983,7 @@ extern "C" int pysa_amd_batched_device(int32_t count, const int32_t* n, const in
   if (max_n > 1024 && R > 8) return fail(PYSA_AMD_EINVAL, "batched: R <= 8 when an instance has n > 1024");
   // Largest instances first, so the short ones fill the tail of the launch.
   // The MFMA form (BLOCKED / AUTO, sequential or block-random order) takes
-  // the instances of three blocks or more; the plain kernel the others.
+  // the instances of kBatchedMfmaMinN spins or more; the plain kernel the others.
   std::vector<int> idx(count), mf, pl;
   for (int k = 0; k < count; ++k) idx[k] = k;
   std::stable_sort(idx.begin(), idx.end(), [&](int a, int b) { return hn[a] > hn[b]; });

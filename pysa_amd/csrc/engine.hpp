@@ -156,7 +156,8 @@ struct BatPack {
   int n, nblk, ld, pad;
   int64_t sgn, frag;
 };
-// Smallest instance of the batched MFMA form (three blocks, one per matrix wave).
+// Smallest instance of the batched MFMA form: three blocks, the least that the
+// pipelined kernel takes in block-random order.
 constexpr int kBatchedMfmaMinN = 65;
 // Enqueues the instances `inst` (indices into the batch, largest first) of a
 // batch on the pipelined MFMA kernel: packs their couplings, builds the

@@ -1,0 +1,32 @@
+"""Rules of the engine's C++ interior that need no GPU, through a test-only host
+library."""
+
+import ctypes
+import os
+import subprocess
+
+import pytest
+import torch
+
+from pysa_amd import _lib
+
+HERE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "host_probe")
+INVALID_VALUE = 1  # hipErrorInvalidValue
+
+
+@pytest.fixture(scope="module")
+def probe():
+    if torch.cuda.device_count():
+        pytest.skip("a launcher that failed to refuse would launch")
+    subprocess.run(["make", "-s", "-C", HERE], check=True)
+    ctypes.CDLL(_lib.load()._name, mode=ctypes.RTLD_GLOBAL)
+    return ctypes.CDLL(os.path.join(HERE, "_build", "libhost_probe.so"))
+
+
+# The schedule of the next sweep is written and read in one step below three
+# blocks (block-random order); below two, steps are read that do not exist.
+@pytest.mark.parametrize("kind", [0, 1, 2])
+@pytest.mark.parametrize("order,nblk", [(3, 1), (3, 2), (0, 1)])
+@pytest.mark.parametrize("tiles", [1, 2])
+def test_pipelined_launchers_refuse_short_schedules(probe, kind, order, nblk, tiles):
+    assert probe.probe_launch_pipe(kind, order, nblk, tiles) == INVALID_VALUE
