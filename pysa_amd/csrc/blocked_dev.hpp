@@ -135,6 +135,15 @@ __device__ __forceinline__ void set_half(Bits<NW>& s, int c, uint32_t v) {
 // read from step nblk - 2 on, so that one has to be a later step: three.
 constexpr bool pipe_takes(int order, int nblk) { return nblk >= (order == kBlockRandom ? 3 : 2); }
 
+// The exchange walk: the lane of the replica in the slot below, for a lane of the
+// read that starts at lane b0 and `below`, the lane below's entry in the slots'
+// list of replicas.  A slot 0 has no slot below (its value is not used): that
+// entry is another read's, and for the first idle lane behind a full read b0 +
+// below lies past the last lane.
+__host__ __device__ __forceinline__ int lane_below(int b0, int below) {
+  return b0 + below < 63 ? b0 + below : 63;
+}
+
 struct BParams {
   int n, nblk, ptype, R, reads, S, rpw, np, use_pt, logw, best_sem;
   int order;  // kSequential or kBlockRandom (pipelined kernel only)

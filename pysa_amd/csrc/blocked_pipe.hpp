@@ -1123,7 +1123,7 @@ __global__ __launch_bounds__(128 * (MW + 1)) void blocked_pipe_kernel(BParams p0
             const int below = L.bi[max(qx - 1, 0)];  // of the slot below
             const float es = L.E[b0 + occ];
             // (a read's last slot and idle lanes: no exchange)
-            L.wl[4 + qx] = make_float4(L.E[b0 + below], bet[slot] - bet[max(slot - 1, 0)],
+            L.wl[4 + qx] = make_float4(L.E[lane_below(b0, below)], bet[slot] - bet[max(slot - 1, 0)],
                                        act && slot > 0 ? L.lu[qx] : __builtin_nanf(""), 0.f);
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
             int to = qx;

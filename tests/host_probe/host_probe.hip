@@ -25,3 +25,7 @@ extern "C" int probe_launch_pipe(int kind, int order, int nblk, int tiles) {
   if (kind == 1) return launch_pipe_bf16_2(p, 4, tiles, 1, nullptr);
   return launch_pipe_ais_i8(p, 4, tiles, 1, nullptr);
 }
+
+extern "C" int probe_lane_below(int b0, int below) {
+  return pysa::blk::lane_below(b0, below);
+}

@@ -30,3 +30,20 @@ def probe():
 @pytest.mark.parametrize("tiles", [1, 2])
 def test_pipelined_launchers_refuse_short_schedules(probe, kind, order, nblk, tiles):
     assert probe.probe_launch_pipe(kind, order, nblk, tiles) == INVALID_VALUE
+
+
+# (lanes a tile, reads' replicas): 64 lanes with whole reads from lane 0, or two
+# batched tiles of 32 lanes; the lanes behind the last whole read are idle.
+@pytest.mark.parametrize("tile", [32, 64])
+def test_exchange_walk_reads_energies_inside_the_workgroup(probe, tile):
+    for R in range(1, tile + 1):
+        per = tile // R * R  # lanes of whole reads
+        for lane in range(64):
+            t, q = lane // tile * tile, lane % tile
+            b0 = t + q // R * R
+            # the last replica everywhere below but in idle lanes
+            below = R - 1 if max(lane - 1, 0) % tile < per else 0
+            got = probe.probe_lane_below(b0, below)
+            assert 0 <= got < 64
+            if q < per and lane > b0:
+                assert got == b0 + below
