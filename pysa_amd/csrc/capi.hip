@@ -14,8 +14,13 @@
 #include "../../include/pysa_amd.h"
 #include "blocked.hpp"
 #include "engine.hpp"
+#include "staging.hpp"
 
 namespace {
+
+using pysa::Arena;
+using pysa::DevBuf;
+using pysa::HostBuf;
 
 thread_local std::string g_err;
 
@@ -30,41 +35,6 @@ int fail(int code, const std::string& msg) {
     if (e_ != hipSuccess)                                                                    \
       return fail(PYSA_AMD_EHIP, std::string(#expr) + ": " + hipGetErrorString(e_));         \
   } while (0)
-
-struct DevBuf {
-  void* p = nullptr;
-  size_t bytes = 0;
-  hipError_t ensure(size_t b) {
-    if (b <= bytes) return hipSuccess;
-    if (p) (void)hipFree(p);
-    p = nullptr;
-    bytes = 0;
-    hipError_t e = hipMalloc(&p, b ? b : 1);
-    if (e == hipSuccess) bytes = b;
-    return e;
-  }
-  ~DevBuf() {
-    if (p) (void)hipFree(p);
-  }
-};
-
-// Pinned host memory.
-struct HostBuf {
-  void* p = nullptr;
-  size_t bytes = 0;
-  hipError_t ensure(size_t b) {
-    if (b <= bytes) return hipSuccess;
-    if (p) (void)hipHostFree(p);
-    p = nullptr;
-    bytes = 0;
-    hipError_t e = hipHostMalloc(&p, b, hipHostMallocDefault);
-    if (e == hipSuccess) bytes = b;
-    return e;
-  }
-  ~HostBuf() {
-    if (p) (void)hipHostFree(p);
-  }
-};
 
 struct Problem {
   int n = 0, ptype = 0, dtype = 0, device = 0;
@@ -307,84 +277,6 @@ int metropolis_device(int64_t handle, const RunArgs& a, double* kernel_ms, void*
   HIP_TRY(hipSetDevice(P->device));
   return metropolis_locked(P, a, kernel_ms, stream ? (hipStream_t)stream : P->stream);
 }
-
-// The device arrays of one host-pointer call in one block of memory that the
-// problem keeps for the next call (up to kKeep bytes; a larger block lives for
-// the call).  Arrays are added in the order inputs, inputs that are also
-// outputs, outputs, scratch, so the copies in and out cover one range each:
-// below kPin bytes each is a single copy through pinned memory.  (Before, a call
-// made and freed a buffer per array and copied each by itself: about 1 ms a
-// call, of which a short run of a small problem is a fraction.)
-struct Arena {
-  static constexpr size_t kKeep = size_t(256) << 20, kPin = size_t(1) << 20;
-  struct Item {
-    const void* src;
-    void* dst;
-    size_t bytes, off;
-  };
-  std::vector<Item> items;
-  size_t total = 0;
-  Problem* P;
-  DevBuf own;
-  char* base = nullptr;
-  explicit Arena(Problem* p) : P(p) { items.reserve(16); }
-  int add(const void* src, void* dst, size_t bytes) {
-    items.push_back({src, dst, bytes, total});
-    total += (bytes + 255) & ~size_t(255);
-    return (int)items.size() - 1;
-  }
-  template <typename T>
-  T* at(int i) const {
-    return reinterpret_cast<T*>(base + items[i].off);
-  }
-  // Allocates and copies the inputs in.
-  hipError_t up(hipStream_t st) {
-    DevBuf& b = total <= kKeep ? P->stage : own;
-    hipError_t e = b.ensure(total ? total : 1);
-    if (e != hipSuccess) return e;
-    base = (char*)b.p;
-    size_t end = 0;
-    for (const Item& it : items)
-      if (it.src) end = it.off + it.bytes;
-    if (end == 0) return hipSuccess;
-    if (end <= kPin && (e = P->pin.ensure(kPin)) == hipSuccess) {
-      for (const Item& it : items)
-        if (it.src) memcpy((char*)P->pin.p + it.off, it.src, it.bytes);
-      return hipMemcpyAsync(base, P->pin.p, end, hipMemcpyHostToDevice, st);
-    }
-    for (const Item& it : items)
-      if (it.src && it.bytes) {
-        e = hipMemcpyAsync(base + it.off, it.src, it.bytes, hipMemcpyHostToDevice, st);
-        if (e != hipSuccess) return e;
-      }
-    return hipSuccess;
-  }
-  // Copies the outputs back and waits for them.
-  hipError_t down(hipStream_t st) {
-    size_t lo = total, hi = 0;
-    for (const Item& it : items)
-      if (it.dst) {
-        lo = it.off < lo ? it.off : lo;
-        hi = it.off + it.bytes;
-      }
-    if (hi <= lo) return hipStreamSynchronize(st);
-    hipError_t e;
-    if (hi - lo <= kPin && (e = P->pin.ensure(kPin)) == hipSuccess) {
-      e = hipMemcpyAsync(P->pin.p, base + lo, hi - lo, hipMemcpyDeviceToHost, st);
-      if (e == hipSuccess) e = hipStreamSynchronize(st);
-      if (e != hipSuccess) return e;
-      for (const Item& it : items)
-        if (it.dst) memcpy(it.dst, (const char*)P->pin.p + (it.off - lo), it.bytes);
-      return hipSuccess;
-    }
-    for (const Item& it : items)
-      if (it.dst && it.bytes) {
-        e = hipMemcpyAsync(it.dst, base + it.off, it.bytes, hipMemcpyDeviceToHost, st);
-        if (e != hipSuccess) return e;
-      }
-    return hipStreamSynchronize(st);
-  }
-};
 
 // Device copies of the replay arrays, freed after the call.
 struct Staged {
@@ -684,7 +576,7 @@ int pysa_amd_metropolis(int64_t handle, int32_t reads, int32_t R, int32_t S, int
   HIP_TRY(sg.up(replay_pt_logu, (size_t)reads * S * (R > 1 ? R - 1 : 1) * sizeof(double), &t, st));
   d.rep_pt = (const double*)t;
   const bool lo = log_omega && log_omegas;
-  Arena ar(P);
+  Arena ar(P->stage, P->pin);
   const int i_be = ar.add(betas, nullptr, R * es);
   const int i_bs = beta_sort ? ar.add(beta_sort, nullptr, R * sizeof(int32_t)) : -1;
   const int i_st = ar.add(states, states, cnt * n);
@@ -744,7 +636,7 @@ int pysa_amd_ais(int64_t handle, const void* temps, int32_t nt, int32_t chains, 
     HIP_TRY(hipSetDevice(P->device));
     hipStream_t st = P->stream;
     const size_t n = P->n;
-    Arena ar(P);
+    Arena ar(P->stage, P->pin);
     const int i_t = ar.add(temps, nullptr, (size_t)nt * sizeof(float));
     const int i_s = ar.add(states, states, (size_t)chains * n);
     const int i_e = ar.add(nullptr, energies, (size_t)chains * sizeof(double));
@@ -912,7 +804,7 @@ int pysa_amd_energy(int64_t handle, const int8_t* states, int64_t count, double*
   std::lock_guard<std::mutex> lk(P->mu);
   HIP_TRY(hipSetDevice(P->device));
   hipStream_t st = P->stream;
-  Arena ar(P);
+  Arena ar(P->stage, P->pin);
   const int i_s = ar.add(states, nullptr, (size_t)count * P->n);
   const int i_o = ar.add(nullptr, out, (size_t)count * sizeof(double));
   const int i_x = ar.add(nullptr, nullptr, pysa::energy_scratch_bytes(P->n, count));

@@ -23,6 +23,16 @@ def probe():
     return ctypes.CDLL(os.path.join(HERE, "_build", "libhost_probe.so"))
 
 
+@pytest.fixture(scope="module")
+def staging():
+    subprocess.run(["make", "-s", "-C", HERE], check=True)
+    lib = ctypes.CDLL(os.path.join(HERE, "_build", "libstaging_check.so"))
+    lib.staging_without_pinned.argtypes = [ctypes.c_size_t]
+    lib.staging_kept.argtypes = [ctypes.POINTER(ctypes.c_size_t), ctypes.c_int]
+    lib.staging_kept.restype = lib.staging_alive.restype = ctypes.c_longlong
+    return lib
+
+
 # The schedule of the next sweep is written and read in one step below three
 # blocks (block-random order); below two, steps are read that do not exist.
 @pytest.mark.parametrize("kind", [0, 1, 2])
@@ -47,3 +57,9 @@ def test_exchange_walk_reads_energies_inside_the_workgroup(probe, tile):
             assert 0 <= got < 64
             if q < per and lane > b0:
                 assert got == b0 + below
+
+
+# 8 KB, and just below, at and above what pinned memory takes
+@pytest.mark.parametrize("bytes_", [1, 8192, (1 << 19) - 256, 1 << 19, (1 << 20) + 1])
+def test_staging_without_pinned_memory_leaves_no_error(staging, bytes_):
+    assert staging.staging_without_pinned(bytes_) == 0
