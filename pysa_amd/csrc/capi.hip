@@ -191,13 +191,16 @@ int run_plain(Problem* P, const RunArgs& a, hipStream_t st, double* ms) {
   p.log_omegas = a.logw ? a.log_omegas : nullptr;
   p.accepted = (unsigned long long*)a.accepted;
   p.plan = sparse ? pysa::kPlanReads : pysa::plan_plain(P->n, a.reads, a.R, (int)sizeof(T));
+  p.sums_chains = 0;
   p.sums = nullptr;
   p.eoff = nullptr;
   p.chain_beta = nullptr;
   if (p.plan == pysa::kPlanChains) {  // sums, offsets and betas of every chain
-    HIP_TRY(P->work.ensure(cnt * (n * sizeof(double) + sizeof(double) + sizeof(T))));
+    p.sums_chains = pysa::chain_sums_chains(P->n, (long long)cnt);
+    const size_t sums = (size_t)p.sums_chains * n;
+    HIP_TRY(P->work.ensure(sums * sizeof(double) + cnt * (sizeof(double) + sizeof(T))));
     p.sums = (double*)P->work.p;
-    p.eoff = p.sums + cnt * n;
+    p.eoff = p.sums + sums;
     p.chain_beta = (T*)(p.eoff + cnt);
   }
   // Per-read starting values: beta_idx = arange(R) (sa.py:325), the initial

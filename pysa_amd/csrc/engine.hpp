@@ -49,7 +49,8 @@ struct PTParams {
   unsigned long long* accepted;  // reads or null
   int plan;               // plan_plain
   // kPlanChains only
-  double* sums;           // reads*R*n: J s in f64
+  int sums_chains;        // chain_sums_chains
+  double* sums;           // sums_chains*n: J s in f64
   double* eoff;           // reads*R: the caller's initial energy minus its f64 recomputation
   T* chain_beta;          // reads*R: the beta of every chain in the coming sweep
 };
@@ -57,6 +58,8 @@ struct PTParams {
 // Where the chains of a plain run go: one workgroup per read or per chain.
 enum PlainPlan : int { kPlanReads = 0, kPlanChains = 1 };
 int plan_plain(int n, int reads, int R, int elem);
+// Chains whose f64 sums are in memory at a time (kPlanChains).
+int chain_sums_chains(int n, long long chains);
 
 // Compute units of the current device (cached per device).
 int device_cus();

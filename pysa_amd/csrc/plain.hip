@@ -804,15 +804,16 @@ __global__ __launch_bounds__((64 * pt_waves<T, G, V>())) void plain_pt_kernel(PT
 
 // ---- one workgroup (one wave) per chain ----
 
-// F = J s and the energy of a chain from its f64 sums (chain_sums_kernel), as
-// Chain::refresh makes them; s: the sweep before which this happens.
+// F = J s and the energy of the chains from c0 on from their f64 sums
+// (chain_sums_kernel), as Chain::refresh makes them; s: the sweep before which
+// this happens.
 template <typename T, int G>
-__global__ __launch_bounds__(64) void chain_refresh_kernel(PTParams<T> p, int s) {
-  const size_t chain = blockIdx.x;
+__global__ __launch_bounds__(64) void chain_refresh_kernel(PTParams<T> p, int s, int c0) {
+  const size_t chain = (size_t)c0 + blockIdx.x;
   const int lane = threadIdx.x, n = p.n;
   Chain<T, G> ch;
   ch.load_spins(p.spins + chain * n, n);
-  const double* sums = p.sums + chain * n;
+  const double* sums = p.sums + (size_t)blockIdx.x * n;
   double e = 0.0;
 #pragma unroll
   for (int g4 = 0; g4 < G / 4; ++g4) {
@@ -1208,11 +1209,14 @@ hipError_t launch_pt_chains(const PTParams<T>& p, hipStream_t st) {
   const bool coupled = coupled_sweeps(p);
   hipLaunchKernelGGL((chain_exchange_kernel<T>), dim3(p.reads), dim3(256), 0, st, p, -1);
   for (int s = 0; s < p.S;) {
-    if (s == 0 || (p.refresh > 0 && s % p.refresh == 0)) {
-      hipLaunchKernelGGL((chain_sums_kernel<T>), dim3((chains + 3) / 4, (p.n + 255) / 256),
-                         dim3(256), 0, st, p.Jt, p.spins, p.n, chains, p.ptype, p.sums);
-      hipLaunchKernelGGL((chain_refresh_kernel<T, G>), dim3(chains), dim3(64), 0, st, p, s);
-    }
+    if (s == 0 || (p.refresh > 0 && s % p.refresh == 0))
+      for (int c0 = 0; c0 < chains; c0 += p.sums_chains) {
+        const int cnt = min(p.sums_chains, chains - c0);
+        hipLaunchKernelGGL((chain_sums_kernel<T>), dim3((cnt + 3) / 4, (p.n + 255) / 256),
+                           dim3(256), 0, st, p.Jt, p.spins + (size_t)c0 * p.n, p.n, cnt, p.ptype,
+                           p.sums);
+        hipLaunchKernelGGL((chain_refresh_kernel<T, G>), dim3(cnt), dim3(64), 0, st, p, s, c0);
+      }
     int e = coupled ? s + 1 : p.S;
     if (p.refresh > 0) e = min(e, s + p.refresh - s % p.refresh);
     hipLaunchKernelGGL((chain_sweep_kernel<T, G>), dim3(chains), dim3(64), 0, st, p, s, e);
@@ -1298,13 +1302,23 @@ hipError_t launch_plain_ais(const AISParams<T>& p, hipStream_t st) {
   }
 }
 
+// States whose f64 values per spin are in memory at a time: 16 MB of them, still
+// 2000 workgroups of 4 states and 256 spins, so a launch fills the device.  (All
+// at once, a problem kept 96 MB behind 4000 energies of 3000 spins.)
+static int f64_piece(int n, long long count) {
+  const long long fit = max(1ll, (16ll << 20) / (8ll * n) / 4) * 4;
+  return (int)min(fit, count);
+}
+
+int chain_sums_chains(int n, long long chains) { return f64_piece(n, chains); }
+
 // Tiling of the energy kernel: 16 states per workgroup once that fills the
 // device, else 4 states and 256 elements each, the sums in a second launch
 // (100 states of 3072 spins: 10.36 -> 0.37 ms).
 constexpr int kEnergyWide = 16 * 256;
 
 size_t energy_scratch_bytes(int n, long long count) {
-  return count >= kEnergyWide || n <= 256 ? 0 : (size_t)count * n * sizeof(double);
+  return count >= kEnergyWide || n <= 256 ? 0 : (size_t)f64_piece(n, count) * n * sizeof(double);
 }
 
 template <typename T>
@@ -1319,11 +1333,16 @@ hipError_t launch_energy_f64(const T* Jt, const T* h, const int8_t* spins, doubl
   }
   const unsigned chunks = (unsigned)((n + 255) / 256);
   if (chunks > 1 && !scratch) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((energy_f64_kernel<T, 4, 1>), dim3((unsigned)((count + 3) / 4), chunks),
-                     dim3(256), 0, st, Jt, h, spins, out, chunks > 1 ? scratch : nullptr, n,
-                     (int)count);
-  if (chunks > 1)
-    hipLaunchKernelGGL(energy_sum_kernel, dim3((unsigned)count), dim3(256), 0, st, scratch, out, n);
+  const int piece = chunks > 1 ? f64_piece(n, count) : (int)count;
+  for (long long s0 = 0; s0 < count; s0 += piece) {
+    const int cnt = (int)min((long long)piece, count - s0);
+    hipLaunchKernelGGL((energy_f64_kernel<T, 4, 1>), dim3((unsigned)((cnt + 3) / 4), chunks),
+                       dim3(256), 0, st, Jt, h, spins + (size_t)s0 * n, out + s0,
+                       chunks > 1 ? scratch : nullptr, n, cnt);
+    if (chunks > 1)
+      hipLaunchKernelGGL(energy_sum_kernel, dim3((unsigned)cnt), dim3(256), 0, st, scratch, out + s0,
+                         n);
+  }
   return hipGetLastError();
 }
 
