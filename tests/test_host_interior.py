@@ -63,3 +63,11 @@ def test_exchange_walk_reads_energies_inside_the_workgroup(probe, tile):
 @pytest.mark.parametrize("bytes_", [1, 8192, (1 << 19) - 256, 1 << 19, (1 << 20) + 1])
 def test_staging_without_pinned_memory_leaves_no_error(staging, bytes_):
     assert staging.staging_without_pinned(bytes_) == 0
+
+
+def test_staging_keeps_little_memory(staging):
+    mb = 1 << 20
+    for sizes in ([1024], [mb, 1024], [1024, 7 * mb, 20 * mb, 100], [8 * mb, 8 * mb + 1]):
+        kept = staging.staging_kept((ctypes.c_size_t * len(sizes))(*sizes), len(sizes))
+        assert 0 < kept <= 32 * mb  # four arrays a call
+        assert staging.staging_alive() == 0
