@@ -53,11 +53,13 @@ struct PTParams {
   double* sums;           // sums_chains*n: J s in f64
   double* eoff;           // reads*R: the caller's initial energy minus its f64 recomputation
   T* chain_beta;          // reads*R: the beta of every chain in the coming sweep
+  // Whether anything at the end of a sweep concerns other chains of the read.
+  bool coupled() const { return (use_pt && R > 1) || (logw && log_omegas) || best_sem == 1; }
 };
 
 // Where the chains of a plain run go: one workgroup per read or per chain.
 enum PlainPlan : int { kPlanReads = 0, kPlanChains = 1 };
-int plan_plain(int n, int reads, int R, int elem);
+int plan_plain(int n, int reads, int R, int elem, bool coupled);
 // Chains whose f64 sums are in memory at a time (kPlanChains).
 int chain_sums_chains(int n, long long chains);
 

@@ -22,7 +22,7 @@
 // to every field happen in the order of the flips, as one visit after another
 // would make them, so the results equal that to the bit.
 //
-// Where the chains run (plan_pt): one workgroup per read that carries all
+// Where the chains run (plan_plain): one workgroup per read that carries all
 // replicas through the whole run and meets at a barrier once per sweep, or,
 // when that leaves most of the device idle, one workgroup per chain with the
 // exchanges in a launch of their own after every sweep.
@@ -1189,12 +1189,6 @@ __global__ __launch_bounds__(256) void chain_sums_kernel(const T* __restrict__ J
     if (s0 + b < count) sums[(size_t)(s0 + b) * n + i] = f[b][0];
 }
 
-// Whether anything at the end of a sweep concerns other chains of the read.
-template <typename T>
-bool coupled_sweeps(const PTParams<T>& p) {
-  return (p.use_pt && p.R > 1) || (p.logw && p.log_omegas) || p.best_sem == 1;
-}
-
 template <typename T, int G, int V>
 hipError_t launch_pt_read(const PTParams<T>& p, hipStream_t st) {
   const int W = min(p.R, pt_waves<T, G, V>());
@@ -1206,7 +1200,7 @@ hipError_t launch_pt_read(const PTParams<T>& p, hipStream_t st) {
 template <typename T, int G>
 hipError_t launch_pt_chains(const PTParams<T>& p, hipStream_t st) {
   const int chains = p.reads * p.R;
-  const bool coupled = coupled_sweeps(p);
+  const bool coupled = p.coupled();
   hipLaunchKernelGGL((chain_exchange_kernel<T>), dim3(p.reads), dim3(256), 0, st, p, -1);
   for (int s = 0; s < p.S;) {
     if (s == 0 || (p.refresh > 0 && s % p.refresh == 0))
@@ -1253,24 +1247,41 @@ hipError_t launch_ais_shape(const AISParams<T>& p, hipStream_t st) {
 
 }  // namespace
 
-// A workgroup per chain when its rounds over the device (8 chains per compute
-// unit, 4 in f64, before they slow each other down) are fewer than the rounds
-// of a workgroup per read over its replicas; with one round each, when the
-// chains leave most of the device idle anyway and a sweep is long beside the
-// two launches it costs.  Microseconds a sweep, per read / per chain: f32 n =
-// 1024, 64 reads of 32: 585 / 442; 1 read of 32: 566 / 209; 32 reads of 16: 313
-// / 237, of n = 200: 40 / 46; 128 reads of 16: 323 / 436; 512 reads of 4: 259 /
-// 446; f64 n = 500, 8 reads of 16: 108 / 89.
-int plan_plain(int n, int reads, int R, int elem) {
+// A workgroup per chain or per read.  A chain alone on its compute unit, with
+// staged windows, takes a time that hardly depends on the replicas, plus about 8
+// us for the two launches of a sweep when its end couples the chains (coupled).
+// A read's time grows with its rounds of replicas and, within a round, with how
+// far its waves crowd the rows of one compute unit.  So (us a sweep, per read /
+// per chain):
+// * More rounds of a read over its waves than of the chains over the device (8
+//   chains a compute unit, 4 in f64, before they slow each other down): per
+//   chain.  n = 200, 1 read of 32: 55 / 41; n = 1024, 64 reads of 32: 585 / 442;
+//   n = 3072, 1 of 17: 26469 / 1260.  Not where the second round is less than
+//   half full and the launches are a good part of a short sweep: n = 16, 1 of
+//   17: 8.7 / 11.7; n = 64, 1 of 20: 15.0 / 18.2; n = 256, 1 of 17: 37 / 46; but
+//   n = 300, 1 of 17: 72 / 62.
+// * Above 2048 spins a wave's fields leave few registers for rows in flight:
+//   per chain while two fit a compute unit (n = 2500, 512 reads of 1: 2261 / 1248;
+//   n = 4096, 1 of 1: 3383 / 1096).
+// * Else per chain while each has a compute unit of its own (f64, n = 1600, 128
+//   reads of 4: 658 / 1055) and either the rows are long (n = 2048, 1 of 4: 775 /
+//   627; n = 1284, 1 of 4: 357 / 401) or the read's waves crowd its compute unit:
+//   n R words 9000 or more (f64, n = 300, 8 of 16: 67 / 62; n = 1024, 1 of 16: 198
+//   / 192, of 8: 170 / 191; n = 512, 1 of 16: 77 / 92), a little earlier without
+//   the launches (f64, n = 1024, 16 of 4: 355 / 325).
+int plan_plain(int n, int reads, int R, int elem, bool coupled) {
   const int64_t chains = (int64_t)reads * R;
-  const int G = regs_for(n);
-  const int W = elem == 8 ? waves_of(2 * G) : waves_of(G);
+  const int W = waves_of(regs_for(n) * (elem / 4));
   const int rounds = (R + W - 1) / W;
-  const int64_t per = (int64_t)device_cus() * (elem == 8 ? 4 : 8);
+  const int cus = device_cus();
+  const int64_t per = (int64_t)cus * (elem == 8 ? 4 : 8);
   const int64_t crounds = (chains + per - 1) / per;
-  if (crounds < rounds) return kPlanChains;
-  return chains <= 2 * device_cus() && (int64_t)n * R * (elem / 4) >= 8000 ? kPlanChains
-                                                                           : kPlanReads;
+  if (crounds < rounds)
+    return coupled && n <= 256 && 2 * R < 3 * W ? kPlanReads : kPlanChains;
+  if (n > 2048) return chains <= 2 * cus ? kPlanChains : kPlanReads;
+  const bool longer =
+      (n > 1800 && R > 1) || (int64_t)n * R * (elem / 4) >= (coupled ? 9000 : 8000);
+  return chains <= cus && longer ? kPlanChains : kPlanReads;
 }
 
 template <typename T>

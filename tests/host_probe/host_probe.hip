@@ -29,3 +29,8 @@ extern "C" int probe_launch_pipe(int kind, int order, int nblk, int tiles) {
 extern "C" int probe_lane_below(int b0, int below) {
   return pysa::blk::lane_below(b0, below);
 }
+
+// The plain form's plan (0 a workgroup per read, 1 per chain) on this device.
+extern "C" int probe_plan_plain(int n, int reads, int R, int elem, int coupled) {
+  return pysa::plan_plain(n, reads, R, elem, coupled != 0);
+}
