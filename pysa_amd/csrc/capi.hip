@@ -190,7 +190,7 @@ int run_plain(Problem* P, const RunArgs& a, hipStream_t st, double* ms) {
   p.best_sweeps = a.best_sweeps;
   p.log_omegas = a.logw ? a.log_omegas : nullptr;
   p.accepted = (unsigned long long*)a.accepted;
-  p.plan = sparse ? pysa::kPlanReads : pysa::plan_plain(P->n, a.reads, a.R, (int)sizeof(T), p.coupled());
+  p.plan = sparse ? pysa::kPlanReads : pysa::plan_plain(P->n, a.reads, a.R, a.S, (int)sizeof(T), p.coupled());
   p.sums_chains = 0;
   p.sums = nullptr;
   p.eoff = nullptr;

@@ -59,7 +59,7 @@ struct PTParams {
 
 // Where the chains of a plain run go: one workgroup per read or per chain.
 enum PlainPlan : int { kPlanReads = 0, kPlanChains = 1 };
-int plan_plain(int n, int reads, int R, int elem, bool coupled);
+int plan_plain(int n, int reads, int R, int S, int elem, bool coupled);
 // Chains whose f64 sums are in memory at a time (kPlanChains).
 int chain_sums_chains(int n, long long chains);
 

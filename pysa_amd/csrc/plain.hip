@@ -1256,32 +1256,40 @@ hipError_t launch_ais_shape(const AISParams<T>& p, hipStream_t st) {
 // * More rounds of a read over its waves than of the chains over the device (8
 //   chains a compute unit, 4 in f64, before they slow each other down): per
 //   chain.  n = 200, 1 read of 32: 55 / 41; n = 1024, 64 reads of 32: 585 / 442;
-//   n = 3072, 1 of 17: 26469 / 1260.  Not where the second round is less than
-//   half full and the launches are a good part of a short sweep: n = 16, 1 of
-//   17: 8.7 / 11.7; n = 64, 1 of 20: 15.0 / 18.2; n = 256, 1 of 17: 37 / 46; but
-//   n = 300, 1 of 17: 72 / 62.
+//   n = 3072, 1 of 17: 26469 / 1260; n = 300, 1 of 17: 72 / 62.  Not where the
+//   launches are a good part of a short sweep and the second round is at most
+//   half full: n = 16, 1 of 17: 8.7 / 11.7; n = 64, 1 of 20: 15.0 / 18.2; n =
+//   256, 1 of 17: 37 / 46; but n = 128, 1 of 24: 31 / 29.
 // * Above 2048 spins a wave's fields leave few registers for rows in flight:
 //   per chain while two fit a compute unit (n = 2500, 512 reads of 1: 2261 / 1248;
 //   n = 4096, 1 of 1: 3383 / 1096).
-// * Else per chain while each has a compute unit of its own (f64, n = 1600, 128
-//   reads of 4: 658 / 1055) and either the rows are long (n = 2048, 1 of 4: 775 /
-//   627; n = 1284, 1 of 4: 357 / 401) or the read's waves crowd its compute unit:
-//   n R words 9000 or more (f64, n = 300, 8 of 16: 67 / 62; n = 1024, 1 of 16: 198
-//   / 192, of 8: 170 / 191; n = 512, 1 of 16: 77 / 92), a little earlier without
-//   the launches (f64, n = 1024, 16 of 4: 355 / 325).
-int plan_plain(int n, int reads, int R, int elem, bool coupled) {
+// * Somewhat below, several replicas: per chain while each has a compute unit of
+//   its own (n = 2048, 1 of 4: 775 / 627; n = 1284, 1 of 4: 357 / 401).
+// * Else per chain where the read's waves crowd its compute unit, n R words 8000
+//   or more (f64, n = 300, 8 of 16: 67 / 62; f64, n = 1024, 1 of 8: 383 / 339), of
+//   sixteen waves with exchanges 9000 (n = 1024, 1 of 16: 198 / 192, of 8: 170 /
+//   191; n = 512, 1 of 16: 77 / 92), and the chains are not two to a compute unit
+//   with rows that are not short (f64, n = 1600, 128 of 4: 658 / 1055; f64, n =
+//   300, 32 of 16: 70 / 68).
+// The first fields take longer in a read's own waves, one row group after
+// another, than spread over the device (n = 824, 1 of 10: 0.9 ms more), so the
+// lines where a sweep is only a little faster per read ask for enough of them.
+int plan_plain(int n, int reads, int R, int S, int elem, bool coupled) {
   const int64_t chains = (int64_t)reads * R;
   const int W = waves_of(regs_for(n) * (elem / 4));
   const int rounds = (R + W - 1) / W;
   const int cus = device_cus();
   const int64_t per = (int64_t)cus * (elem == 8 ? 4 : 8);
   const int64_t crounds = (chains + per - 1) / per;
-  if (crounds < rounds)
-    return coupled && n <= 256 && 2 * R < 3 * W ? kPlanReads : kPlanChains;
+  if (crounds < rounds) {
+    const bool brief = n <= 256 && 2 * R <= 3 * W && (R - W) * n <= 320;
+    return coupled && S >= 16 && brief ? kPlanReads : kPlanChains;
+  }
   if (n > 2048) return chains <= 2 * cus ? kPlanChains : kPlanReads;
-  const bool longer =
-      (n > 1800 && R > 1) || (int64_t)n * R * (elem / 4) >= (coupled ? 9000 : 8000);
-  return chains <= cus && longer ? kPlanChains : kPlanReads;
+  if (n > 1800 && R > 1 && chains <= cus) return kPlanChains;
+  const bool many = S >= 64;
+  const bool crowded = (int64_t)n * R * (elem / 4) >= (coupled && many && W == 16 ? 9000 : 8000);
+  return crowded && chains <= (many && n > 512 ? cus : 2 * cus) ? kPlanChains : kPlanReads;
 }
 
 template <typename T>

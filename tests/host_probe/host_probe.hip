@@ -31,6 +31,6 @@ extern "C" int probe_lane_below(int b0, int below) {
 }
 
 // The plain form's plan (0 a workgroup per read, 1 per chain) on this device.
-extern "C" int probe_plan_plain(int n, int reads, int R, int elem, int coupled) {
-  return pysa::plan_plain(n, reads, R, elem, coupled != 0);
+extern "C" int probe_plan_plain(int n, int reads, int R, int S, int elem, int coupled) {
+  return pysa::plan_plain(n, reads, R, S, elem, coupled != 0);
 }

@@ -22,22 +22,32 @@ def plan():
     ctypes.CDLL(_lib.load()._name, mode=ctypes.RTLD_GLOBAL)
     probe = ctypes.CDLL(os.path.join(os.path.dirname(os.path.abspath(__file__)), "host_probe",
                                      "_build", "libhost_probe.so"))
-    return lambda n, reads, R, dtype, coupled: probe.probe_plan_plain(
-        n, reads, R, np.dtype(dtype).itemsize, int(coupled))
+    return lambda n, reads, R, S, dtype, coupled: probe.probe_plan_plain(
+        n, reads, R, S, np.dtype(dtype).itemsize, int(coupled))
 
 
 # The faster plan of each, measured on 256 compute units.
-@pytest.mark.parametrize("n,reads,R,dtype,coupled,want", [
-    (16, 1, 17, "f4", True, READS), (64, 8, 20, "f4", True, READS), (50, 1, 20, "f8", True, READS),
-    (256, 1, 23, "f4", True, READS), (300, 1, 17, "f4", True, CHAINS), (64, 1, 32, "f4", True, CHAINS),
-    (16, 1, 17, "f4", False, CHAINS), (50, 1, 16, "f4", True, READS), (512, 1, 16, "f4", True, READS),
-    (1024, 1, 8, "f4", True, READS), (1024, 1, 16, "f4", True, CHAINS), (300, 8, 16, "f8", True, CHAINS),
-    (512, 1, 8, "f8", True, READS), (1600, 128, 4, "f8", True, READS), (1024, 64, 8, "f8", True, READS),
-    (2048, 1, 2, "f4", True, CHAINS), (2048, 1, 1, "f4", False, READS), (2500, 512, 1, "f4", False, CHAINS),
-    (4096, 1, 1, "f4", False, CHAINS), (4096, 513, 1, "f4", False, READS), (33, 130, 17, "f4", True, READS),
+@pytest.mark.parametrize("n,reads,R,S,dtype,coupled,want", [
+    # rounds of a read; short sweeps, short runs
+    (16, 1, 17, 100, "f4", True, READS), (64, 8, 20, 100, "f4", True, READS),
+    (50, 1, 20, 100, "f8", True, READS), (16, 1, 17, 2, "f4", True, CHAINS),
+    (16, 1, 17, 100, "f4", False, CHAINS), (64, 1, 32, 100, "f4", True, CHAINS),
+    (256, 1, 23, 100, "f4", True, CHAINS), (300, 1, 17, 100, "f4", True, CHAINS),
+    (33, 130, 17, 100, "f4", True, READS),
+    # long rows
+    (2048, 1, 2, 9, "f4", True, CHAINS), (2048, 1, 1, 9, "f4", False, READS),
+    (2048, 200, 2, 100, "f4", True, READS), (2500, 512, 1, 9, "f4", False, CHAINS),
+    (4096, 1, 1, 9, "f4", False, CHAINS), (4096, 513, 1, 9, "f4", False, READS),
+    # crowded compute units
+    (50, 1, 16, 100, "f4", True, READS), (512, 1, 16, 100, "f4", True, READS),
+    (512, 1, 16, 10, "f4", True, CHAINS), (1024, 1, 8, 100, "f4", True, READS),
+    (1024, 1, 16, 100, "f4", True, CHAINS), (300, 8, 16, 100, "f8", True, CHAINS),
+    (300, 32, 16, 100, "f8", True, CHAINS), (512, 1, 8, 100, "f8", True, READS),
+    (1600, 128, 4, 100, "f8", True, READS), (1600, 64, 4, 100, "f8", True, CHAINS),
+    (1024, 64, 8, 100, "f8", True, READS),
 ])
-def test_plan(plan, n, reads, R, dtype, coupled, want):
-    assert plan(n, reads, R, dtype, coupled) == want
+def test_plan(plan, n, reads, R, S, dtype, coupled, want):
+    assert plan(n, reads, R, S, dtype, coupled) == want
 
 
 def run(n, R, reads, S, dtype, ptype, order, best_sem=0, use_pt=True, log_omega=False):
@@ -65,16 +75,16 @@ def run(n, R, reads, S, dtype, ptype, order, best_sem=0, use_pt=True, log_omega=
                                              (1100, 1, 300, "f8"), (1030, 5, 210, "f8")])
 @pytest.mark.parametrize("ptype,order", [(0, 0), (1, 1)])
 def test_large_reads(plan, n, R, reads, dtype, ptype, order):
-    assert plan(n, reads, R, dtype, R > 1) == READS
+    assert plan(n, reads, R, 1, dtype, R > 1) == READS
     run(n, R, reads, 1, np.dtype(dtype), ptype, order)
 
 
 # Replicas carried through memory: ends of sweeps and, in float32, a refresh.
-@pytest.mark.parametrize("dtype,reads,S", [("f4", 2, 131), ("f4", 130, 131), ("f8", 2, 5)])
+@pytest.mark.parametrize("dtype,reads,S", [("f4", 2, 131), ("f4", 130, 131), ("f8", 2, 16)])
 @pytest.mark.parametrize("use_pt,best_sem,log_omega", [(True, 1, False), (True, 0, True),
                                                        (False, 1, False), (False, 0, True)])
 def test_carried_replicas(plan, dtype, reads, S, use_pt, best_sem, log_omega):
-    assert plan(70, reads, 17, dtype, True) == READS
+    assert plan(70, reads, 17, S, dtype, True) == READS
     run(70, 17, reads, S, np.dtype(dtype), 0, 1, best_sem, use_pt, log_omega)
 
 
