@@ -1174,7 +1174,11 @@ int regs_for(int n) {
   return g;
 }
 
-// J s in f64 of every chain (the input of chain_refresh_kernel).
+// J s in f64 of every chain (the input of chain_refresh_kernel).  The tiling
+// multiplies by an unset QUBO spin, which makes NaN of an infinite coupling where
+// Chain::refresh adds nothing; no other sum is NaN without one of its terms being
+// so, and those that are, are taken again over the set spins.  (Leaving unset
+// spins out of every sum cost the RBM step 0.13 of 3.73 ms.)
 template <typename T>
 __global__ __launch_bounds__(256) void chain_sums_kernel(const T* __restrict__ Jt,
                                                          const int8_t* __restrict__ spins, int n,
@@ -1186,7 +1190,16 @@ __global__ __launch_bounds__(256) void chain_sums_kernel(const T* __restrict__ J
   if (i >= n) return;
 #pragma unroll
   for (int b = 0; b < 4; ++b)
-    if (s0 + b < count) sums[(size_t)(s0 + b) * n + i] = f[b][0];
+    if (s0 + b < count) {
+      double x = f[b][0];
+      if (ptype == 1 && x != x) {
+        const int8_t* s = spins + (size_t)(s0 + b) * n;
+        x = 0.0;
+        for (int j = 0; j < n; ++j)
+          if (s[j] == 1) x += (double)Jt[(size_t)j * n + i];
+      }
+      sums[(size_t)(s0 + b) * n + i] = x;
+    }
 }
 
 template <typename T, int G, int V>
