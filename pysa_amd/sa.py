@@ -123,6 +123,16 @@ class Solver(object):
             flat *= 2
             flat -= 1
 
+    def _bernoulli_spins(self, states, p):
+        """States whose entries are -1/0 with probability p into the rows, from the
+        global NumPy RNG: the draws and their order are those of
+        ais.bernoulli_prob_initialization for one row after another."""
+        for row in states:
+            row[:] = np.random.binomial(1, 1 - p, size=row.size)
+        if self.problem_type == 'ising':
+            states *= 2
+            states -= 1
+
     def metropolis_update_async(self, **kwargs):
         kwargs['send_background'] = False
         return self.metropolis_update(**kwargs)
@@ -488,11 +498,7 @@ class Solver(object):
         if ref_code == 0:
             self._random_spins(spins)
         else:
-            for k in range(num_samps):
-                spins[k] = np.random.binomial(1, 1 - reference_args[0], size=self.n_vars)
-            if self.problem_type == 'ising':
-                spins *= 2
-                spins -= 1
+            self._bernoulli_spins(spins, reference_args[0])
         rep_lr = rep_perm = None
         if replay is not None:
             rep_lr = np.ascontiguousarray(replay['log_r'], dtype=np.float64)
