@@ -227,8 +227,9 @@ int pysa_amd_plain_fields(int64_t handle, int64_t count, void* out);
  *           1 = pipelined, 2 = split-K (the block-random order always runs
  *           the pipelined kernel)
  *   tiles   replicas per workgroup of the pipelined kernel in tiles of 32:
- *           0 = by occupancy (one tile when two-tile workgroups would leave
- *           compute units idle), 1 or 2 (R > 32 always takes 2)
+ *           0 = by the rounds of workgroups over the compute units (one tile
+ *           until it takes 25/18 times the rounds of two), 1 or 2 (R > 32
+ *           always takes 2)
  */
 int pysa_amd_problem_set_shape(int64_t handle, int32_t kernel, int32_t tiles);
 

@@ -152,7 +152,7 @@ class Problem:
     def set_shape(self, kernel=0, tiles=0):
         """Launch shape of the MFMA form on this problem: kernel 0 = by size,
         1 = pipelined, 2 = split-K; tiles of 32 replicas per workgroup 0 = by
-        occupancy, 1 or 2.  Results do not depend on it."""
+        the rounds of workgroups, 1 or 2.  Results do not depend on it."""
         check(load().pysa_amd_problem_set_shape(self.handle, int(kernel), int(tiles)))
 
     def plain_fields(self, count):

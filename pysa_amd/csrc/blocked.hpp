@@ -32,7 +32,7 @@ struct BlockedProblem {
   int jtl_kind = -1;
   // Launch shape (results do not depend on it): kernel 0 = by size,
   // 1 = pipelined, 2 = split-K; tiles of 32 replicas per workgroup of the
-  // pipelined kernel, 0 = by occupancy, 1 or 2.
+  // pipelined kernel, 0 = by the rounds of workgroups, 1 or 2.
   int shape_kernel = 0;
   int shape_tiles = 0;
 };

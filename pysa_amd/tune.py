@@ -25,8 +25,8 @@ every valid shape on the caller's problem and batch size (random spins, a
 few sweeps, device time of the engine call, best of two), keeps the fastest
 and stores it in a JSON cache: $PYSA_AMD_TUNE_CACHE, else
 ~/.cache/pysa_amd/tune.json.  PYSA_AMD_TUNE=0 skips tuning and leaves the
-library's rule (two tiles once one-tile workgroups would take more rounds
-over the compute units than they save).
+library's rule (two tiles once one-tile workgroups would take more than 25/18
+times their rounds over the compute units).
 """
 
 import json
@@ -154,7 +154,7 @@ def tune(problem, R, reads, order, force=False, path=None):
 
 def apply(problem, R, reads, order):
     """Set the problem's launch shape for a run: the tuned one, or the
-    library's occupancy rule when PYSA_AMD_TUNE=0."""
+    library's rule when PYSA_AMD_TUNE=0."""
     if os.environ.get("PYSA_AMD_TUNE", "1") == "0":
         problem.set_shape(0, 0)
         return None
