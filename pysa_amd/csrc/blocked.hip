@@ -732,7 +732,7 @@ BlockedPlan plan_blocked(const BlockedProblem& b, int n, int reads, int R, int o
             (pipe_takes(order, pl.nblk) && (b.shape_kernel == 1 || !want_splitk));
   // Tiles of 32 replicas per workgroup of the pipelined kernel (one workgroup
   // per CU either way): the fewer rounds over the device, a one-tile block step
-  // taking about 18 / 25 of a two-tile one (n = 1024: 2.7 and 3.8 us).
+  // taking about 18 / 25 of a two-tile one (n = 1024: 2.5 and 3.4 us).
   if (R > 32)
     pl.nt = 2;
   else if (b.shape_tiles == 1 || b.shape_tiles == 2)

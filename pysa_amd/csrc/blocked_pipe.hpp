@@ -271,7 +271,7 @@ __global__ __launch_bounds__(128 * (MW + 1)) void blocked_pipe_kernel(BParams p0
     }
   }
   // fragment stages in flight per matrix wave (slot ring), within the registers
-  // (two tiles, N = 1024, us a sweep: two pieces 121 with 3, 127 with 5; three
+  // (two tiles, N = 1024, us a sweep of 200: two pieces 121 with 3, 127 with 5; three
   // pieces 151 with 2, 160 with 3, which spills)
   constexpr int PF = I8 || NP == 1 ? 6 : NT == 1 ? (NP == 2 ? 6 : 4) : NP == 2 ? 3 : 2;
   const uint32_t emul = p.ptype == 0 ? 0xFEu : 1u;
