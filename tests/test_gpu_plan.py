@@ -79,6 +79,26 @@ def test_large_reads(plan, n, R, reads, dtype, ptype, order):
     run(n, R, reads, 1, np.dtype(dtype), ptype, order)
 
 
+# Real couplings: the same chains in both plans (log-omega couples the sweeps and
+# so takes the run to a workgroup per read, but changes nothing in the chains).
+@pytest.mark.parametrize("n,R", [(16, 17), (64, 20), (130, 18), (255, 17)])
+@pytest.mark.parametrize("dtype", ["f4", "f8"])
+@pytest.mark.parametrize("ptype,order", [(0, 0), (0, 1), (1, 1), (1, 2), (1, 3)])
+def test_plans_agree_on_real_couplings(plan, n, R, dtype, ptype, order):
+    S = 131  # across a refresh in float32
+    assert plan(n, 2, R, S, dtype, True) == READS and plan(n, 2, R, S, dtype, False) == CHAINS
+    rng = np.random.default_rng([n, R, order])
+    A = np.triu(rng.standard_normal((n, n)), 1) / np.sqrt(n)
+    J, h = (A + A.T).astype(dtype), (0.1 * rng.standard_normal(n)).astype(dtype)
+    betas = np.geomspace(3.0, 0.5, R).astype(dtype)
+    betas[-1] = 0.0
+    st = random_spins((2, R, n), rng, ptype)
+    en = np.zeros((2, R), dtype)
+    kw = dict(order=order, use_pt=False, seed=3)
+    assert_same(engine_metropolis(J, h, ptype, betas, st, en, S, log_omega=True, **kw),
+                engine_metropolis(J, h, ptype, betas, st, en, S, log_omega=False, **kw))
+
+
 # Replicas carried through memory: ends of sweeps and, in float32, a refresh.
 @pytest.mark.parametrize("dtype,reads,S", [("f4", 2, 131), ("f4", 130, 131), ("f8", 2, 16)])
 @pytest.mark.parametrize("use_pt,best_sem,log_omega", [(True, 1, False), (True, 0, True),
